@@ -40,6 +40,15 @@ int tiles_workspace_bytes(const pbr_scene_desc* D, const pbr_render_opts* opts, 
 int launch_tiles(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_render_opts* opts,
                  void* workspace, size_t workspace_bytes, hipStream_t st);
 
+// The band path (pbr_bands.hip): whether it draws the batch with these
+// options, and its launch.  `scene_off` holds each scene's first slot of the
+// batch when instance counts differ per scene (not `uniform`); slots past
+// `budget` are not drawn.  hdr[0] of the workspace is the overflow flag.
+bool bands_supported(const pbr_scene_desc* D, const pbr_render_opts* opts);
+int launch_bands(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_render_opts* opts,
+                 uint32_t max_slots, uint32_t budget, bool uniform, const uint32_t* scene_off,
+                 uint32_t* hdr, hipStream_t st);
+
 // The row-span kernel (pbr_rows.hip): whether it serves the descriptor, and
 // its launch (no workspace).  With `npose` > 0 the launch first applies
 // `poses` as pbr_set_poses would (each workgroup the rows of its own scenes)

@@ -1121,11 +1121,16 @@ int launch_tiles(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rend
   const int persistent = (opts && opts->persistent) ? 1 : 0;
   const Light lt = host_light(D);
   hipError_t e = hipSuccess;
+  const bool bands = bands_supported(D, opts);
+  if (bands && !T.counts)
+    return launch_bands(D, O, opts, F.max_slots, F.budget, true, nullptr, P.hdr, st);
   // prep: zero the per-scene visible counts (and the queue head), and with
   // per-scene instance counts the scenes' first pool slots
   hipLaunchKernelGGL(tile_prep_kernel, dim3(1), dim3(1024), 0, st, *D, F, P, T.counts ? 1 : 0);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(PBR_ERR_LAUNCH, "tile prep launch failed: %s", hipGetErrorString(e));
+  if (bands) return launch_bands(D, O, opts, F.max_slots, F.budget, false, P.scene_off,
+                                 P.hdr, st);
   // setup: 64 waves per CU, about three rounds of resident ones (measured
   // on MI355X for the 8192-scene uneven batch: one round of equal ranges
   // 1123 us, three 900 us), never more than the pool needs
