@@ -72,12 +72,19 @@ struct NodeLds {
   uint32_t base, chunk0;  // first slot and first chunk of the node in this scene
   uint32_t cnt;           // active instances
   int32_t ntri, voff, ioff, ips;
+  float inv_nt;           // 1 / ntri
   uint32_t flags;         // bit 0: shared, bit 1: flat
 };
 
-// Vertex table entry: X << 6 | outcode, Y << 6 | inside all planes << 1 |
-// snapped.  |X|, |Y| <= 2^24 (snap_vertex), so both shifts fit 32 bits.
-constexpr int kInAll = 2, kSnapped = 1;
+// Vertex table entry: X << 6 | outcode, Y << 1 | not snapped.  |X|, |Y| <=
+// 2^24 (snap_vertex), so both shifts fit 32 bits.
+constexpr int kOutMask = 0x3f;
+
+// Snapped extents (1/256 pixel) up to which edge values are evaluated in 32
+// bits: coordinate differences are at most 2^14, their products 2^28, and
+// the two products, the fill-rule bias and the overshoot of a block of
+// pixels stay below 2^30.
+constexpr int kIntExtent = 1 << 14;
 
 typedef const __attribute__((address_space(4))) float const_float;
 typedef const __attribute__((address_space(1))) float global_cfloat;
@@ -121,76 +128,97 @@ struct BandCtx {
   int j0, j1;  // GL rows of the band; LDS row 0 is j1
 };
 
-__device__ __forceinline__ void band_fragment(unsigned long long* pix, const BandCtx& t, int i,
-                                              int j, float z, uint32_t rank) {
-  const unsigned long long key = ((unsigned long long)__float_as_uint(z) << 32) | rank;
-  unsigned long long* q = pix + (t.j1 - j) * t.W + i;
-  // keys only decrease, so a read that is already <= the key proves the
-  // atomic would change nothing
-  if (key < *q) atomicMin(q, key);
+// Depth test of one fragment: LDS atomicMin on the key (depth bits, rank).
+// No read before it: with few fragments per pixel the read's latency costs
+// more than the atomics it would save.
+__device__ __forceinline__ void band_fragment(unsigned long long* q, float z, uint32_t rank) {
+  atomicMin(q, ((unsigned long long)__float_as_uint(z) << 32) | rank);
 }
 
-// Biased edge values e_k = A_k Px + B_k Py + C_k >= 0 <=> inside, at pixel
-// (i, j); every term is an integer below 2^53.
+// Edge function steps in 1/256 pixel: edge k is opposite vertex k,
+// e_k(x, y) = A_k (x - X_a) + B_k (y - Y_a) - bias_k, inside <=> e_k >= 0.
+// Num is int32_t (see kIntExtent) or double (every term an integer below
+// 2^53, so the arithmetic is exact in either).
+template <typename Num>
 struct BandEdges {
-  double A[3], B[3], C[3];
+  Num A[3], B[3], e[3];  // e at the first pixel centre
 };
 
-__device__ __forceinline__ void band_edges(const int32_t X[3], const int32_t Y[3], uint32_t bias,
-                                           BandEdges& E) {
+template <typename Num>
+__device__ __forceinline__ void band_edges(const FixTri& T, int i, int j, BandEdges<Num>& E) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int a = (k + 1) % 3, b = (k + 2) % 3;
-    E.A[k] = (double)(Y[a] - Y[b]);
-    E.B[k] = (double)(X[b] - X[a]);
-    E.C[k] = -fma(E.A[k], (double)X[a], E.B[k] * (double)Y[a]) - (double)((bias >> k) & 1u);
+    const int32_t A = T.Y[a] - T.Y[b], B = T.X[b] - T.X[a];
+    const int32_t dx = 256 * i + 128 - T.X[a], dy = 256 * j + 128 - T.Y[a];
+    const int32_t bias = (int32_t)((T.bias >> k) & 1u);
+    if constexpr (sizeof(Num) == 4) {
+      E.e[k] = __mul24(A, dx) + __mul24(B, dy) - bias;
+      E.A[k] = A * 256;
+      E.B[k] = B * 256;
+    } else {
+      E.e[k] = fma((double)A, (double)dx, (double)B * (double)dy) - (double)bias;
+      E.A[k] = (double)A * 256.0;
+      E.B[k] = (double)B * 256.0;
+    }
   }
+}
+
+__device__ __forceinline__ bool band_inside(const int32_t e[3]) { return (e[0] | e[1] | e[2]) >= 0; }
+__device__ __forceinline__ bool band_inside(const double e[3]) {
+  return e[0] >= 0.0 && e[1] >= 0.0 && e[2] >= 0.0;
 }
 
 // One lane, the whole box.
 __device__ __forceinline__ void band_raster_lane(unsigned long long* pix, const BandCtx& t,
                                                  const FixTri& T, uint32_t rank) {
-  BandEdges E;
-  band_edges(T.X, T.Y, T.bias, E);
-  const double px0 = (double)(256 * T.i0 + 128);
-  for (int j = T.j0; j <= T.j1; ++j) {
-    const double py = (double)(256 * j + 128);
-    double e0 = fma(E.A[0], px0, fma(E.B[0], py, E.C[0]));
-    double e1 = fma(E.A[1], px0, fma(E.B[1], py, E.C[1]));
-    double e2 = fma(E.A[2], px0, fma(E.B[2], py, E.C[2]));
-    const float tz = fmaf(T.zy, (float)j + 0.5f, T.zc);
-    for (int i = T.i0; i <= T.i1; ++i) {
-      if (e0 >= 0.0 && e1 >= 0.0 && e2 >= 0.0)
-        band_fragment(pix, t, i, j, clamp_depth(fmaf(T.zx, (float)i + 0.5f, tz)), rank);
-      e0 += E.A[0] * 256.0;
-      e1 += E.A[1] * 256.0;
-      e2 += E.A[2] * 256.0;
+  BandEdges<int32_t> E;
+  band_edges(T, T.i0, T.j0, E);
+  const float x0 = (float)T.i0 + 0.5f;
+  unsigned long long* row = pix + (t.j1 - T.j0) * t.W + T.i0;
+  const int w = T.i1 - T.i0;
+  float y = (float)T.j0 + 0.5f;
+  for (int h = T.j1 - T.j0; h >= 0; --h) {
+    int32_t e[3] = {E.e[0], E.e[1], E.e[2]};
+    const float tz = fmaf(T.zy, y, T.zc);
+    float x = x0;
+    for (int i = 0; i <= w; ++i) {
+      if (band_inside(e)) band_fragment(row + i, clamp_depth(fmaf(T.zx, x, tz)), rank);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) e[k] += E.A[k];
+      x += 1.0f;  // exact: a pixel centre
     }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) E.e[k] += E.B[k];
+    y += 1.0f;
+    row -= t.W;
   }
 }
 
 // The whole wave, in blocks of 8 x 8 pixels.  Every argument is uniform.
+template <typename Num>
 __device__ __forceinline__ void band_raster_wave(unsigned long long* pix, const BandCtx& t,
                                                  int lane, const FixTri& T, uint32_t rank) {
-  BandEdges E;
-  band_edges(T.X, T.Y, T.bias, E);
+  BandEdges<Num> E;
+  band_edges(T, T.i0, T.j0, E);
   const int li = lane & 7, lj = lane >> 3;
+  Num row[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) row[k] = E.e[k] + E.A[k] * (Num)li + E.B[k] * (Num)lj;
   for (int jb = T.j0; jb <= T.j1; jb += 8) {
     const int j = jb + lj;
-    const double py = (double)(256 * j + 128);
-    const double px = (double)(256 * (T.i0 + li) + 128);
-    double e0 = fma(E.A[0], px, fma(E.B[0], py, E.C[0]));
-    double e1 = fma(E.A[1], px, fma(E.B[1], py, E.C[1]));
-    double e2 = fma(E.A[2], px, fma(E.B[2], py, E.C[2]));
     const float tz = fmaf(T.zy, (float)j + 0.5f, T.zc);
-    for (int ib = T.i0; ib <= T.i1; ib += 8) {
+    unsigned long long* q = pix + (t.j1 - j) * t.W + T.i0 + li;
+    Num e[3] = {row[0], row[1], row[2]};
+    for (int ib = T.i0; ib <= T.i1; ib += 8, q += 8) {
       const int i = ib + li;
-      if (i <= T.i1 && j <= T.j1 && e0 >= 0.0 && e1 >= 0.0 && e2 >= 0.0)
-        band_fragment(pix, t, i, j, clamp_depth(fmaf(T.zx, (float)i + 0.5f, tz)), rank);
-      e0 += E.A[0] * 2048.0;
-      e1 += E.A[1] * 2048.0;
-      e2 += E.A[2] * 2048.0;
+      if (i <= T.i1 && j <= T.j1 && band_inside(e))
+        band_fragment(q, clamp_depth(fmaf(T.zx, (float)i + 0.5f, tz)), rank);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) e[k] += E.A[k] * (Num)8;
     }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) row[k] += E.B[k] * (Num)8;
   }
 }
 
@@ -199,76 +227,143 @@ __device__ __forceinline__ float rlf(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Clip polygon of slot `local` of node j; only triangles that straddle a clip
-// plane get here.
-__device__ __noinline__ int band_clip(const pbr_scene_desc* D, float guard, int s, int j,
-                                      uint32_t local, CVert* poly) {
-  CVert cv[3];
-  float rgba[4];
-  bool flat;
-  fetch_node_triangle(*D, s, j, local, cv, rgba, flat);
-  poly[0] = cv[0];
-  poly[1] = cv[1];
-  poly[2] = cv[2];
-  return clip_polygon(poly, guard);
+// Bit p: not inside clip plane p (NaN distances count as outside, as the
+// clipper takes them).
+__device__ __forceinline__ uint32_t outcode(const CVert& v, float guard) {
+  uint32_t oc = 0;
+#pragma unroll
+  for (int p = 0; p < 6; ++p) oc |= plane_dist(v, p, guard) >= 0.0f ? 0u : 1u << p;
+  return oc;
 }
 
-__device__ __noinline__ bool band_clip_sub(const CVert* poly, int q, int W, int H, int j0, int j1,
-                                           FixTri* T) {
-  return setup_fixed(poly[0], poly[q + 1], poly[q + 2], W, H, j0, j1, *T);
+// A value of lane `src`.
+__device__ __forceinline__ int from_lane(int src, int v) {
+  return __builtin_amdgcn_ds_bpermute(src << 2, v);
+}
+__device__ __forceinline__ float from_lane(int src, float v) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(v)));
+}
+// Sends v to lane `dst`; the lane's result is 0 if no lane sends to it.
+__device__ __forceinline__ float to_lane(int dst, float v) {
+  return __int_as_float(__builtin_amdgcn_ds_permute(dst << 2, __float_as_int(v)));
 }
 
-// Smooth colour of sub-triangle q of a clipped slot at pixel centre (px, py).
-__device__ __noinline__ void band_clipped_colour(const pbr_scene_desc* D, float guard, int s,
-                                                 int j, uint32_t local, int q, const float* rgba,
-                                                 Light lt, double px, double py, float* col) {
-  CVert poly[kMaxPoly];
-  const int n = band_clip(D, guard, s, j, local, poly);
-  FixTri T;
-  if (q + 2 >= n || !band_clip_sub(poly, q, D->width, D->height, 0, D->height - 1, &T)) return;
-  double A[3], B[3], C[3];
-  edges_from_fixed(T.X, T.Y, T.bias, A, B, C);
-  const CVert* v[3] = {&poly[0], &poly[q + 1], &poly[q + 2]};
-  float sh[kShadeFloats];
-  for (int k = 0; k < 3; ++k) {
-    for (int c = 0; c < 3; ++c) sh[3 * k + c] = v[k]->n[c];
-    sh[9 + k] = T.invw[k];
+// Sutherland-Hodgman on four polygons at once, one per group of 16 lanes: lane
+// k of a group holds vertex k < n (every lane of the wave takes part; NC = 4
+// clips positions, 7 normals too).  The same planes, order, intersections and
+// vertex limit as clip_polygon; a plane that has every vertex inside leaves
+// the polygons as they are and is skipped.  In registers: clip_polygon's
+// arrays lie in scratch memory, where clipping 64 triangles at a time took
+// most of the 95 us a steering scene's workgroup spent on setup.
+template <int NC>
+__device__ __forceinline__ void clip_groups(float v[NC], int& n, float guard, int lane) {
+  const int k = lane & 15, base = lane & 48;
+  for (int plane = 0; plane < 6; ++plane) {
+    CVert a, b;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a.p[c] = v[c];
+    const float da = plane_dist(a, plane, guard);
+    const bool act = k < n, ina = act && da >= 0.0f;
+    if (!__ballot(act && !ina)) continue;
+    const int nx = base + (k + 1 >= n ? 0 : k + 1);
+    float w[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) w[c] = from_lane(nx, v[c]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b.p[c] = w[c];
+    const float db = plane_dist(b, plane, guard);
+    const bool cross = act && ina != (db >= 0.0f);
+    const float di = ina ? da : db, dout = ina ? db : da;
+    const float t = di / (di - dout);
+    float r[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const float vi = ina ? v[c] : w[c], vo = ina ? w[c] : v[c];
+      r[c] = vi + t * (vo - vi);
+    }
+    const uint32_t mi = (uint32_t)(__ballot(ina) >> base) & 0xffffu;
+    const uint32_t mx = (uint32_t)(__ballot(cross) >> base) & 0xffffu;
+    const uint32_t below = (1u << k) - 1u;
+    const int pa = __popc(mi & below) + __popc(mx & below), px = pa + (ina ? 1 : 0);
+    // lane 15 of a group takes what goes nowhere (a polygon has <= 9 vertices)
+    const int ta = base + (ina && pa < kMaxPoly ? pa : 15);
+    const int tx = base + (cross && px < kMaxPoly ? px : 15);
+    const bool is_x = to_lane(tx, 1.0f) != 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const float va = to_lane(ta, v[c]), vx = to_lane(tx, r[c]);
+      v[c] = is_x ? vx : va;
+    }
+    n = min(__popc(mi) + __popc(mx), kMaxPoly);
   }
-  for (int c = 0; c < 4; ++c) sh[12 + c] = rgba[c];
-  shade_smooth(A, B, C, T.bias, sh, px, py, lt, col);
 }
 
-// Colour of the pixel whose winner is slot `slot`, sub-triangle q, of node j.
-template <bool SMOOTH>
-__device__ __forceinline__ void band_shade(const pbr_scene_desc& D, const BandFrame& F,
-                                           const Light& lt, int s, const float VP[16],
-                                           const NodeLds* nodes, int nn, const uint32_t* tab,
-                                           uint32_t slot, int q, int x, int j, float col[4]) {
+// Vertices (clip position, world normal) of the mesh triangles of four slots,
+// vertex k of group g's triangle in lane 16 g + k (k < 3).
+__device__ __forceinline__ void group_vertex(const pbr_scene_desc& D, const float* trans,
+                                             size_t row, int voff, uint32_t tri,
+                                             const float VP[16], int lane, CVert& cv) {
+  const int k = lane & 15;
+  const uint32_t id = k == 0 ? tri & 0xffu : (k == 1 ? (tri >> 8) & 0xffu : tri >> 16);
+  float M[16], vv[6];
+  load_mat4_global(trans + row * 16, M);
+  load_vertex(D.vertices, voff + (int)id, vv);
+  transform_vertex(M, VP, vv, cv);
+}
+
+// A slot's node, its instance row in the node's buffers and its mesh triangle.
+struct SlotRef {
+  const float* trans;
+  const float* cols;
+  size_t row;
+  int voff;
+  uint32_t tri;    // vertex indices a | b << 8 | c << 16
+  uint32_t flags;  // the node's (NodeLds)
+};
+
+__device__ __forceinline__ SlotRef band_slot(const pbr_scene_desc& D, const BandFrame& F, int s,
+                                             const NodeLds* nodes, int nn, const uint32_t* tab,
+                                             uint32_t slot) {
   int nj = 0;
   for (int k = 1; k < nn; ++k) nj = slot >= nodes[k].base ? k : nj;
   const NodeLds& nd = nodes[nj];
-  const uint32_t local = slot - nd.base, nt = (uint32_t)nd.ntri;
-  // local / nt from a float reciprocal: the quotient is below 2^24, so the
+  const uint32_t local = slot - nd.base;
+  // local / ntri from a float reciprocal: the quotient is below 2^24, so the
   // truncated product is off by at most one and one step corrects it
-  uint32_t i = (uint32_t)((float)local * (1.0f / (float)nt));
-  int32_t t = (int32_t)(local - i * nt);
+  uint32_t i = (uint32_t)((float)local * nd.inv_nt);
+  int32_t t = (int32_t)(local - i * (uint32_t)nd.ntri);
   if (t < 0) {
     --i;
-    t += (int32_t)nt;
-  } else if (t >= (int32_t)nt) {
+    t += nd.ntri;
+  } else if (t >= nd.ntri) {
     ++i;
-    t -= (int32_t)nt;
+    t -= nd.ntri;
   }
-  const size_t row = (nd.flags & 1u) ? (size_t)i : (size_t)s * (size_t)nd.ips + i;
-  float M[16];
-  load_mat4_global(nd.trans + row * 16, M);
-  const f32x4 c4 = ((global_cfloat4*)(uintptr_t)nd.cols)[row];
-  const float rgba[4] = {c4.x, c4.y, c4.z, c4.w};
-  const uint32_t tri = F.ntab ? tab[nd.ioff + t] : pool_triangle(D, nd.ioff + t);
-  float v[6];
-  load_vertex(D.vertices, nd.voff + (int)(tri & 0xffu), v);
-  if (!SMOOTH || (nd.flags & 2u)) {
-    float nw[3], n[3];
+  SlotRef R;
+  R.trans = nd.trans;
+  R.cols = nd.cols;
+  R.row = (nd.flags & 1u) ? (size_t)i : (size_t)s * (size_t)nd.ips + i;
+  R.voff = nd.voff;
+  R.tri = F.ntab ? tab[nd.ioff + t] : pool_triangle(D, nd.ioff + t);
+  R.flags = nd.flags;
+  return R;
+}
+
+// Colours of the pixels in lanes 0 .. take - 1 (GL pixel (x, j), winner `slot`
+// and sub-triangle q); returns how many leading lanes were shaded.
+
+// Flat scenes: every lane shades its own winner's first normal.
+__device__ __forceinline__ uint32_t band_shade_flat(const pbr_scene_desc& D, const BandFrame& F,
+                                                    const Light& lt, int s, const NodeLds* nodes,
+                                                    int nn, const uint32_t* tab, int lane,
+                                                    uint32_t take, uint32_t slot, float col[4]) {
+  if ((uint32_t)lane < take) {
+    const SlotRef R = band_slot(D, F, s, nodes, nn, tab, slot);
+    float M[16], v[6], nw[3], n[3];
+    load_mat4_global(R.trans + R.row * 16, M);
+    const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
+    const float rgba[4] = {c4.x, c4.y, c4.z, c4.w};
+    load_vertex(D.vertices, R.voff + (int)(R.tri & 0xffu), v);
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
       const float a = M[r * 4 + 0] * v[3] + M[r * 4 + 1] * v[4];
@@ -276,43 +371,140 @@ __device__ __forceinline__ void band_shade(const pbr_scene_desc& D, const BandFr
     }
     normalize3(nw, n);
     shade(n, rgba, lt, col);
-    return;
   }
-  if constexpr (SMOOTH) {
-    float v1[6], v2[6];
-    load_vertex(D.vertices, nd.voff + (int)((tri >> 8) & 0xffu), v1);
-    load_vertex(D.vertices, nd.voff + (int)(tri >> 16), v2);
-    VertRec r[3];
-    vertex_record(M, VP, v, F.W, F.H, F.guard, r[0]);
-    vertex_record(M, VP, v1, F.W, F.H, F.guard, r[1]);
-    vertex_record(M, VP, v2, F.W, F.H, F.guard, r[2]);
-    if ((((r[0].bits & r[1].bits & r[2].bits) >> 1) & 0x3fu) != 0x3fu) {
-      const double px = (double)(256 * x + 128), py = (double)(256 * j + 128);
-      col[0] = col[1] = col[2] = col[3] = 0.0f;
-      band_clipped_colour(kernarg_scene(), F.guard, s, nj, local, q, rgba, lt, px, py, col);
-      return;
-    }
-    // e_k = A_k Px + B_k Py + C_k without the fill-rule bias: edge k runs from
-    // vertex k + 1 to vertex k + 2, and every difference and product is an
-    // exact integer in double
-    const int32_t X[3] = {r[0].X, r[1].X, r[2].X}, Y[3] = {r[0].Y, r[1].Y, r[2].Y};
-    const int32_t cx = 256 * x + 128, cy = 256 * j + 128;
-    float bw[3];
+  return take;
+}
+
+// Runs of pixels with one winner share its vertices: lane 3 u + k transforms
+// vertex k of the u-th run's triangle, and every pixel of the run reads the
+// three back.  At most 21 runs fit a wave, so a pass may shade fewer pixels
+// than it was given.  `heads` is 64 bytes of the wave's LDS.
+constexpr int kShadeRuns = 21;
+__device__ __forceinline__ uint32_t band_shade_smooth(const pbr_scene_desc& D, const BandFrame& F,
+                                                      const Light& lt, int s, const float VP[16],
+                                                      const NodeLds* nodes, int nn,
+                                                      const uint32_t* tab, int lane, uint32_t take,
+                                                      uint32_t slot, int q, int x, int j,
+                                                      uint8_t* heads, float col[4]) {
+  const bool valid = (uint32_t)lane < take;
+  const int prev = from_lane(lane > 0 ? lane - 1 : 0, (int)slot);
+  const bool head = valid && (lane == 0 || (uint32_t)prev != slot);
+  const uint64_t hm = __ballot(head);
+  const int run = __popcll(hm & ((2ull << lane) - 1ull)) - 1;
+  const int runs = min(__popcll(hm), kShadeRuns);
+  if (head) heads[run] = (uint8_t)lane;
+  wave_fence();
+  const int u = (lane * 86) >> 8, k = lane - 3 * u;
+  CVert cv = {};
+  SnapVert sv = {};
+  uint32_t fl = 0;
+  float rgba[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // every lane takes part in the reads of other lanes' slots
+  const uint32_t vslot = (uint32_t)from_lane(u < runs ? (int)heads[u] : 0, (int)slot);
+  if (u < runs) {
+    const SlotRef R = band_slot(D, F, s, nodes, nn, tab, vslot);
+    const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
+    rgba[0] = c4.x;
+    rgba[1] = c4.y;
+    rgba[2] = c4.z;
+    rgba[3] = c4.w;
+    const uint32_t id = k == 0 ? R.tri & 0xffu : (k == 1 ? (R.tri >> 8) & 0xffu : R.tri >> 16);
+    float M[16], vv[6];
+    load_mat4_global(R.trans + R.row * 16, M);
+    load_vertex(D.vertices, R.voff + (int)id, vv);
+    transform_vertex(M, VP, vv, cv);
+    snap_vertex(cv, F.W, F.H, sv);
+    fl = outcode(cv, F.guard) | ((R.flags & 2u) << 5);  // bit 6: flat
+  }
+  const bool mine = valid && run < kShadeRuns;
+  const int src = mine ? 3 * run : 0;
+  int32_t X[3], Y[3];
+  float iw[3], n[3][3];
+  uint32_t code = 0;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int a = (k + 1) % 3, b = (k + 2) % 3;
-      const double e = fma((double)(Y[a] - Y[b]), (double)(cx - X[a]),
-                           (double)(X[b] - X[a]) * (double)(cy - Y[a]));
-      bw[k] = (float)e * r[k].invw;
+  for (int v = 0; v < 3; ++v) {
+    X[v] = from_lane(src + v, sv.X);
+    Y[v] = from_lane(src + v, sv.Y);
+    iw[v] = from_lane(src + v, sv.invw);
+    code |= (uint32_t)from_lane(src + v, (int)fl);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) n[v][c] = from_lane(src + v, cv.n[c]);
+  }
+  float base[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) base[c] = from_lane(src, rgba[c]);
+  const bool flat = (code & 64u) != 0u;
+
+  // winners that straddle a clip plane: their polygons, four slots at a time
+  bool clipped = mine && !flat && (code & (uint32_t)kOutMask) != 0u;
+  for (uint64_t cm = __ballot(clipped); cm; cm = __ballot(clipped)) {
+    uint32_t gs = 0;
+    int group = -1, count = 0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (!cm) break;
+      const uint32_t sl = (uint32_t)__builtin_amdgcn_readlane(
+          (int)slot, __ffsll((unsigned long long)cm) - 1);
+      if ((lane >> 4) == g) gs = sl;
+      const bool hit = clipped && slot == sl;
+      if (hit) group = g;
+      cm &= ~__ballot(hit);
+      ++count;
     }
-    float n[3];
+    CVert p = {};
+    int pn = 0;
+    if ((lane >> 4) < count) {
+      pn = 3;
+      if ((lane & 15) < 3) {
+        const SlotRef R = band_slot(D, F, s, nodes, nn, tab, gs);
+        group_vertex(D, R.trans, R.row, R.voff, R.tri, VP, lane, p);
+      }
+    }
+    float v[7] = {p.p[0], p.p[1], p.p[2], p.p[3], p.n[0], p.n[1], p.n[2]};
+    clip_groups<7>(v, pn, F.guard, lane);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) p.p[c] = v[c];
+    SnapVert ps;
+    snap_vertex(p, F.W, F.H, ps);
+    const int at = group < 0 ? 0 : group * 16;
+    const int from[3] = {at, at + q + 1, at + q + 2};
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const int px = from_lane(from[e], ps.X), py = from_lane(from[e], ps.Y);
+      const float pw = from_lane(from[e], ps.invw);
+      float pnm[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) pnm[c] = from_lane(from[e], v[4 + c]);
+      if (group >= 0) {
+        X[e] = px;
+        Y[e] = py;
+        iw[e] = pw;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) n[e][c] = pnm[c];
+      }
+    }
+    clipped = clipped && group < 0;
+  }
+  if (mine) {
+    // weights e_k / w_k, e_k the edge function without the fill-rule bias:
+    // every difference and product is an exact integer in double
+    const int32_t cx = 256 * x + 128, cy = 256 * j + 128;
+    float bw[3], nn3[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const int a = (e + 1) % 3, b = (e + 2) % 3;
+      const double ev = fma((double)(Y[a] - Y[b]), (double)(cx - X[a]),
+                            (double)(X[b] - X[a]) * (double)(cy - Y[a]));
+      bw[e] = (float)ev * iw[e];
+    }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const float a = bw[0] * r[0].n[c] + bw[1] * r[1].n[c];
-      n[c] = a + bw[2] * r[2].n[c];
+      const float a = bw[0] * n[0][c] + bw[1] * n[1][c];
+      nn3[c] = flat ? n[0][c] : a + bw[2] * n[2][c];
     }
-    shade(n, rgba, lt, col);
+    shade(nn3, base, lt, col);
   }
+  return (uint32_t)__popcll(__ballot(mine));
 }
 
 // Byte c of each of four packed RGBA8 colours -> one dword.
@@ -325,8 +517,7 @@ __device__ __forceinline__ uint32_t band_gather(uint32_t p0, uint32_t p1, uint32
 
 // OM: 0 uint8, 1 bf16, 2 float32 colours.  Dynamic LDS: pixel keys
 // [th][W], per wave a vertex table (int2 [verts], float depth [verts]) and a
-// queue of 128 bytes, then the index table.  D stays the first parameter: the
-// out-of-line clipper reads it through the kernarg segment (kernarg_scene).
+// queue of 128 bytes, then the index table.
 template <bool SMOOTH, int OM>
 __global__ __launch_bounds__(kBandBlock)
 __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_frame_out O,
@@ -393,6 +584,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       e.chunk0 = ic - nchunk;
       e.cnt = cnt;
       e.ntri = max(me.num_triangles, 1);
+      e.inv_nt = 1.0f / (float)e.ntri;
       e.voff = me.vertex_offset;
       e.ioff = me.index_offset;
       e.ips = nd.instances_per_scene;
@@ -444,16 +636,16 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       float M[16], vv[6];
       load_mat4_global(nd.transforms + (row0 + di) * 16, M);
       load_vertex(D.vertices, me.vertex_offset + (int)k, vv);
-      VertRec r;
-      vertex_record(M, VP, vv, W, H, F.guard, r);
-      const uint32_t oc = (r.bits >> 7) & 0x3fu;
-      const bool in = ((r.bits >> 1) & 0x3fu) == 0x3fu;
+      CVert cv;
+      transform_vertex(M, VP, vv, cv);
+      SnapVert r;
+      snap_vertex(cv, W, H, r);
+      const uint32_t oc = outcode(cv, F.guard);
       vxy[v] = make_int2((int)(((uint32_t)r.X << 6) | oc),
-                         (int)(((uint32_t)r.Y << 6) | (in ? (uint32_t)kInAll : 0u) |
-                               (r.bits & 1u)));
+                         (int)(((uint32_t)r.Y << 1) | (r.ok ? 0u : 1u)));
       vd[v] = r.d;
       uint32_t side = 0;
-      if (in && (r.bits & 1u))
+      if (oc == 0u && r.ok)
         side = (r.Y < ylo ? 64u : 0u) | (r.Y > yhi ? 128u : 0u) | (r.X < 128 ? 256u : 0u) |
                (r.X > xhi ? 512u : 0u);
       out &= oc | side;
@@ -465,24 +657,50 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     wave_fence();
 
     // triangles: test, queue, set up 64 queued ones at a time, rasterise.
-    // Sub-triangles of clipped ones take the place of a set-up round.
-    uint32_t pend = 0, q0 = 0;
-    int nsub = 0;  // vertices of this lane's clip polygon
-    int sub = 0, subs = 0;  // sub-triangle rounds done and due
-    uint32_t clip_slot = 0;
-    CVert poly[kMaxPoly];
+    // Those that straddle a clip plane are clipped four at a time.
+    uint32_t pend = 0, q0 = 0, clip_u = 0;
+    uint64_t clipm = 0;  // lanes whose clip_u awaits its clipping
     for (;;) {
       FixTri T;
       bool has = false;
       uint32_t rank = 0;
-      if (sub < subs) {
-        const int q = sub++;
-        if (q + 2 < nsub) {
-          FixTri S;
-          has = band_clip_sub(poly, q, W, H, t.j0, t.j1, &S);
-          T = S;
-          rank = (clip_slot << 3) | (uint32_t)q;
+      if (clipm) {
+        int from = -1;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (!clipm) break;
+          if ((lane >> 4) == k) from = __ffsll((unsigned long long)clipm) - 1;
+          clipm &= clipm - 1ull;
         }
+        const uint32_t u = (uint32_t)from_lane(from < 0 ? 0 : from, (int)clip_u);
+        int pn = from < 0 ? 0 : 3;
+        CVert cv = {};
+        if (pn && (lane & 15) < 3) {
+          const uint32_t di = (u * bn.inv_nt) >> 16, tt = u - di * nt;
+          const uint32_t tri = F.ntab ? tab[me.index_offset + (int)tt]
+                                      : pool_triangle(D, me.index_offset + (int)tt);
+          group_vertex(D, nd.transforms, row0 + di, me.vertex_offset, tri, VP, lane, cv);
+        }
+        clip_groups<4>(cv.p, pn, F.guard, lane);
+        SnapVert S;
+        snap_vertex(cv, W, H, S);
+        const int lost = 0x7fffffff;  // X of a vertex that did not snap
+        const int X = S.ok ? S.X : lost;
+        const int at = lane & 48, q = lane & 15;
+        const bool tri = q + 2 < pn;
+        const int f1 = tri ? at + q + 1 : at, f2 = tri ? at + q + 2 : at;
+        SnapVert V[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const int f = k == 0 ? at : (k == 1 ? f1 : f2);
+          V[k].X = from_lane(f, X);
+          V[k].Y = from_lane(f, S.Y);
+          V[k].d = from_lane(f, S.d);
+          V[k].invw = 0.0f;
+          V[k].ok = V[k].X != lost;
+        }
+        has = tri && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
+        rank = ((slot0 + u) << 3) | (uint32_t)q;
       } else if (pend >= 64u || (q0 >= n && pend > 0u)) {
         const uint32_t take = min(pend, 64u);
         if ((uint32_t)lane < take) {
@@ -494,9 +712,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu),
                          ic = vb + (tri >> 16);
           const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
-          const SnapVert sa = {a.x >> 6, a.y >> 6, vd[ia], 0.0f, true};
-          const SnapVert sb = {b.x >> 6, b.y >> 6, vd[ib], 0.0f, true};
-          const SnapVert sc = {cc.x >> 6, cc.y >> 6, vd[ic], 0.0f, true};
+          const SnapVert sa = {a.x >> 6, a.y >> 1, vd[ia], 0.0f, true};
+          const SnapVert sb = {b.x >> 6, b.y >> 1, vd[ib], 0.0f, true};
+          const SnapVert sc = {cc.x >> 6, cc.y >> 1, vd[ic], 0.0f, true};
           has = setup_snapped(sa, sb, sc, W, H, t.j0, t.j1, T);
           rank = (slot0 + u) << 3;
         }
@@ -516,13 +734,12 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           const uint32_t vb = di * nv;
           const int2 a = vxy[vb + (tri & 0xffu)], b = vxy[vb + ((tri >> 8) & 0xffu)],
                      cc = vxy[vb + (tri >> 16)];
-          const int fl = a.y & b.y & cc.y;
-          if ((a.x & b.x & cc.x & 0x3f) == 0) {
-            if (!(fl & kInAll)) {
+          if ((a.x & b.x & cc.x & kOutMask) == 0) {
+            if ((a.x | b.x | cc.x) & kOutMask) {
               clip = true;
-            } else if (fl & kSnapped) {
+            } else if (!((a.y | b.y | cc.y) & 1)) {
               const int32_t X0 = a.x >> 6, X1 = b.x >> 6, X2 = cc.x >> 6;
-              const int32_t Y0 = a.y >> 6, Y1 = b.y >> 6, Y2 = cc.y >> 6;
+              const int32_t Y0 = a.y >> 1, Y1 = b.y >> 1, Y2 = cc.y >> 1;
               const double area = (double)(X1 - X0) * (double)(Y2 - Y0) -
                                   (double)(X2 - X0) * (double)(Y1 - Y0);
               const int32_t xmin = min(X0, min(X1, X2)), xmax = max(X0, max(X1, X2));
@@ -537,23 +754,21 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         if (live) qu[pend + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)u;
         pend += (uint32_t)__popcll(m);
         q0 += 64u;
-        if (__ballot(clip)) {
-          nsub = 0;
-          if (clip) {
-            clip_slot = slot0 + u;
-            nsub = band_clip(kernarg_scene(), F.guard, t.s, j, clip_slot - base, poly);
-          }
-          sub = subs = 0;
-          while (__ballot(subs + 2 < nsub)) ++subs;
-        }
+        clip_u = u;
+        clipm = __ballot(clip);
         wave_fence();
         continue;
       } else {
         break;
       }
       // rasterise the lanes' triangles
-      const bool small = has && (T.i1 - T.i0 + 1) * (T.j1 - T.j0 + 1) <= kSmallPixels;
+      const bool fits =  // edge values fit 32 bits
+          has &&
+          max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
+          max(T.Y[0], max(T.Y[1], T.Y[2])) - min(T.Y[0], min(T.Y[1], T.Y[2])) <= kIntExtent;
+      const bool small = fits && (T.i1 - T.i0 + 1) * (T.j1 - T.j0 + 1) <= kSmallPixels;
       if (small) band_raster_lane(pix, t, T, rank);
+      const uint64_t fm = __ballot(fits);
       for (uint64_t m = __ballot(has && !small); m; m &= m - 1ull) {
         const int l = __ffsll((unsigned long long)m) - 1;
         FixTri U;
@@ -570,7 +785,11 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         U.j0 = rl(T.j0, l);
         U.j1 = rl(T.j1, l);
         U.bias = (uint32_t)rl((int)T.bias, l);
-        band_raster_wave(pix, t, lane, U, (uint32_t)rl((int)rank, l));
+        const uint32_t ur = (uint32_t)rl((int)rank, l);
+        if ((fm >> l) & 1ull)
+          band_raster_wave<int32_t>(pix, t, lane, U, ur);
+        else
+          band_raster_wave<double>(pix, t, lane, U, ur);
       }
     }
     wave_fence();  // the next chunk rewrites the table
@@ -591,6 +810,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           ((unsigned long long)(bf16_rne(bgc[2]) | (bf16_rne(bgc[3]) << 16)) << 32);
   float* fout = reinterpret_cast<float*>(O.color) + (size_t)t.s * C * plane + pix0;  // OM 2
   uint16_t* pq = reinterpret_cast<uint16_t*>(vxy);  // covered pixels awaiting their shading
+  const float inv_w = 1.0f / (float)W;
   uint32_t pend = 0;
   for (int p0 = wave * 64; p0 < npx || pend > 0u;) {
     if (p0 < npx && pend < 64u) {
@@ -618,21 +838,25 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       continue;
     }
     const uint32_t take = min(pend, 64u);
-    if ((uint32_t)lane < take) {
-      const int p = pq[lane];
-      const uint32_t rank = (uint32_t)pix[p];
-      int y = (int)((float)p * (1.0f / (float)W));
-      int x = p - y * W;
-      if (x < 0) {
-        --y;
-        x += W;
-      } else if (x >= W) {
-        ++y;
-        x -= W;
-      }
-      float col[4];
-      band_shade<SMOOTH>(D, F, lt, t.s, VP, nodes, nn, tab, rank >> 3, (int)(rank & 7u), x,
-                         t.j1 - y, col);
+    const int p = (uint32_t)lane < take ? (int)pq[lane] : 0;
+    const uint32_t rank = (uint32_t)pix[p];
+    int y = (int)((float)p * inv_w);
+    int x = p - y * W;
+    if (x < 0) {
+      --y;
+      x += W;
+    } else if (x >= W) {
+      ++y;
+      x -= W;
+    }
+    float col[4];
+    uint32_t done;
+    if constexpr (SMOOTH)
+      done = band_shade_smooth(D, F, lt, t.s, VP, nodes, nn, tab, lane, take, rank >> 3,
+                               (int)(rank & 7u), x, t.j1 - y, qu, col);
+    else
+      done = band_shade_flat(D, F, lt, t.s, nodes, nn, tab, lane, take, rank >> 3, col);
+    if ((uint32_t)lane < done) {
       if constexpr (OM == 0) {
         pix[p] = pack_rgba8(col);
       } else if constexpr (OM == 1) {
@@ -644,11 +868,14 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           if (ch < C) fout[(size_t)ch * plane + p] = col[ch];
       }
     }
-    uint16_t rest = 0;
-    if ((uint32_t)lane + 64u < pend) rest = pq[lane + 64];
+    const uint32_t ra = (uint32_t)lane + done, rb = ra + 64u;
+    uint16_t na = 0, nb = 0;
+    if (ra < pend) na = pq[ra];
+    if (rb < pend) nb = pq[rb];
     wave_fence();
-    if ((uint32_t)lane + 64u < pend) pq[lane] = rest;
-    pend -= take;
+    if (ra < pend) pq[lane] = na;
+    if (rb < pend) pq[lane + 64] = nb;
+    pend -= done;
     wave_fence();
   }
   if constexpr (OM == 2) return;

@@ -398,13 +398,11 @@ struct VertRec {
 };
 static_assert(sizeof(VertRec) == 32, "VertRec is 32 bytes");
 
-// (a) + per-vertex (b) of model-space vertex vv (px py pz nx ny nz) under
-// instance matrix M and the scene's VP: the same products, snap and plane
-// distances fetch_node_triangle, snap_vertex and clip_class evaluate.
-__device__ __forceinline__ void vertex_record(const float M[16], const float VP[16],
-                                              const float* vv, int W, int H, float guard,
-                                              VertRec& out) {
-  CVert cv;
+// (a) of model-space vertex vv (px py pz nx ny nz) under instance matrix M
+// and the scene's VP: clip position and world normal, the products
+// fetch_node_triangle evaluates.
+__device__ __forceinline__ void transform_vertex(const float M[16], const float VP[16],
+                                                 const float* vv, CVert& cv) {
   float wp[4], nw[3];
 #pragma unroll
   for (int rr = 0; rr < 4; ++rr) {
@@ -424,6 +422,15 @@ __device__ __forceinline__ void vertex_record(const float M[16], const float VP[
     nw[rr] = a + M[rr * 4 + 2] * vv[5];
   }
   normalize3(nw, cv.n);
+}
+
+// transform_vertex + per-vertex (b): the same snap and plane distances
+// snap_vertex and clip_class evaluate.
+__device__ __forceinline__ void vertex_record(const float M[16], const float VP[16],
+                                              const float* vv, int W, int H, float guard,
+                                              VertRec& out) {
+  CVert cv;
+  transform_vertex(M, VP, vv, cv);
   SnapVert sv;
   snap_vertex(cv, W, H, sv);
   uint32_t bits = sv.ok ? 1u : 0u;
