@@ -39,8 +39,8 @@ namespace {
 constexpr int kBandBlock = 512;
 constexpr int kBandWaves = kBandBlock / 64;
 constexpr int kBandVerts = 136;   // vertices a wave's table holds at most
-constexpr int kBandTris = 256;    // triangles of one mesh (8-bit queue entries)
-constexpr int kBandTable = 512;   // triangles of the LDS index table at most
+constexpr int kBandTris = 256;    // triangles of one chunk (8-bit queue entries)
+constexpr int kBandTable = 512;   // triangles of all meshes (LDS index table) at most
 constexpr int kMaxBands = 4;      // bands per scene at most: each repeats the vertex work
 constexpr int kBandPixels = 8192;
 constexpr int kBandLds = 80 * 1024;  // half a CU's LDS: two workgroups share a CU
@@ -61,7 +61,8 @@ struct BandFrame {
   uint32_t budget;     // slots drawn of the whole batch at most
   int uniform;         // 1: no node has per-scene counts
   int verts;           // entries of a wave's vertex table
-  int ntab;            // triangles in the LDS index table (0: read from memory)
+  int ntab;            // triangles in the LDS index table
+  int vec;             // 1: four pixels of a plane are whole aligned dwords / float4s
   BandNode node[PBR_MAX_NODES];
 };
 
@@ -321,9 +322,8 @@ struct SlotRef {
   uint32_t flags;  // the node's (NodeLds)
 };
 
-__device__ __forceinline__ SlotRef band_slot(const pbr_scene_desc& D, const BandFrame& F, int s,
-                                             const NodeLds* nodes, int nn, const uint32_t* tab,
-                                             uint32_t slot) {
+__device__ __forceinline__ SlotRef band_slot(int s, const NodeLds* nodes, int nn,
+                                             const uint32_t* tab, uint32_t slot) {
   int nj = 0;
   for (int k = 1; k < nn; ++k) nj = slot >= nodes[k].base ? k : nj;
   const NodeLds& nd = nodes[nj];
@@ -344,7 +344,7 @@ __device__ __forceinline__ SlotRef band_slot(const pbr_scene_desc& D, const Band
   R.cols = nd.cols;
   R.row = (nd.flags & 1u) ? (size_t)i : (size_t)s * (size_t)nd.ips + i;
   R.voff = nd.voff;
-  R.tri = F.ntab ? tab[nd.ioff + t] : pool_triangle(D, nd.ioff + t);
+  R.tri = tab[nd.ioff + t];
   R.flags = nd.flags;
   return R;
 }
@@ -353,12 +353,12 @@ __device__ __forceinline__ SlotRef band_slot(const pbr_scene_desc& D, const Band
 // and sub-triangle q); returns how many leading lanes were shaded.
 
 // Flat scenes: every lane shades its own winner's first normal.
-__device__ __forceinline__ uint32_t band_shade_flat(const pbr_scene_desc& D, const BandFrame& F,
-                                                    const Light& lt, int s, const NodeLds* nodes,
-                                                    int nn, const uint32_t* tab, int lane,
-                                                    uint32_t take, uint32_t slot, float col[4]) {
+__device__ __forceinline__ uint32_t band_shade_flat(const pbr_scene_desc& D, const Light& lt,
+                                                    int s, const NodeLds* nodes, int nn,
+                                                    const uint32_t* tab, int lane, uint32_t take,
+                                                    uint32_t slot, float col[4]) {
   if ((uint32_t)lane < take) {
-    const SlotRef R = band_slot(D, F, s, nodes, nn, tab, slot);
+    const SlotRef R = band_slot(s, nodes, nn, tab, slot);
     float M[16], v[6], nw[3], n[3];
     load_mat4_global(R.trans + R.row * 16, M);
     const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
@@ -402,7 +402,7 @@ __device__ __forceinline__ uint32_t band_shade_smooth(const pbr_scene_desc& D, c
   // every lane takes part in the reads of other lanes' slots
   const uint32_t vslot = (uint32_t)from_lane(u < runs ? (int)heads[u] : 0, (int)slot);
   if (u < runs) {
-    const SlotRef R = band_slot(D, F, s, nodes, nn, tab, vslot);
+    const SlotRef R = band_slot(s, nodes, nn, tab, vslot);
     const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
     rgba[0] = c4.x;
     rgba[1] = c4.y;
@@ -456,7 +456,7 @@ __device__ __forceinline__ uint32_t band_shade_smooth(const pbr_scene_desc& D, c
     if ((lane >> 4) < count) {
       pn = 3;
       if ((lane & 15) < 3) {
-        const SlotRef R = band_slot(D, F, s, nodes, nn, tab, gs);
+        const SlotRef R = band_slot(s, nodes, nn, tab, gs);
         group_vertex(D, R.trans, R.row, R.voff, R.tri, VP, lane, p);
       }
     }
@@ -516,14 +516,14 @@ __device__ __forceinline__ uint32_t band_gather(uint32_t p0, uint32_t p1, uint32
 }
 
 // OM: 0 uint8, 1 bf16, 2 float32 colours.  Dynamic LDS: pixel keys
-// [th][W], per wave a vertex table (int2 [verts], float depth [verts]) and a
-// queue of 128 bytes, then the index table.
+// [th][W], the waves' vertex tables (int2 [verts], float depth [verts]) and
+// triangle queues, then the index table.
 template <bool SMOOTH, int OM>
 __global__ __launch_bounds__(kBandBlock)
 __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_frame_out O,
                                                           BandFrame F, const uint32_t* scene_off,
                                                           uint32_t* hdr, Light lt, float4 bg) {
-  extern __shared__ unsigned long long pix[];
+  extern __shared__ __align__(16) unsigned long long pix[];
   __shared__ NodeLds nodes[PBR_MAX_NODES];
   __shared__ uint32_t next_chunk, total_chunks;
   const int tid = (int)threadIdx.x;
@@ -537,15 +537,13 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   t.j1 = H - 1 - yo0;
   t.j0 = t.j1 - (rows - 1);
   const int npx = rows * W;
-  int2* vxy = reinterpret_cast<int2*>(pix + F.th * W) + wave * F.verts;
-  float* vd = reinterpret_cast<float*>(reinterpret_cast<int2*>(pix + F.th * W) +
-                                       kBandWaves * F.verts) + wave * F.verts;
-  uint8_t* qu = reinterpret_cast<uint8_t*>(reinterpret_cast<int2*>(pix + F.th * W) +
-                                           kBandWaves * F.verts) +
-                sizeof(float) * kBandWaves * F.verts + wave * 128;
-  uint32_t* tab = reinterpret_cast<uint32_t*>(
-      reinterpret_cast<uint8_t*>(reinterpret_cast<int2*>(pix + F.th * W) + kBandWaves * F.verts) +
-      sizeof(float) * kBandWaves * F.verts + kBandWaves * 128);
+  int2* tables = reinterpret_cast<int2*>(pix + ((F.th * W + 1) & ~1));
+  int2* vxy = tables + wave * F.verts;
+  unsigned char* after = reinterpret_cast<unsigned char*>(tables + kBandWaves * F.verts);
+  float* vd = reinterpret_cast<float*>(after) + wave * F.verts;
+  after += sizeof(float) * (size_t)kBandWaves * F.verts;
+  uint8_t* qu = after + wave * kBandTris;
+  uint32_t* tab = reinterpret_cast<uint32_t*>(after + kBandWaves * kBandTris);
 
   if (F.uniform && blockIdx.x == 0 && tid == 0) hdr[0] = 0u;  // no overflow
   // slots of this scene that are drawn (all, unless the batch exceeds its
@@ -558,7 +556,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     const uint32_t o = min(scene_off[t.s], F.budget), e = min(scene_off[t.s + 1], F.budget);
     ndraw = e > o ? e - o : 0u;
   }
-  for (int p = tid; p < npx; p += kBandBlock) pix[p] = (unsigned long long)kDepthOne << 32;
+  // two keys per store (the key area is padded to an even count)
+  for (int p = tid; p < (npx + 1) / 2; p += kBandBlock)
+    reinterpret_cast<uint4*>(pix)[p] = make_uint4(0u, kDepthOne, 0u, kDepthOne);
   for (int q = tid; q < F.ntab; q += kBandBlock) tab[q] = pool_triangle(D, q);
   if (wave == 0) {
     uint32_t cnt = 0, nslot = 0, nchunk = 0;
@@ -614,15 +614,19 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     int j = 0;
     for (int k = 1; k < nn; ++k)
       j = c >= (uint32_t)__builtin_amdgcn_readfirstlane((int)nodes[k].chunk0) ? k : j;
+    // the node's facts in scalar registers, loaded once per chunk
     const pbr_node& nd = D.nodes[j];
     const pbr_mesh& me = D.meshes[nd.mesh];
-    const BandNode bn = F.node[j];
+    const uint32_t group = F.node[j].group, inv_nv = F.node[j].inv_nv, inv_nt = F.node[j].inv_nt;
+    const float* trans = nd.transforms;
+    const int voff = me.vertex_offset;
+    const uint32_t nt = (uint32_t)me.num_triangles, nv = (uint32_t)me.num_vertices;
+    const uint32_t* mtab = tab + me.index_offset;
     const uint32_t cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)nodes[j].cnt);
     const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)nodes[j].base);
-    const uint32_t i0 = (c - (uint32_t)__builtin_amdgcn_readfirstlane((int)nodes[j].chunk0)) *
-                        bn.group;
-    const uint32_t g = min(bn.group, cnt - i0);
-    const uint32_t nt = (uint32_t)me.num_triangles, nv = (uint32_t)me.num_vertices;
+    const uint32_t i0 =
+        (c - (uint32_t)__builtin_amdgcn_readfirstlane((int)nodes[j].chunk0)) * group;
+    const uint32_t g = min(group, cnt - i0);
     const uint32_t slot0 = base + i0 * nt;
     if (slot0 >= ndraw) continue;
     const uint32_t n = min(g * nt, ndraw - slot0);
@@ -631,11 +635,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     // vertices of the chunk into the wave's table; `out` gathers what all of
     // them lie outside of (bits 0-5 clip planes, 6-9 the band's sides)
     uint32_t out = 0x3ffu;
-    for (uint32_t v = (uint32_t)lane; v < g * nv; v += 64u) {
-      const uint32_t di = (v * bn.inv_nv) >> 16, k = v - di * nv;
-      float M[16], vv[6];
-      load_mat4_global(nd.transforms + (row0 + di) * 16, M);
-      load_vertex(D.vertices, me.vertex_offset + (int)k, vv);
+    auto vertex = [&](uint32_t v, uint32_t k, const float* M) {
+      float vv[6];
+      load_vertex(D.vertices, voff + (int)k, vv);
       CVert cv;
       transform_vertex(M, VP, vv, cv);
       SnapVert r;
@@ -644,11 +646,21 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       vxy[v] = make_int2((int)(((uint32_t)r.X << 6) | oc),
                          (int)(((uint32_t)r.Y << 1) | (r.ok ? 0u : 1u)));
       vd[v] = r.d;
-      uint32_t side = 0;
-      if (oc == 0u && r.ok)
-        side = (r.Y < ylo ? 64u : 0u) | (r.Y > yhi ? 128u : 0u) | (r.X < 128 ? 256u : 0u) |
-               (r.X > xhi ? 512u : 0u);
-      out &= oc | side;
+      const uint32_t side = (r.Y < ylo ? 64u : 0u) | (r.Y > yhi ? 128u : 0u) |
+                            (r.X < 128 ? 256u : 0u) | (r.X > xhi ? 512u : 0u);
+      out &= oc | (oc == 0u && r.ok ? side : 0u);
+    };
+    if (group == 1u) {
+      float M[16];
+      load_mat4_uniform(trans + row0 * 16, M);
+      for (uint32_t v = (uint32_t)lane; v < nv; v += 64u) vertex(v, v, M);
+    } else {
+      for (uint32_t v = (uint32_t)lane; v < g * nv; v += 64u) {
+        const uint32_t di = __umul24(v, inv_nv) >> 16;
+        float M[16];
+        load_mat4_global(trans + (row0 + di) * 16, M);
+        vertex(v, v - __umul24(di, nv), M);
+      }
     }
     bool gone = false;
 #pragma unroll
@@ -656,59 +668,51 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     if (gone) continue;
     wave_fence();
 
-    // triangles: test, queue, set up 64 queued ones at a time, rasterise.
-    // Those that straddle a clip plane are clipped four at a time.
-    uint32_t pend = 0, q0 = 0, clip_u = 0;
-    uint64_t clipm = 0;  // lanes whose clip_u awaits its clipping
-    for (;;) {
+    // triangles: every one is tested on its table entries; the live ones are
+    // queued from the front, those that straddle a clip plane from the back
+    uint32_t live_n = 0, clip_n = 0;
+    for (uint32_t q0 = 0; q0 < n; q0 += 64u) {
+      const uint32_t u = min(q0 + (uint32_t)lane, n - 1u);
+      const uint32_t di = __umul24(u, inv_nt) >> 16;
+      const uint32_t tri = mtab[u - __umul24(di, nt)];
+      const int2* vt = vxy + __umul24(di, nv);
+      const int2 a = vt[tri & 0xffu], b = vt[(tri >> 8) & 0xffu], cc = vt[tri >> 16];
+      const int32_t X0 = a.x >> 6, X1 = b.x >> 6, X2 = cc.x >> 6;
+      const int32_t Y0 = a.y >> 1, Y1 = b.y >> 1, Y2 = cc.y >> 1;
+      const double area = (double)(X1 - X0) * (double)(Y2 - Y0) -
+                          (double)(X2 - X0) * (double)(Y1 - Y0);
+      const int32_t a0 = max((min(X0, min(X1, X2)) + 127) >> 8, 0);
+      const int32_t a1 = min((max(X0, max(X1, X2)) - 128) >> 8, W - 1);
+      const int32_t b0 = max((min(Y0, min(Y1, Y2)) + 127) >> 8, t.j0);
+      const int32_t b1 = min((max(Y0, max(Y1, Y2)) - 128) >> 8, t.j1);
+      const bool here = q0 + (uint32_t)lane < n;
+      const uint32_t any = (uint32_t)(a.x | b.x | cc.x) & (uint32_t)kOutMask;
+      const bool clip = here && any != 0u && (a.x & b.x & cc.x & kOutMask) == 0;
+      const bool live = here && any == 0u && ((a.y | b.y | cc.y) & 1) == 0 && area > 0.0 &&
+                        a0 <= a1 && b0 <= b1;
+      const uint64_t ml = __ballot(live), mc = __ballot(clip);
+      const uint64_t below = (1ull << lane) - 1ull;
+      if (live) qu[live_n + (uint32_t)__popcll(ml & below)] = (uint8_t)u;
+      live_n += (uint32_t)__popcll(ml);
+      if (mc) {
+        if (clip) qu[kBandTris - 1u - (clip_n + (uint32_t)__popcll(mc & below))] = (uint8_t)u;
+        clip_n += (uint32_t)__popcll(mc);
+      }
+    }
+    wave_fence();
+
+    // 64 live triangles are set up at a time, then clipped ones four at a
+    // time (a lane per sub-triangle); each set is rasterised at once
+    for (uint32_t k0 = 0; k0 < live_n + clip_n;) {
       FixTri T;
       bool has = false;
       uint32_t rank = 0;
-      if (clipm) {
-        int from = -1;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          if (!clipm) break;
-          if ((lane >> 4) == k) from = __ffsll((unsigned long long)clipm) - 1;
-          clipm &= clipm - 1ull;
-        }
-        const uint32_t u = (uint32_t)from_lane(from < 0 ? 0 : from, (int)clip_u);
-        int pn = from < 0 ? 0 : 3;
-        CVert cv = {};
-        if (pn && (lane & 15) < 3) {
-          const uint32_t di = (u * bn.inv_nt) >> 16, tt = u - di * nt;
-          const uint32_t tri = F.ntab ? tab[me.index_offset + (int)tt]
-                                      : pool_triangle(D, me.index_offset + (int)tt);
-          group_vertex(D, nd.transforms, row0 + di, me.vertex_offset, tri, VP, lane, cv);
-        }
-        clip_groups<4>(cv.p, pn, F.guard, lane);
-        SnapVert S;
-        snap_vertex(cv, W, H, S);
-        const int lost = 0x7fffffff;  // X of a vertex that did not snap
-        const int X = S.ok ? S.X : lost;
-        const int at = lane & 48, q = lane & 15;
-        const bool tri = q + 2 < pn;
-        const int f1 = tri ? at + q + 1 : at, f2 = tri ? at + q + 2 : at;
-        SnapVert V[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const int f = k == 0 ? at : (k == 1 ? f1 : f2);
-          V[k].X = from_lane(f, X);
-          V[k].Y = from_lane(f, S.Y);
-          V[k].d = from_lane(f, S.d);
-          V[k].invw = 0.0f;
-          V[k].ok = V[k].X != lost;
-        }
-        has = tri && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
-        rank = ((slot0 + u) << 3) | (uint32_t)q;
-      } else if (pend >= 64u || (q0 >= n && pend > 0u)) {
-        const uint32_t take = min(pend, 64u);
-        if ((uint32_t)lane < take) {
-          const uint32_t u = qu[lane];
-          const uint32_t di = (u * bn.inv_nt) >> 16, tt = u - di * nt;
-          const uint32_t tri = F.ntab ? tab[me.index_offset + (int)tt]
-                                      : pool_triangle(D, me.index_offset + (int)tt);
-          const uint32_t vb = di * nv;
+      if (k0 < live_n) {
+        if (k0 + (uint32_t)lane < live_n) {
+          const uint32_t u = qu[k0 + (uint32_t)lane];
+          const uint32_t di = __umul24(u, inv_nt) >> 16;
+          const uint32_t tri = mtab[u - __umul24(di, nt)];
+          const uint32_t vb = __umul24(di, nv);
           const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu),
                          ic = vb + (tri >> 16);
           const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
@@ -718,50 +722,38 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           has = setup_snapped(sa, sb, sc, W, H, t.j0, t.j1, T);
           rank = (slot0 + u) << 3;
         }
-        uint8_t rest = 0;
-        if ((uint32_t)lane + 64u < pend) rest = qu[lane + 64];
-        wave_fence();
-        if ((uint32_t)lane + 64u < pend) qu[lane] = rest;
-        pend -= take;
-        wave_fence();
-      } else if (q0 < n) {
-        const uint32_t u = q0 + (uint32_t)lane;
-        bool live = false, clip = false;
-        if (u < n) {
-          const uint32_t di = (u * bn.inv_nt) >> 16, tt = u - di * nt;
-          const uint32_t tri = F.ntab ? tab[me.index_offset + (int)tt]
-                                      : pool_triangle(D, me.index_offset + (int)tt);
-          const uint32_t vb = di * nv;
-          const int2 a = vxy[vb + (tri & 0xffu)], b = vxy[vb + ((tri >> 8) & 0xffu)],
-                     cc = vxy[vb + (tri >> 16)];
-          if ((a.x & b.x & cc.x & kOutMask) == 0) {
-            if ((a.x | b.x | cc.x) & kOutMask) {
-              clip = true;
-            } else if (!((a.y | b.y | cc.y) & 1)) {
-              const int32_t X0 = a.x >> 6, X1 = b.x >> 6, X2 = cc.x >> 6;
-              const int32_t Y0 = a.y >> 1, Y1 = b.y >> 1, Y2 = cc.y >> 1;
-              const double area = (double)(X1 - X0) * (double)(Y2 - Y0) -
-                                  (double)(X2 - X0) * (double)(Y1 - Y0);
-              const int32_t xmin = min(X0, min(X1, X2)), xmax = max(X0, max(X1, X2));
-              const int32_t ymin = min(Y0, min(Y1, Y2)), ymax = max(Y0, max(Y1, Y2));
-              const int32_t a0 = max((xmin + 127) >> 8, 0), a1 = min((xmax - 128) >> 8, W - 1);
-              const int32_t b0 = max((ymin + 127) >> 8, t.j0), b1 = min((ymax - 128) >> 8, t.j1);
-              live = area > 0.0 && a0 <= a1 && b0 <= b1;
-            }
-          }
-        }
-        const uint64_t m = __ballot(live);
-        if (live) qu[pend + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)u;
-        pend += (uint32_t)__popcll(m);
-        q0 += 64u;
-        clip_u = u;
-        clipm = __ballot(clip);
-        wave_fence();
-        continue;
+        k0 = min(k0 + 64u, live_n);
       } else {
-        break;
+        const uint32_t k = k0 - live_n + (uint32_t)(lane >> 4);
+        int pn = k < clip_n ? 3 : 0;
+        const uint32_t u = qu[kBandTris - 1u - min(k, clip_n - 1u)];
+        CVert cv = {};
+        if (pn && (lane & 15) < 3) {
+          const uint32_t di = __umul24(u, inv_nt) >> 16;
+          group_vertex(D, trans, row0 + di, voff, mtab[u - __umul24(di, nt)], VP, lane, cv);
+        }
+        clip_groups<4>(cv.p, pn, F.guard, lane);
+        SnapVert S;
+        snap_vertex(cv, W, H, S);
+        const int lost = 0x7fffffff;  // X of a vertex that did not snap
+        const int X = S.ok ? S.X : lost;
+        const int at = lane & 48, q = lane & 15;
+        const bool sub = q + 2 < pn;
+        const int f1 = sub ? at + q + 1 : at, f2 = sub ? at + q + 2 : at;
+        SnapVert V[3];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const int f = e == 0 ? at : (e == 1 ? f1 : f2);
+          V[e].X = from_lane(f, X);
+          V[e].Y = from_lane(f, S.Y);
+          V[e].d = from_lane(f, S.d);
+          V[e].invw = 0.0f;
+          V[e].ok = V[e].X != lost;
+        }
+        has = sub && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
+        rank = ((slot0 + u) << 3) | (uint32_t)q;
+        k0 += 4u;
       }
-      // rasterise the lanes' triangles
       const bool fits =  // edge values fit 32 bits
           has &&
           max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
@@ -809,36 +801,99 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     bgk = (unsigned long long)(bf16_rne(bgc[0]) | (bf16_rne(bgc[1]) << 16)) |
           ((unsigned long long)(bf16_rne(bgc[2]) | (bf16_rne(bgc[3]) << 16)) << 32);
   float* fout = reinterpret_cast<float*>(O.color) + (size_t)t.s * C * plane + pix0;  // OM 2
-  uint16_t* pq = reinterpret_cast<uint16_t*>(vxy);  // covered pixels awaiting their shading
+  // covered pixels awaiting their shading: at most 63 + 256
+  uint16_t* pq = reinterpret_cast<uint16_t*>(vxy);
   const float inv_w = 1.0f / (float)W;
-  uint32_t pend = 0;
-  for (int p0 = wave * 64; p0 < npx || pend > 0u;) {
+  uint32_t pend = 0, head = 0;
+  const int step = F.vec ? 4 : 1;  // pixels per lane of a scan
+  for (int p0 = wave * 64 * step; p0 < npx || pend > 0u;) {
     if (p0 < npx && pend < 64u) {
-      const int p = p0 + lane;
-      bool covered = false;
-      if (p < npx) {
-        const unsigned long long key = pix[p];
-        const uint32_t zb = (uint32_t)(key >> 32);
-        covered = zb < kDepthOne;
-        if (dep) dep[p] = covered ? __uint_as_float(zb) : 1.0f;
-        if (vis) vis[p] = covered ? (int32_t)((uint32_t)key >> 3) : -1;
-        if (!covered) {
-          if constexpr (OM < 2) {
-            pix[p] = bgk;
-          } else {
-            for (int ch = 0; ch < C; ++ch) fout[(size_t)ch * plane + p] = bgc[ch];
+      const uint64_t below = (1ull << lane) - 1ull;
+      if (head) {  // the rest of the queue moves to its front
+        const uint16_t v = (uint32_t)lane < pend ? pq[head + lane] : (uint16_t)0;
+        wave_fence();
+        if ((uint32_t)lane < pend) pq[lane] = v;
+        head = 0;
+      }
+      if (F.vec) {
+        const int p = p0 + lane * 4;
+        uint32_t cov = 0;  // bit k: pixel p + k is covered
+        if (p < npx) {
+          const ulonglong2 ka = *reinterpret_cast<const ulonglong2*>(pix + p);
+          const ulonglong2 kb = *reinterpret_cast<const ulonglong2*>(pix + p + 2);
+          const unsigned long long key[4] = {ka.x, ka.y, kb.x, kb.y};
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            cov |= (uint32_t)(key[k] >> 32) < kDepthOne ? 1u << k : 0u;
+          if (dep) {
+            float z[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              z[k] = (cov >> k) & 1u ? __uint_as_float((uint32_t)(key[k] >> 32)) : 1.0f;
+            *reinterpret_cast<float4*>(dep + p) = make_float4(z[0], z[1], z[2], z[3]);
+          }
+          if (vis) {
+            int v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              v[k] = (cov >> k) & 1u ? (int)((uint32_t)key[k] >> 3) : -1;
+            *reinterpret_cast<int4*>(vis + p) = make_int4(v[0], v[1], v[2], v[3]);
+          }
+          if constexpr (OM == 1) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (!((cov >> k) & 1u)) pix[p + k] = bgk;
+          } else if constexpr (OM == 2) {
+            if (cov == 0u) {
+              for (int ch = 0; ch < C; ++ch)
+                *reinterpret_cast<float4*>(fout + (size_t)ch * plane + p) =
+                    make_float4(bgc[ch], bgc[ch], bgc[ch], bgc[ch]);
+            } else if (cov != 15u) {
+              for (int ch = 0; ch < C; ++ch)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                  if (!((cov >> k) & 1u)) fout[(size_t)ch * plane + p + k] = bgc[ch];
+            }
           }
         }
+        uint64_t m[4];
+        uint32_t at = pend;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          m[k] = __ballot((cov >> k) & 1u);
+          at += (uint32_t)__popcll(m[k] & below);
+          pend += (uint32_t)__popcll(m[k]);
+        }
+        if (cov) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if ((cov >> k) & 1u) pq[at++] = (uint16_t)(p + k);
+        }
+      } else {
+        const int p = p0 + lane;
+        bool covered = false;
+        if (p < npx) {
+          const unsigned long long key = pix[p];
+          const uint32_t zb = (uint32_t)(key >> 32);
+          covered = zb < kDepthOne;
+          if (dep) dep[p] = covered ? __uint_as_float(zb) : 1.0f;
+          if (vis) vis[p] = covered ? (int32_t)((uint32_t)key >> 3) : -1;
+          if (!covered) {
+            if constexpr (OM == 1) pix[p] = bgk;
+            if constexpr (OM == 2)
+              for (int ch = 0; ch < C; ++ch) fout[(size_t)ch * plane + p] = bgc[ch];
+          }
+        }
+        const uint64_t m = __ballot(covered);
+        if (covered) pq[pend + (uint32_t)__popcll(m & below)] = (uint16_t)p;
+        pend += (uint32_t)__popcll(m);
       }
-      const uint64_t m = __ballot(covered);
-      if (covered) pq[pend + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)p;
-      pend += (uint32_t)__popcll(m);
-      p0 += kBandBlock;
+      p0 += kBandBlock * step;
       wave_fence();
       continue;
     }
     const uint32_t take = min(pend, 64u);
-    const int p = (uint32_t)lane < take ? (int)pq[lane] : 0;
+    const int p = (uint32_t)lane < take ? (int)pq[head + lane] : 0;
     const uint32_t rank = (uint32_t)pix[p];
     int y = (int)((float)p * inv_w);
     int x = p - y * W;
@@ -855,7 +910,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       done = band_shade_smooth(D, F, lt, t.s, VP, nodes, nn, tab, lane, take, rank >> 3,
                                (int)(rank & 7u), x, t.j1 - y, qu, col);
     else
-      done = band_shade_flat(D, F, lt, t.s, nodes, nn, tab, lane, take, rank >> 3, col);
+      done = band_shade_flat(D, lt, t.s, nodes, nn, tab, lane, take, rank >> 3, col);
     if ((uint32_t)lane < done) {
       if constexpr (OM == 0) {
         pix[p] = pack_rgba8(col);
@@ -868,24 +923,48 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           if (ch < C) fout[(size_t)ch * plane + p] = col[ch];
       }
     }
-    const uint32_t ra = (uint32_t)lane + done, rb = ra + 64u;
-    uint16_t na = 0, nb = 0;
-    if (ra < pend) na = pq[ra];
-    if (rb < pend) nb = pq[rb];
-    wave_fence();
-    if (ra < pend) pq[lane] = na;
-    if (rb < pend) pq[lane + 64] = nb;
+    head += done;
     pend -= done;
     wave_fence();
   }
   if constexpr (OM == 2) return;
   __syncthreads();
-  // the band's colours as whole dwords of each channel plane: dword k of the
-  // plane's aligned range starts at pixel k * PER - mis
+  unsigned char* cout = reinterpret_cast<unsigned char*>(O.color) +
+                        ((size_t)t.s * C * plane + pix0) * (OM == 0 ? 1 : 2);
+  // colour of pixel p as its plane's bytes; an uncovered pixel of a uint8
+  // frame still holds its key
+  auto pixel = [&](unsigned long long v) {
+    if constexpr (OM == 0)
+      return (uint32_t)(v >> 32) == kDepthOne ? (uint32_t)bgk : (uint32_t)v;
+    else
+      return v;
+  };
+  if (F.vec) {
+    // four pixels of every channel from one read of their keys
+    for (int p = tid * 4; p < npx; p += kBandBlock * 4) {
+      const ulonglong2 ka = *reinterpret_cast<const ulonglong2*>(pix + p);
+      const ulonglong2 kb = *reinterpret_cast<const ulonglong2*>(pix + p + 2);
+      const auto v0 = pixel(ka.x), v1 = pixel(ka.y), v2 = pixel(kb.x), v3 = pixel(kb.y);
+      unsigned char* dst = cout + (size_t)p * (OM == 0 ? 1 : 2);
+#pragma unroll 1
+      for (int ch = 0; ch < C; ++ch) {
+        if constexpr (OM == 0) {
+          *reinterpret_cast<uint32_t*>(dst + (size_t)ch * plane) =
+              band_gather((uint32_t)v0, (uint32_t)v1, (uint32_t)v2, (uint32_t)v3, ch);
+        } else {
+          const int sh = 16 * ch;
+          *reinterpret_cast<uint2*>(dst + (size_t)ch * plane * 2) = make_uint2(
+              ((uint32_t)(v0 >> sh) & 0xffffu) | ((uint32_t)(v1 >> sh) << 16),
+              ((uint32_t)(v2 >> sh) & 0xffffu) | ((uint32_t)(v3 >> sh) << 16));
+        }
+      }
+    }
+    return;
+  }
+  // whole dwords of each channel plane: dword k of the plane's aligned range
+  // starts at pixel k * PER - mis
   constexpr int PER = OM == 0 ? 4 : 2;
   constexpr size_t ES = OM == 0 ? 1 : 2;
-  unsigned char* cout = reinterpret_cast<unsigned char*>(O.color) +
-                        ((size_t)t.s * C * plane + pix0) * ES;
   for (int ch = 0; ch < C; ++ch) {
     unsigned char* dst = cout + (size_t)ch * plane * ES;
     const int mis = (int)(((uintptr_t)dst & 3u) / ES);
@@ -894,8 +973,8 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       if (p >= 0 && p + PER <= npx) {
         uint32_t v;
         if constexpr (OM == 0) {
-          v = band_gather((uint32_t)pix[p], (uint32_t)pix[p + 1], (uint32_t)pix[p + 2],
-                          (uint32_t)pix[p + 3], ch);
+          v = band_gather(pixel(pix[p]), pixel(pix[p + 1]), pixel(pix[p + 2]), pixel(pix[p + 3]),
+                          ch);
         } else {
           v = ((uint32_t)(pix[p] >> (16 * ch)) & 0xffffu) |
               ((uint32_t)(pix[p + 1] >> (16 * ch)) << 16);
@@ -906,7 +985,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         for (int b = 0; b < PER; ++b) {
           if (p + b < 0 || p + b >= npx) continue;
           if constexpr (OM == 0)
-            dst[p + b] = (uint8_t)(pix[p + b] >> (8 * ch));
+            dst[p + b] = (uint8_t)(pixel(pix[p + b]) >> (8 * ch));
           else
             reinterpret_cast<uint16_t*>(dst)[p + b] = (uint16_t)(pix[p + b] >> (16 * ch));
         }
@@ -942,7 +1021,7 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
     verts = std::max(verts, me.num_vertices);
     ntab = std::max(ntab, me.index_offset + me.num_triangles);
   }
-  verts = std::max(verts, 120);
+  verts = (std::max(verts, 120) + 1) & ~1;  // tables and keys stay 16-byte aligned
   for (int j = 0; j < D->num_nodes; ++j) {
     const pbr_mesh& me = D->meshes[D->nodes[j].mesh];
     if (D->nodes[j].instances_per_scene == 0 || me.num_triangles == 0) continue;
@@ -953,9 +1032,10 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
     F.node[j].inv_nt = (uint32_t)((65536 + me.num_triangles - 1) / me.num_triangles);
   }
   F.verts = verts;
-  F.ntab = ntab <= kBandTable ? ntab : 0;
+  if (ntab > kBandTable) return false;
+  F.ntab = ntab;
   const size_t stat = sizeof(NodeLds) * PBR_MAX_NODES + 64;
-  const size_t rest = (size_t)kBandWaves * ((size_t)verts * 12 + 128) + 4 * (size_t)F.ntab;
+  const size_t rest = (size_t)kBandWaves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)F.ntab;
   const int fit = (int)((kBandLds - stat - rest) / 8);
   const int px = std::min(fit, kBandPixels);
   if (D->width > px) return false;
@@ -964,7 +1044,7 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   if (F.bands > kMaxBands) return false;
   F.th = (D->height + F.bands - 1) / F.bands;
   F.bands = (D->height + F.th - 1) / F.th;
-  P.lds = (size_t)8 * F.th * F.W + rest;
+  P.lds = (size_t)8 * ((F.th * F.W + 1) & ~1) + rest;
   return true;
 }
 
@@ -1002,6 +1082,12 @@ int launch_bands(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rend
   F.max_slots = max_slots;
   F.budget = budget;
   F.uniform = uniform ? 1 : 0;
+  // every channel plane, depth and id row of a band starts on a multiple of
+  // four pixels from an aligned base, and the band is whole groups of four
+  const uintptr_t align = O->dtype == PBR_DTYPE_U8 ? 3 : (O->dtype == PBR_DTYPE_BF16 ? 7 : 15);
+  F.vec = (D->width * D->height) % 4 == 0 && (F.th * D->width) % 4 == 0 &&
+          !((uintptr_t)O->color & align) && !((uintptr_t)O->depth & 15) &&
+          !((uintptr_t)O->vis & 15);
   const uint64_t items = (uint64_t)D->num_scenes * (uint64_t)F.bands;
   if (items >= 0x7fffffffull) return fail(PBR_ERR_INVALID, "too many bands");
   const Light lt = host_light(D);
