@@ -44,7 +44,7 @@ constexpr int kBandTable = 512;   // triangles of all meshes (LDS index table) a
 constexpr int kMaxBands = 4;      // bands per scene at most: each repeats the vertex work
 constexpr int kBandPixels = 8192;
 constexpr int kBandLds = 80 * 1024;  // half a CU's LDS: two workgroups share a CU
-constexpr int kSmallPixels = 48;  // box pixels one lane rasterises alone
+constexpr int kSmallPixels = 12;  // box pixels one lane rasterises alone
 constexpr uint32_t kDepthOne = 0x3f800000u;
 
 // Per-node launch constants.
@@ -124,6 +124,18 @@ __device__ __forceinline__ uint32_t pool_triangle(const pbr_scene_desc& D, int q
   return (uint32_t)t[0] | ((uint32_t)t[1] << 8) | ((uint32_t)t[2] << 16);
 }
 
+// A value of lane `src`.
+__device__ __forceinline__ int from_lane(int src, int v) {
+  return __builtin_amdgcn_ds_bpermute(src << 2, v);
+}
+__device__ __forceinline__ float from_lane(int src, float v) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(v)));
+}
+// Sends v to lane `dst`; the lane's result is 0 if no lane sends to it.
+__device__ __forceinline__ float to_lane(int dst, float v) {
+  return __int_as_float(__builtin_amdgcn_ds_permute(dst << 2, __float_as_int(v)));
+}
+
 struct BandCtx {
   int s, W;
   int j0, j1;  // GL rows of the band; LDS row 0 is j1
@@ -196,6 +208,50 @@ __device__ __forceinline__ void band_raster_lane(unsigned long long* pix, const 
   }
 }
 
+// The rows of the lanes' triangles (`has`, extents within kIntExtent) dealt to
+// the lanes of the wave, 64 rows at a time: a lane finds its triangle by a
+// binary search of the running row counts and walks the row.  Triangles of
+// more than a few pixels keep the whole wave busy this way, where a lane per
+// triangle would walk as long as the largest box.
+__device__ __forceinline__ void band_raster_rows(unsigned long long* pix, const BandCtx& t,
+                                                 int lane, bool has, const FixTri& T,
+                                                 uint32_t rank) {
+  const int incl = wave_scan_add(has ? T.j1 - T.j0 + 1 : 0);
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  // columns (W <= 8192) and fill-rule bias in one word
+  const int box = T.i0 | (T.i1 << 13) | (int)(T.bias << 26);
+  for (int r0 = 0; r0 < total; r0 += 64) {
+    const int r = min(r0 + lane, total - 1);
+    int l = 0;  // the first lane whose running count exceeds r
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) l = from_lane(l + d - 1, incl) <= r ? l + d : l;
+    FixTri U;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      U.X[k] = from_lane(l, T.X[k]);
+      U.Y[k] = from_lane(l, T.Y[k]);
+    }
+    const float zx = from_lane(l, T.zx), zy = from_lane(l, T.zy), zc = from_lane(l, T.zc);
+    const int b = from_lane(l, box);
+    const int j = from_lane(l, T.j1) - (from_lane(l, incl) - 1 - r);
+    const uint32_t ur = (uint32_t)from_lane(l, (int)rank);
+    U.bias = (uint32_t)b >> 26;
+    const int i0 = b & 0x1fff, w = ((b >> 13) & 0x1fff) - i0;
+    BandEdges<int32_t> E;
+    band_edges(U, i0, j, E);
+    const float tz = fmaf(zy, (float)j + 0.5f, zc);
+    float x = (float)i0 + 0.5f;
+    unsigned long long* q = pix + (t.j1 - j) * t.W + i0;
+    if (r0 + lane < total)
+      for (int i = 0; i <= w; ++i) {
+        if (band_inside(E.e)) band_fragment(q + i, clamp_depth(fmaf(zx, x, tz)), ur);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) E.e[k] += E.A[k];
+        x += 1.0f;
+      }
+  }
+}
+
 // The whole wave, in blocks of 8 x 8 pixels.  Every argument is uniform.
 template <typename Num>
 __device__ __forceinline__ void band_raster_wave(unsigned long long* pix, const BandCtx& t,
@@ -235,18 +291,6 @@ __device__ __forceinline__ uint32_t outcode(const CVert& v, float guard) {
 #pragma unroll
   for (int p = 0; p < 6; ++p) oc |= plane_dist(v, p, guard) >= 0.0f ? 0u : 1u << p;
   return oc;
-}
-
-// A value of lane `src`.
-__device__ __forceinline__ int from_lane(int src, int v) {
-  return __builtin_amdgcn_ds_bpermute(src << 2, v);
-}
-__device__ __forceinline__ float from_lane(int src, float v) {
-  return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(v)));
-}
-// Sends v to lane `dst`; the lane's result is 0 if no lane sends to it.
-__device__ __forceinline__ float to_lane(int dst, float v) {
-  return __int_as_float(__builtin_amdgcn_ds_permute(dst << 2, __float_as_int(v)));
 }
 
 // Sutherland-Hodgman on four polygons at once, one per group of 16 lanes: lane
@@ -350,89 +394,113 @@ __device__ __forceinline__ SlotRef band_slot(int s, const NodeLds* nodes, int nn
 }
 
 // Colours of the pixels in lanes 0 .. take - 1 (GL pixel (x, j), winner `slot`
-// and sub-triangle q); returns how many leading lanes were shaded.
+// and sub-triangle q).
 
 // Flat scenes: every lane shades its own winner's first normal.
-__device__ __forceinline__ uint32_t band_shade_flat(const pbr_scene_desc& D, const Light& lt,
-                                                    int s, const NodeLds* nodes, int nn,
-                                                    const uint32_t* tab, int lane, uint32_t take,
-                                                    uint32_t slot, float col[4]) {
-  if ((uint32_t)lane < take) {
-    const SlotRef R = band_slot(s, nodes, nn, tab, slot);
-    float M[16], v[6], nw[3], n[3];
-    load_mat4_global(R.trans + R.row * 16, M);
-    const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
-    const float rgba[4] = {c4.x, c4.y, c4.z, c4.w};
-    load_vertex(D.vertices, R.voff + (int)(R.tri & 0xffu), v);
+__device__ __forceinline__ void band_shade_flat(const pbr_scene_desc& D, const Light& lt, int s,
+                                                const NodeLds* nodes, int nn, const uint32_t* tab,
+                                                int lane, uint32_t take, uint32_t slot,
+                                                float col[4]) {
+  if ((uint32_t)lane >= take) return;
+  const SlotRef R = band_slot(s, nodes, nn, tab, slot);
+  float M[16], v[6], nw[3], n[3];
+  load_mat4_global(R.trans + R.row * 16, M);
+  const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
+  const float rgba[4] = {c4.x, c4.y, c4.z, c4.w};
+  load_vertex(D.vertices, R.voff + (int)(R.tri & 0xffu), v);
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const float a = M[r * 4 + 0] * v[3] + M[r * 4 + 1] * v[4];
-      nw[r] = a + M[r * 4 + 2] * v[5];
-    }
-    normalize3(nw, n);
-    shade(n, rgba, lt, col);
+  for (int r = 0; r < 3; ++r) {
+    const float a = M[r * 4 + 0] * v[3] + M[r * 4 + 1] * v[4];
+    nw[r] = a + M[r * 4 + 2] * v[5];
   }
-  return take;
+  normalize3(nw, n);
+  shade(n, rgba, lt, col);
 }
 
-// Runs of pixels with one winner share its vertices: lane 3 u + k transforms
-// vertex k of the u-th run's triangle, and every pixel of the run reads the
-// three back.  At most 21 runs fit a wave, so a pass may shade fewer pixels
-// than it was given.  `heads` is 64 bytes of the wave's LDS.
+// Smooth scenes.  Runs of pixels with one winner share its vertices when the
+// pixels form at most kShadeRuns runs: lane 3 u + k transforms vertex k of
+// the u-th run's triangle, and every pixel of the run reads the three back.
+// With more runs (triangles of a pixel or two) every lane transforms its own
+// winner's three vertices.  `heads` is 64 bytes of the wave's LDS.
 constexpr int kShadeRuns = 21;
-__device__ __forceinline__ uint32_t band_shade_smooth(const pbr_scene_desc& D, const BandFrame& F,
-                                                      const Light& lt, int s, const float VP[16],
-                                                      const NodeLds* nodes, int nn,
-                                                      const uint32_t* tab, int lane, uint32_t take,
-                                                      uint32_t slot, int q, int x, int j,
-                                                      uint8_t* heads, float col[4]) {
-  const bool valid = (uint32_t)lane < take;
+__device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const BandFrame& F,
+                                                  const Light& lt, int s, const float VP[16],
+                                                  const NodeLds* nodes, int nn,
+                                                  const uint32_t* tab, int lane, uint32_t take,
+                                                  uint32_t slot, int q, int x, int j,
+                                                  uint8_t* heads, float col[4]) {
+  const bool mine = (uint32_t)lane < take;
   const int prev = from_lane(lane > 0 ? lane - 1 : 0, (int)slot);
-  const bool head = valid && (lane == 0 || (uint32_t)prev != slot);
+  const bool head = mine && (lane == 0 || (uint32_t)prev != slot);
   const uint64_t hm = __ballot(head);
-  const int run = __popcll(hm & ((2ull << lane) - 1ull)) - 1;
-  const int runs = min(__popcll(hm), kShadeRuns);
-  if (head) heads[run] = (uint8_t)lane;
-  wave_fence();
-  const int u = (lane * 86) >> 8, k = lane - 3 * u;
-  CVert cv = {};
-  SnapVert sv = {};
-  uint32_t fl = 0;
-  float rgba[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  // every lane takes part in the reads of other lanes' slots
-  const uint32_t vslot = (uint32_t)from_lane(u < runs ? (int)heads[u] : 0, (int)slot);
-  if (u < runs) {
-    const SlotRef R = band_slot(s, nodes, nn, tab, vslot);
+  const int runs = __popcll(hm);
+  int32_t X[3] = {0, 0, 0}, Y[3] = {0, 0, 0};
+  float iw[3] = {0.0f, 0.0f, 0.0f}, n[3][3] = {}, base[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  uint32_t code = 0;  // outcodes; bit 6: flat
+  if (runs <= kShadeRuns) {
+    const int run = __popcll(hm & ((2ull << lane) - 1ull)) - 1;
+    if (head) heads[run] = (uint8_t)lane;
+    wave_fence();
+    const int u = (lane * 86) >> 8, k = lane - 3 * u;
+    CVert cv = {};
+    SnapVert sv = {};
+    uint32_t fl = 0;
+    float rgba[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // every lane takes part in the reads of other lanes' slots
+    const uint32_t vslot = (uint32_t)from_lane(u < runs ? (int)heads[u] : 0, (int)slot);
+    if (u < runs) {
+      const SlotRef R = band_slot(s, nodes, nn, tab, vslot);
+      const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
+      rgba[0] = c4.x;
+      rgba[1] = c4.y;
+      rgba[2] = c4.z;
+      rgba[3] = c4.w;
+      const uint32_t id = k == 0 ? R.tri & 0xffu : (k == 1 ? (R.tri >> 8) & 0xffu : R.tri >> 16);
+      float M[16], vv[6];
+      load_mat4_global(R.trans + R.row * 16, M);
+      load_vertex(D.vertices, R.voff + (int)id, vv);
+      transform_vertex(M, VP, vv, cv);
+      snap_vertex(cv, F.W, F.H, sv);
+      fl = outcode(cv, F.guard) | ((R.flags & 2u) << 5);
+    }
+    const int src = mine ? 3 * run : 0;
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      X[v] = from_lane(src + v, sv.X);
+      Y[v] = from_lane(src + v, sv.Y);
+      iw[v] = from_lane(src + v, sv.invw);
+      code |= (uint32_t)from_lane(src + v, (int)fl);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) n[v][c] = from_lane(src + v, cv.n[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) base[c] = from_lane(src, rgba[c]);
+  } else if (mine) {
+    const SlotRef R = band_slot(s, nodes, nn, tab, slot);
     const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
-    rgba[0] = c4.x;
-    rgba[1] = c4.y;
-    rgba[2] = c4.z;
-    rgba[3] = c4.w;
-    const uint32_t id = k == 0 ? R.tri & 0xffu : (k == 1 ? (R.tri >> 8) & 0xffu : R.tri >> 16);
-    float M[16], vv[6];
+    base[0] = c4.x;
+    base[1] = c4.y;
+    base[2] = c4.z;
+    base[3] = c4.w;
+    float M[16];
     load_mat4_global(R.trans + R.row * 16, M);
-    load_vertex(D.vertices, R.voff + (int)id, vv);
-    transform_vertex(M, VP, vv, cv);
-    snap_vertex(cv, F.W, F.H, sv);
-    fl = outcode(cv, F.guard) | ((R.flags & 2u) << 5);  // bit 6: flat
+    code = (R.flags & 2u) << 5;
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      float vv[6];
+      load_vertex(D.vertices, R.voff + (int)((R.tri >> (8 * v)) & 0xffu), vv);
+      CVert cv;
+      SnapVert sv;
+      transform_vertex(M, VP, vv, cv);
+      snap_vertex(cv, F.W, F.H, sv);
+      code |= outcode(cv, F.guard);
+      X[v] = sv.X;
+      Y[v] = sv.Y;
+      iw[v] = sv.invw;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) n[v][c] = cv.n[c];
+    }
   }
-  const bool mine = valid && run < kShadeRuns;
-  const int src = mine ? 3 * run : 0;
-  int32_t X[3], Y[3];
-  float iw[3], n[3][3];
-  uint32_t code = 0;
-#pragma unroll
-  for (int v = 0; v < 3; ++v) {
-    X[v] = from_lane(src + v, sv.X);
-    Y[v] = from_lane(src + v, sv.Y);
-    iw[v] = from_lane(src + v, sv.invw);
-    code |= (uint32_t)from_lane(src + v, (int)fl);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) n[v][c] = from_lane(src + v, cv.n[c]);
-  }
-  float base[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) base[c] = from_lane(src, rgba[c]);
   const bool flat = (code & 64u) != 0u;
 
   // winners that straddle a clip plane: their polygons, four slots at a time
@@ -504,7 +572,6 @@ __device__ __forceinline__ uint32_t band_shade_smooth(const pbr_scene_desc& D, c
     }
     shade(nn3, base, lt, col);
   }
-  return (uint32_t)__popcll(__ballot(mine));
 }
 
 // Byte c of each of four packed RGBA8 colours -> one dword.
@@ -525,7 +592,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
                                                           uint32_t* hdr, Light lt, float4 bg) {
   extern __shared__ __align__(16) unsigned long long pix[];
   __shared__ NodeLds nodes[PBR_MAX_NODES];
-  __shared__ uint32_t next_chunk, total_chunks;
+  __shared__ uint32_t next_chunk, total_chunks, covered_n;
   const int tid = (int)threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = F.W, H = F.H, nn = D.num_nodes;
@@ -593,6 +660,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     }
     if (lane == 63) {
       next_chunk = 0u;
+      covered_n = 0u;
       total_chunks = ic;
     }
   }
@@ -758,10 +826,12 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           has &&
           max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
           max(T.Y[0], max(T.Y[1], T.Y[2])) - min(T.Y[0], min(T.Y[1], T.Y[2])) <= kIntExtent;
-      const bool small = fits && (T.i1 - T.i0 + 1) * (T.j1 - T.j0 + 1) <= kSmallPixels;
+      const int w = T.i1 - T.i0 + 1, h = T.j1 - T.j0 + 1;
+      const bool small = fits && w * h <= kSmallPixels;
       if (small) band_raster_lane(pix, t, T, rank);
-      const uint64_t fm = __ballot(fits);
-      for (uint64_t m = __ballot(has && !small); m; m &= m - 1ull) {
+      const bool rows = fits && !small;
+      if (__ballot(rows)) band_raster_rows(pix, t, lane, rows, T, rank);
+      for (uint64_t m = __ballot(has && !fits); m; m &= m - 1ull) {
         const int l = __ffsll((unsigned long long)m) - 1;
         FixTri U;
 #pragma unroll
@@ -777,11 +847,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         U.j0 = rl(T.j0, l);
         U.j1 = rl(T.j1, l);
         U.bias = (uint32_t)rl((int)T.bias, l);
-        const uint32_t ur = (uint32_t)rl((int)rank, l);
-        if ((fm >> l) & 1ull)
-          band_raster_wave<int32_t>(pix, t, lane, U, ur);
-        else
-          band_raster_wave<double>(pix, t, lane, U, ur);
+        band_raster_wave<double>(pix, t, lane, U, (uint32_t)rl((int)rank, l));
       }
     }
     wave_fence();  // the next chunk rewrites the table
@@ -801,117 +867,106 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     bgk = (unsigned long long)(bf16_rne(bgc[0]) | (bf16_rne(bgc[1]) << 16)) |
           ((unsigned long long)(bf16_rne(bgc[2]) | (bf16_rne(bgc[3]) << 16)) << 32);
   float* fout = reinterpret_cast<float*>(O.color) + (size_t)t.s * C * plane + pix0;  // OM 2
-  // covered pixels awaiting their shading: at most 63 + 256
-  uint16_t* pq = reinterpret_cast<uint16_t*>(vxy);
   const float inv_w = 1.0f / (float)W;
-  uint32_t pend = 0, head = 0;
   const int step = F.vec ? 4 : 1;  // pixels per lane of a scan
-  for (int p0 = wave * 64 * step; p0 < npx || pend > 0u;) {
-    if (p0 < npx && pend < 64u) {
-      const uint64_t below = (1ull << lane) - 1ull;
-      if (head) {  // the rest of the queue moves to its front
-        const uint16_t v = (uint32_t)lane < pend ? pq[head + lane] : (uint16_t)0;
-        wave_fence();
-        if ((uint32_t)lane < pend) pq[lane] = v;
-        head = 0;
+  const uint64_t below = (1ull << lane) - 1ull;
+  // Scan of the 64 x step pixels from p0 (those below `end`): depths, ids and
+  // backgrounds leave; bit k of the result: the lane's pixel k is covered
+  // (pixels p0 + lane * step + k).
+  auto scan = [&](int p0, int end) -> uint32_t {
+    uint32_t cov = 0;
+    const int p = p0 + lane * step;
+    if (p >= end) return 0u;
+    if (F.vec) {
+      const ulonglong2 ka = *reinterpret_cast<const ulonglong2*>(pix + p);
+      const ulonglong2 kb = *reinterpret_cast<const ulonglong2*>(pix + p + 2);
+      const unsigned long long key[4] = {ka.x, ka.y, kb.x, kb.y};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) cov |= (uint32_t)(key[k] >> 32) < kDepthOne ? 1u << k : 0u;
+      if (dep) {
+        float z[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          z[k] = (cov >> k) & 1u ? __uint_as_float((uint32_t)(key[k] >> 32)) : 1.0f;
+        *reinterpret_cast<float4*>(dep + p) = make_float4(z[0], z[1], z[2], z[3]);
       }
-      if (F.vec) {
-        const int p = p0 + lane * 4;
-        uint32_t cov = 0;  // bit k: pixel p + k is covered
-        if (p < npx) {
-          const ulonglong2 ka = *reinterpret_cast<const ulonglong2*>(pix + p);
-          const ulonglong2 kb = *reinterpret_cast<const ulonglong2*>(pix + p + 2);
-          const unsigned long long key[4] = {ka.x, ka.y, kb.x, kb.y};
+      if (vis) {
+        int v[4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            cov |= (uint32_t)(key[k] >> 32) < kDepthOne ? 1u << k : 0u;
-          if (dep) {
-            float z[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              z[k] = (cov >> k) & 1u ? __uint_as_float((uint32_t)(key[k] >> 32)) : 1.0f;
-            *reinterpret_cast<float4*>(dep + p) = make_float4(z[0], z[1], z[2], z[3]);
-          }
-          if (vis) {
-            int v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              v[k] = (cov >> k) & 1u ? (int)((uint32_t)key[k] >> 3) : -1;
-            *reinterpret_cast<int4*>(vis + p) = make_int4(v[0], v[1], v[2], v[3]);
-          }
-          if constexpr (OM == 1) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              if (!((cov >> k) & 1u)) pix[p + k] = bgk;
-          } else if constexpr (OM == 2) {
-            if (cov == 0u) {
-              for (int ch = 0; ch < C; ++ch)
-                *reinterpret_cast<float4*>(fout + (size_t)ch * plane + p) =
-                    make_float4(bgc[ch], bgc[ch], bgc[ch], bgc[ch]);
-            } else if (cov != 15u) {
-              for (int ch = 0; ch < C; ++ch)
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                  if (!((cov >> k) & 1u)) fout[(size_t)ch * plane + p + k] = bgc[ch];
-            }
-          }
-        }
-        uint64_t m[4];
-        uint32_t at = pend;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          m[k] = __ballot((cov >> k) & 1u);
-          at += (uint32_t)__popcll(m[k] & below);
-          pend += (uint32_t)__popcll(m[k]);
-        }
-        if (cov) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if ((cov >> k) & 1u) pq[at++] = (uint16_t)(p + k);
-        }
-      } else {
-        const int p = p0 + lane;
-        bool covered = false;
-        if (p < npx) {
-          const unsigned long long key = pix[p];
-          const uint32_t zb = (uint32_t)(key >> 32);
-          covered = zb < kDepthOne;
-          if (dep) dep[p] = covered ? __uint_as_float(zb) : 1.0f;
-          if (vis) vis[p] = covered ? (int32_t)((uint32_t)key >> 3) : -1;
-          if (!covered) {
-            if constexpr (OM == 1) pix[p] = bgk;
-            if constexpr (OM == 2)
-              for (int ch = 0; ch < C; ++ch) fout[(size_t)ch * plane + p] = bgc[ch];
-          }
-        }
-        const uint64_t m = __ballot(covered);
-        if (covered) pq[pend + (uint32_t)__popcll(m & below)] = (uint16_t)p;
-        pend += (uint32_t)__popcll(m);
+        for (int k = 0; k < 4; ++k) v[k] = (cov >> k) & 1u ? (int)((uint32_t)key[k] >> 3) : -1;
+        *reinterpret_cast<int4*>(vis + p) = make_int4(v[0], v[1], v[2], v[3]);
       }
-      p0 += kBandBlock * step;
-      wave_fence();
-      continue;
+      if constexpr (OM == 1) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (!((cov >> k) & 1u)) pix[p + k] = bgk;
+      } else if constexpr (OM == 2) {
+        if (cov == 0u) {
+          for (int ch = 0; ch < C; ++ch)
+            *reinterpret_cast<float4*>(fout + (size_t)ch * plane + p) =
+                make_float4(bgc[ch], bgc[ch], bgc[ch], bgc[ch]);
+        } else if (cov != 15u) {
+          for (int ch = 0; ch < C; ++ch)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (!((cov >> k) & 1u)) fout[(size_t)ch * plane + p + k] = bgc[ch];
+        }
+      }
+    } else {
+      const unsigned long long key = pix[p];
+      const uint32_t zb = (uint32_t)(key >> 32);
+      cov = zb < kDepthOne ? 1u : 0u;
+      if (dep) dep[p] = cov ? __uint_as_float(zb) : 1.0f;
+      if (vis) vis[p] = cov ? (int32_t)((uint32_t)key >> 3) : -1;
+      if (!cov) {
+        if constexpr (OM == 1) pix[p] = bgk;
+        if constexpr (OM == 2)
+          for (int ch = 0; ch < C; ++ch) fout[(size_t)ch * plane + p] = bgc[ch];
+      }
     }
-    const uint32_t take = min(pend, 64u);
-    const int p = (uint32_t)lane < take ? (int)pq[head + lane] : 0;
+    return cov;
+  };
+  // Position of the lane's first covered pixel among the scan's, their number
+  // in `sum`.
+  auto place = [&](uint32_t cov, uint32_t& sum) -> uint32_t {
+    uint32_t at = 0;
+    sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (k >= step) break;
+      const uint64_t m = __ballot((cov >> k) & 1u);
+      at += (uint32_t)__popcll(m & below);
+      sum += (uint32_t)__popcll(m);
+    }
+    return at;
+  };
+  auto push = [&](uint16_t* q, uint32_t cov, int p0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if ((cov >> k) & 1u) *q++ = (uint16_t)(p0 + lane * step + k);
+  };
+  // Shades the pixels q[0 .. take) (take <= 64).
+  uint8_t* heads = reinterpret_cast<uint8_t*>(tab) - 64 * kBandWaves + 64 * wave;
+  auto shade_batch = [&](const uint16_t* q, uint32_t take) {
+    const int p = q[min((uint32_t)lane, take - 1u)];
     const uint32_t rank = (uint32_t)pix[p];
-    int y = (int)((float)p * inv_w);
-    int x = p - y * W;
-    if (x < 0) {
-      --y;
-      x += W;
-    } else if (x >= W) {
-      ++y;
-      x -= W;
-    }
     float col[4];
-    uint32_t done;
-    if constexpr (SMOOTH)
-      done = band_shade_smooth(D, F, lt, t.s, VP, nodes, nn, tab, lane, take, rank >> 3,
-                               (int)(rank & 7u), x, t.j1 - y, qu, col);
-    else
-      done = band_shade_flat(D, lt, t.s, nodes, nn, tab, lane, take, rank >> 3, col);
-    if ((uint32_t)lane < done) {
+    if constexpr (SMOOTH) {
+      int y = (int)((float)p * inv_w);
+      int x = p - y * W;
+      if (x < 0) {
+        --y;
+        x += W;
+      } else if (x >= W) {
+        ++y;
+        x -= W;
+      }
+      band_shade_smooth(D, F, lt, t.s, VP, nodes, nn, tab, lane, take, rank >> 3,
+                        (int)(rank & 7u), x, t.j1 - y, heads, col);
+    } else {
+      band_shade_flat(D, lt, t.s, nodes, nn, tab, lane, take, rank >> 3, col);
+    }
+    if ((uint32_t)lane < take) {
       if constexpr (OM == 0) {
         pix[p] = pack_rgba8(col);
       } else if constexpr (OM == 1) {
@@ -923,12 +978,65 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           if (ch < C) fout[(size_t)ch * plane + p] = col[ch];
       }
     }
-    head += done;
-    pend -= done;
     wave_fence();
+  };
+  if constexpr (SMOOTH) {
+    // one queue for the workgroup (in the space of the vertex tables and
+    // triangle queues), so that only one batch per block of pixels is not
+    // full; a block is what the queue holds
+    uint16_t* pq = reinterpret_cast<uint16_t*>(tables);
+    const int hold = (kBandWaves * (12 * F.verts + kBandTris - 64) / 2) & ~255;
+    for (int b0 = 0; b0 < npx; b0 += hold) {
+      const int bend = min(npx, b0 + hold);
+      for (int p0 = b0 + wave * 64 * step; p0 < bend; p0 += kBandBlock * step) {
+        uint32_t sum;
+        const uint32_t cov = scan(p0, bend), at = place(cov, sum);
+        if (sum) {
+          uint32_t first = 0;
+          if (lane == 0) first = atomicAdd(&covered_n, sum);
+          first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+          push(pq + first + at, cov, p0);
+        }
+      }
+      __syncthreads();
+      const uint32_t total = (uint32_t)__builtin_amdgcn_readfirstlane((int)covered_n);
+      for (uint32_t k0 = (uint32_t)wave * 64u; k0 < total; k0 += (uint32_t)kBandBlock)
+        shade_batch(pq + k0, min(total - k0, 64u));
+      __syncthreads();
+      if (bend < npx) {  // the next block starts with an empty queue
+        if (tid == 0) covered_n = 0u;
+        __syncthreads();
+      }
+    }
+  } else {
+    // a queue per wave: flat shading is cheap enough that partial batches
+    // cost less than two more barriers
+    uint16_t* pq = reinterpret_cast<uint16_t*>(vxy);
+    uint32_t pend = 0;
+    for (int p0 = wave * 64 * step; p0 < npx || pend > 0u;) {
+      while (p0 < npx && pend < 64u) {  // at most 63 + 256 pixels are queued
+        uint32_t sum;
+        const uint32_t cov = scan(p0, npx), at = place(cov, sum);
+        push(pq + pend + at, cov, p0);
+        pend += sum;
+        p0 += kBandBlock * step;
+      }
+      wave_fence();
+      uint32_t done = 0;
+      while (done + 64u <= pend || (p0 >= npx && done < pend)) {
+        const uint32_t take = min(pend - done, 64u);
+        shade_batch(pq + done, take);
+        done += take;
+      }
+      const uint16_t v = done + (uint32_t)lane < pend ? pq[done + lane] : (uint16_t)0;
+      wave_fence();
+      if (done + (uint32_t)lane < pend) pq[lane] = v;
+      pend -= done;
+      wave_fence();
+    }
+    __syncthreads();
   }
   if constexpr (OM == 2) return;
-  __syncthreads();
   unsigned char* cout = reinterpret_cast<unsigned char*>(O.color) +
                         ((size_t)t.s * C * plane + pix0) * (OM == 0 ? 1 : 2);
   // colour of pixel p as its plane's bytes; an uncovered pixel of a uint8
@@ -1035,9 +1143,8 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   if (ntab > kBandTable) return false;
   F.ntab = ntab;
   const size_t stat = sizeof(NodeLds) * PBR_MAX_NODES + 64;
-  const size_t rest = (size_t)kBandWaves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)F.ntab;
-  const int fit = (int)((kBandLds - stat - rest) / 8);
-  const int px = std::min(fit, kBandPixels);
+  const size_t rest = (size_t)kBandWaves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)ntab;
+  const int px = std::min((int)((kBandLds - stat - rest) / 8), kBandPixels);
   if (D->width > px) return false;
   const int most = px / D->width;
   F.bands = (D->height + most - 1) / most;
