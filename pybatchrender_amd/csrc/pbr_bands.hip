@@ -589,7 +589,7 @@ template <bool SMOOTH, int OM>
 __global__ __launch_bounds__(kBandBlock)
 __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_frame_out O,
                                                           BandFrame F, const uint32_t* scene_off,
-                                                          uint32_t* hdr, Light lt, float4 bg) {
+                                                          const uint32_t* order, uint32_t* hdr, Light lt, float4 bg) {
   extern __shared__ __align__(16) unsigned long long pix[];
   __shared__ NodeLds nodes[PBR_MAX_NODES];
   __shared__ uint32_t next_chunk, total_chunks, covered_n;
@@ -597,8 +597,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = F.W, H = F.H, nn = D.num_nodes;
   BandCtx t;
-  t.s = (int)(blockIdx.x / (uint32_t)F.bands);
-  const int band = (int)(blockIdx.x - (uint32_t)t.s * (uint32_t)F.bands);
+  const uint32_t at = blockIdx.x / (uint32_t)F.bands;
+  const int band = (int)(blockIdx.x - at * (uint32_t)F.bands);
+  t.s = (int)(order ? order[at] : at);
   const int yo0 = band * F.th, rows = min(F.th, H - yo0);
   t.W = W;
   t.j1 = H - 1 - yo0;
@@ -1157,7 +1158,7 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
 
 template <bool SMOOTH, int OM>
 hipError_t launch_bands_t(const pbr_scene_desc* D, const pbr_frame_out* O, const BandPlan& P,
-                          const uint32_t* scene_off, uint32_t* hdr, const Light& lt, float4 bg,
+                          const uint32_t* scene_off, const uint32_t* order, uint32_t* hdr, const Light& lt, float4 bg,
                           uint32_t grid, hipStream_t st) {
   auto k = bands_kernel<SMOOTH, OM>;
   if (P.lds > 64 * 1024) {
@@ -1165,7 +1166,7 @@ hipError_t launch_bands_t(const pbr_scene_desc* D, const pbr_frame_out* O, const
         (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k, dim3(grid), dim3(kBandBlock), P.lds, st, *D, *O, P.F, scene_off, hdr, lt,
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kBandBlock), P.lds, st, *D, *O, P.F, scene_off, order, hdr, lt,
                      bg);
   return hipGetLastError();
 }
@@ -1181,7 +1182,7 @@ bool bands_supported(const pbr_scene_desc* D, const pbr_render_opts* opts) {
 
 int launch_bands(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_render_opts* opts,
                  uint32_t max_slots, uint32_t budget, bool uniform, const uint32_t* scene_off,
-                 uint32_t* hdr, hipStream_t st) {
+                 const uint32_t* order, uint32_t* hdr, hipStream_t st) {
   BandPlan P;
   if (!bands_plan(D, opts, P)) return fail(PBR_ERR_UNSUPPORTED, "band path cannot draw this batch");
   BandFrame& F = P.F;
@@ -1205,16 +1206,16 @@ int launch_bands(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rend
   const bool smooth = any_smooth(D);
   switch (O->dtype) {
     case PBR_DTYPE_U8:
-      e = smooth ? launch_bands_t<true, 0>(D, O, P, scene_off, hdr, lt, bg, grid, st)
-                 : launch_bands_t<false, 0>(D, O, P, scene_off, hdr, lt, bg, grid, st);
+      e = smooth ? launch_bands_t<true, 0>(D, O, P, scene_off, order, hdr, lt, bg, grid, st)
+                 : launch_bands_t<false, 0>(D, O, P, scene_off, order, hdr, lt, bg, grid, st);
       break;
     case PBR_DTYPE_BF16:
-      e = smooth ? launch_bands_t<true, 1>(D, O, P, scene_off, hdr, lt, bg, grid, st)
-                 : launch_bands_t<false, 1>(D, O, P, scene_off, hdr, lt, bg, grid, st);
+      e = smooth ? launch_bands_t<true, 1>(D, O, P, scene_off, order, hdr, lt, bg, grid, st)
+                 : launch_bands_t<false, 1>(D, O, P, scene_off, order, hdr, lt, bg, grid, st);
       break;
     default:
-      e = smooth ? launch_bands_t<true, 2>(D, O, P, scene_off, hdr, lt, bg, grid, st)
-                 : launch_bands_t<false, 2>(D, O, P, scene_off, hdr, lt, bg, grid, st);
+      e = smooth ? launch_bands_t<true, 2>(D, O, P, scene_off, order, hdr, lt, bg, grid, st)
+                 : launch_bands_t<false, 2>(D, O, P, scene_off, order, hdr, lt, bg, grid, st);
   }
   if (e != hipSuccess) return fail(PBR_ERR_LAUNCH, "band launch failed: %s", hipGetErrorString(e));
   return PBR_OK;

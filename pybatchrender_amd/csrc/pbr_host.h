@@ -42,12 +42,13 @@ int launch_tiles(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rend
 
 // The band path (pbr_bands.hip): whether it draws the batch with these
 // options, and its launch.  `scene_off` holds each scene's first slot of the
-// batch when instance counts differ per scene (not `uniform`); slots past
-// `budget` are not drawn.  hdr[0] of the workspace is the overflow flag.
+// batch when instance counts differ per scene (not `uniform`), `order` the
+// scenes in the order their workgroups start; slots past `budget` are not
+// drawn.  hdr[0] of the workspace is the overflow flag.
 bool bands_supported(const pbr_scene_desc* D, const pbr_render_opts* opts);
 int launch_bands(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_render_opts* opts,
                  uint32_t max_slots, uint32_t budget, bool uniform, const uint32_t* scene_off,
-                 uint32_t* hdr, hipStream_t st);
+                 const uint32_t* order, uint32_t* hdr, hipStream_t st);
 
 // The row-span kernel (pbr_rows.hip): whether it serves the descriptor, and
 // its launch (no workspace).  With `npose` > 0 the launch first applies
