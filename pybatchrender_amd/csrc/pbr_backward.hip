@@ -19,20 +19,26 @@
 // per-instance colours, the light (direction, colour, ambient, strength) and
 // the model-space vertex positions and normals of the meshes.
 //
-// Kernel layout: one workgroup per scene.
+// Kernel layout: one workgroup per (scene, band of rows).
 //   phase 0  (more slots than fit in LDS) mark the slots the visibility
 //            buffer names in an LDS bitmap and number them by a block scan;
-//   phase 1  per visible slot: fetch and transform the triangle, keep the
-//            per-pixel factors of smooth ones (h_a x h_b, normals, colour);
-//   phase 2  each lane walks runs of 16 pixels of a row: flat slots sum the
-//            output gradient, smooth slots accumulate the 32 per-pixel
-//            gradient terms; a run flushes into the slot's LDS accumulator
-//            when the slot changes;
-//   phase 3  per visible slot: chain the accumulated terms to instance
-//            colours (global atomics; LDS for rows shared by all scenes),
-//            light and vertex gradients (LDS tables);
+//   phase 1  clear the accumulators of the pass's slots;
+//   phase 2  the pixels are sorted by slot, and a lane per eight pixels of
+//            a slot sums its terms: the output gradient of a flat slot, the
+//            28 sums below of a smooth one (whose triangle the lane transforms);
+//   phase 3  per visible slot: chain the sums to instance colours (global
+//            atomics; LDS for rows shared by all scenes), light and
+//            vertex gradients (LDS tables);
 //   phase 4  the workgroup writes its light / vertex / shared-colour partial
 //            row; reduce_kernel sums the rows of all workgroups.
+//
+// The sums of a smooth slot: with u_k the weights, gn the gradient of the loss
+// with respect to n, G that with respect to the Lambert term ndl and P =
+// (px, py, 1): sum g_c, sum g_c ndl, sum G n^, sum u_k gn and
+// sum (gn . n_k) P.  Colour and light gradients are linear in the first two.
+// The last two keep one sum per vertex: their common factor sum P gn^T would
+// need only nine, but its products with the vertices' coefficients cancel
+// for slivers (vertex gradients moved by 4e-5 of their norm).
 //
 // Scenes whose nodes all shade flat and whose slots fit one LDS pass take
 // backward_flat_kernel instead: a persistent grid of five-wave workgroups in
@@ -56,16 +62,19 @@ using namespace pbr_host;
 namespace {
 
 constexpr int kBwdBlock = 256;
-constexpr int kRun = 16;   // pixels of one row walked by a lane
-constexpr int kAcc = 32;   // accumulator floats per slot
-constexpr int kRecF = 24;  // per-pixel factors per slot
+constexpr int kRun = 16;   // flat kernel: pixels of one column walked by a lane
+constexpr int kPix = 8;    // per-scene kernel: pixels of one row a thread sorts, and of
+                           // one slot a lane then sums
+constexpr int kSortPixels = kBwdBlock * kPix;  // pixels sorted at a time
+constexpr int kAcc = 29;   // accumulator floats per slot (28, odd to spread LDS banks)
+constexpr int kRecF = 23;  // per-pixel factors per slot
 constexpr int kLightF = 10;
 constexpr int kMaxCap = 512;          // flat kernel: slots held in LDS
-// per-scene kernel: slots held in LDS per pass (43 KiB of factors and
-// accumulators: three workgroups fit a CU).  Measured on MI355X for the
-// 512-scene 128 x 128 smooth workload's backward: 128 -> 525 us, 160 -> 462,
-// 192 -> 442, 224 -> 541, 320 -> 502 (two workgroups per CU).
-constexpr int kPassCap = 192;
+// per-scene kernel: slots held in LDS per pass (at most one per thread): with
+// the vertex table of a few hundred vertices 38 KiB, four workgroups per CU.
+// Measured on MI355X for the 512-scene 128 x 128 smooth workload: 128 -> 259
+// us, 160 -> 252, 192 -> 251, 224 -> 243, 256 (three workgroups per CU) -> 307.
+constexpr int kPassCap = 224;
 // per-scene kernel: rows per band when a scene is split over several
 // workgroups, and the workgroup count up to which scenes are split
 constexpr int kBandRows = 16;
@@ -74,13 +83,19 @@ constexpr int kMaxVtab = 2048;        // vertices whose gradients an LDS table h
 constexpr int kMaxStab = 1024;        // shared instance rows held in LDS
 constexpr int kMaxBitmapSlots = 1 << 17;
 
-// accumulator layout of a smooth slot (a flat slot keeps sum g_c in 0..3)
-constexpr int A_COL = 0, A_ALPHA = 3, A_GL = 4, A_GCOL = 7, A_GAMB = 10, A_GS = 13, A_GN = 14,
-              A_GP = 23;
-static_assert(A_GP + 9 == kAcc, "accumulator layout");
+// accumulator layout of a slot: sum g_c (a flat slot keeps only these), then
+// of a smooth one sum g_c ndl, sum G n^, sum u_k gn and sum (gn . n_k) P
+constexpr int A_G = 0, A_GD = 4, A_GL = 7, A_GN = 10, A_GP = 19;
+static_assert(A_GP + 9 <= kAcc, "accumulator layout");
 
-// per-pixel factors of a smooth slot
-constexpr int R_C = 0, R_N = 9, R_RGBA = 18, R_O = 22;
+// per-pixel factors of a smooth slot: h_a x h_b and the normal of each vertex,
+// rgba_c s col_c, the frame's origin
+constexpr int R_C = 0, R_N = 9, R_W = 18, R_O = 21;
+static_assert(R_O + 2 == kRecF, "factor layout");
+
+// Shading terms of a summed output gradient (shade_back): colour, alpha and
+// the light in the order of kLightF.
+constexpr int T_COL = 0, T_ALPHA = 3, T_GL = 4, T_GCOL = 7, T_GAMB = 10, T_GS = 13, kTerms = 14;
 
 struct BwdLight {
   float dir[3];  // L^
@@ -125,47 +140,76 @@ struct BTri {
   float rgba[4];
 };
 
-__device__ __forceinline__ void bwd_fetch(const pbr_scene_desc& D, int s, const uint32_t* base,
-                                          uint32_t slot, BTri& T) {
+// Node facts of the per-scene kernel in LDS.
+struct BNode {
+  const float* trans;
+  const float* cols;
+  float* gcol;
+  float inv_nt;    // 1 / triangles
+  int32_t ntri, ips, voff, ioff, soff;
+  uint32_t flags;  // bit 0: shared, bit 1: flat
+  uint32_t pad;
+};
+static_assert(sizeof(BNode) == 56, "BNode layout");
+
+typedef __attribute__((address_space(1))) const float global_cfloat;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const f32x4 global_cfloat4;
+typedef __attribute__((address_space(1))) const int32_t global_cint;
+
+// Float atomic add through a global-address-space pointer (a generic
+// pointer would take the flat atomic's shared / private aperture checks).
+typedef __attribute__((address_space(1))) float global_float;
+__device__ __forceinline__ void global_add(float* p, float v) {
+  __hip_atomic_fetch_add((global_float*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// `s` is wave-uniform (the view-projection sits in scalar registers).
+// `base`: first slots of the scene's nodes.
+__device__ __forceinline__ void bwd_fetch(const pbr_scene_desc& D, int s, const BNode* nodes,
+                                          const uint32_t* base, uint32_t slot, BTri& T) {
   int j = 0;
-  while (j + 1 < D.num_nodes && slot >= base[j + 1]) ++j;
-  const pbr_node& nd = D.nodes[j];
-  const pbr_mesh& me = D.meshes[nd.mesh];
+  for (int k = 1; k < D.num_nodes; ++k) j = slot >= base[k] ? k : j;
+  const BNode& nd = nodes[j];
   const uint32_t local = slot - base[j];
-  const uint32_t ntri = (uint32_t)me.num_triangles;
-  const uint32_t i = local / ntri, t = local - i * ntri;
-  const size_t row = nd.shared ? (size_t)i : (size_t)s * (size_t)nd.instances_per_scene + i;
+  // local / ntri from a float reciprocal: below 2^17, so the truncated product
+  // is off by at most one and one step corrects it
+  uint32_t i = (uint32_t)((float)local * nd.inv_nt);
+  int32_t t = (int32_t)(local - i * (uint32_t)nd.ntri);
+  if (t < 0) {
+    --i;
+    t += nd.ntri;
+  } else if (t >= nd.ntri) {
+    ++i;
+    t -= nd.ntri;
+  }
+  const size_t row = (nd.flags & 1u) ? (size_t)i : (size_t)s * (size_t)nd.ips + i;
   T.node = j;
   T.row = (uint32_t)row;
-  T.flat = nd.flat != 0;
-  const float4* M4 = reinterpret_cast<const float4*>(nd.transforms + row * 16);
+  T.flat = (nd.flags & 2u) != 0u;
+  global_cfloat4* M4 = (global_cfloat4*)(nd.trans + row * 16);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float4 m = M4[r];
+    const f32x4 m = M4[r];
     T.M[r * 4 + 0] = m.x;
     T.M[r * 4 + 1] = m.y;
     T.M[r * 4 + 2] = m.z;
     T.M[r * 4 + 3] = m.w;
   }
-  const float4* V4 = reinterpret_cast<const float4*>(D.view_proj + (size_t)s * 16);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float4 q = V4[r];
-    T.VP[r * 4 + 0] = q.x;
-    T.VP[r * 4 + 1] = q.y;
-    T.VP[r * 4 + 2] = q.z;
-    T.VP[r * 4 + 3] = q.w;
-  }
-  const float4 c4 = reinterpret_cast<const float4*>(nd.colors)[row];
+  load_mat4_uniform(D.view_proj + (size_t)s * 16, T.VP);
+  const f32x4 c4 = ((global_cfloat4*)nd.cols)[row];
   T.rgba[0] = c4.x;
   T.rgba[1] = c4.y;
   T.rgba[2] = c4.z;
   T.rgba[3] = c4.w;
-  const int32_t* tri = D.indices + (size_t)(me.index_offset + (int)t) * 3;
+  global_cint* tri = (global_cint*)D.indices + (size_t)(nd.ioff + t) * 3;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) T.vidx[k] = nd.voff + tri[k];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    T.vidx[k] = me.vertex_offset + tri[k];
-    const float* vv = D.vertices + (size_t)T.vidx[k] * 6;
+    float vv[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) vv[q] = ((global_cfloat*)D.vertices)[(size_t)T.vidx[k] * 6 + q];
     float wp[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -253,7 +297,7 @@ __device__ __forceinline__ float len3(const float v[3]) {
 
 // Shading terms shared by the per-pixel and per-slot chains: given the
 // interpolated normal n and the output gradient g, add the colour, light and
-// normal gradients to a[] (layout A_*) and return d loss / d n in gn.
+// normal gradients to a[] (layout T_*) and return d loss / d n in gn.
 __device__ __forceinline__ void shade_back(const float n[3], const float rgba[4], const float g[4],
                                            int C, const BwdLight& L, float* a, float gn[3]) {
   const float r = len3(n);
@@ -272,19 +316,19 @@ __device__ __forceinline__ void shade_back(const float n[3], const float rgba[4]
       const float light = L.amb[c] + ndl * L.col[c];
       const float l = (1.0f - L.s) + light * L.s;
       const float t = g[c] * rgba[c];
-      a[A_COL + c] += g[c] * l;
-      a[A_GAMB + c] += t * L.s;
-      a[A_GCOL + c] += t * L.s * ndl;
-      a[A_GS] += t * (light - 1.0f);
+      a[T_COL + c] += g[c] * l;
+      a[T_GAMB + c] += t * L.s;
+      a[T_GCOL + c] += t * L.s * ndl;
+      a[T_GS] += t * (light - 1.0f);
       G += t * L.s * L.col[c];
     }
   }
-  if (C > 3) a[A_ALPHA] += g[3];
+  if (C > 3) a[T_ALPHA] += g[3];
   float gnn[3] = {0.0f, 0.0f, 0.0f};
   if (ndl_raw > 0.0f) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      a[A_GL + c] += G * nn[c];
+      a[T_GL + c] += G * nn[c];
       gnn[c] = G * L.dir[c];
     }
   }
@@ -292,18 +336,21 @@ __device__ __forceinline__ void shade_back(const float n[3], const float rgba[4]
 }
 
 struct BwdLds {
-  float* rec;       // [cap][kRecF]
-  float* acc;       // [cap][kAcc]
-  uint32_t* flags;  // [cap] bit 0: smooth
-  uint32_t* list;   // [cap] slot of pass entry (compact)
+  float* acc;       // [cap][kAcc], or [cap][kAccFlat]
+  uint32_t* list;   // [cap] slot of pass entry, bit 31: smooth
   uint32_t* bitmap; // [nwords]
   uint32_t* wpre;   // [nwords] visible slots before word w
-  float* light;     // [kLightF]
+  float* light;     // [16]
   float* vtab;      // [vtab][6]
   float* stab;      // [stab][4]
   uint32_t* base;   // [PBR_MAX_NODES + 1]
-  uint32_t* misc;   // [0] visible slots, [1..] scan scratch (kBwdBlock)
+  uint32_t* misc;   // [kBwdBlock / 64] scan totals of the waves
+  BNode* nodes;     // [PBR_MAX_NODES]
+  uint32_t* count;  // [cap] pixels of pass entry in the current chunk
+  uint32_t* first;  // [cap] their first place in `order` | first unit << 16
+  uint16_t* order;  // [kSortPixels] pixels of the chunk by pass entry
 };
+constexpr int kAccFlat = 5;  // four sums, odd to spread LDS banks
 
 __device__ __forceinline__ void lds_add(float* p, float v) {
   if (v != 0.0f) atomicAdd(p, v);
@@ -319,6 +366,23 @@ __device__ __forceinline__ int pass_index(const BwdFrame& F, const BwdLds& S, ui
   }
   ci -= pbase;
   return (ci >= 0 && ci < cnt) ? ci : -1;
+}
+
+// Sum of v over the 64 lanes, in lane 63 (every lane active): row-wise
+// inclusive scans by row shifts 1, 2, 4, 8, then row broadcasts of lanes 15
+// and 31; lanes without a source add 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_src(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float wave_sum63(float v) {
+  v += dpp_src<0x111, 0xf>(v);  // row_shr:1
+  v += dpp_src<0x112, 0xf>(v);  // row_shr:2
+  v += dpp_src<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_src<0x118, 0xf>(v);  // row_shr:8
+  v += dpp_src<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_src<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
 }
 
 // The light, vertex and shared-colour sums of one workgroup as its partial
@@ -341,35 +405,50 @@ __device__ __forceinline__ void write_partial(const BwdFrame& F, const BwdLight&
   for (int i = tid; i < F.stab * 4; i += nthreads) row[F.off_s + i] = stab[i];
 }
 
-// SMOOTH: some node shades with interpolated normals (32 accumulators per
-// run, 8-pixel runs); otherwise every slot is flat (4 accumulators, 16-pixel
-// runs).
-template <bool SMOOTH>
-__global__ __launch_bounds__(kBwdBlock) void backward_kernel(pbr_scene_desc D, BwdFrame F,
+// Visible slots of the RUN pixels at vr (n of them in the row, -1 past it).
+template <int RUN>
+__device__ __forceinline__ void load_ids(int32_t v[RUN], const int32_t* vr, int n, bool vec) {
+  if (vec && n == RUN) {
+#pragma unroll
+    for (int q = 0; q < RUN / 4; ++q) {
+      const int4 t = reinterpret_cast<const int4*>(vr)[q];
+      v[4 * q] = t.x;
+      v[4 * q + 1] = t.y;
+      v[4 * q + 2] = t.z;
+      v[4 * q + 3] = t.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) v[i] = i < n ? vr[i] : -1;
+  }
+}
+
+// SMOOTH: some node shades with interpolated normals (28 sums per slot);
+// otherwise every slot is flat (4 sums).  Held to 128 VGPRs: four workgroups
+// share a CU where their LDS allows it.
+template <bool SMOOTH, int NC>
+__global__ __launch_bounds__(kBwdBlock)
+__attribute__((amdgpu_waves_per_eu(4))) void backward_kernel(pbr_scene_desc D, BwdFrame F,
                                                              BwdLight L, BwdGrads G,
-                                                             const int32_t* vis,
-                                                             const float* gout, float* partial) {
-  constexpr int RUN = SMOOTH ? 8 : kRun;
+                                                             const int32_t* vis, const float* gout,
+                                                             float* partial) {
+  constexpr int RUN = kPix;
+  constexpr int ACC = SMOOTH ? kAcc : kAccFlat;
+  constexpr int NL = NC < 3 ? NC : 3;  // channels the light shades
   extern __shared__ __align__(16) unsigned char smem[];
-  // workgroup -> (scene, band of rows [y0, y1))
-  const int s = (int)blockIdx.x / F.bands;
-  const int band = (int)blockIdx.x - s * F.bands;
-  const int y0 = band * F.band_rows;
-  const int y1 = min(F.H, y0 + F.band_rows);
-  const int tid = (int)threadIdx.x;
-  const int W = F.W, H = F.H, C = F.C;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int W = F.W, H = F.H;
   const size_t plane = (size_t)W * (size_t)H;
 
   // carve LDS
   BwdLds S;
   {
     unsigned char* p = smem;
-    S.rec = reinterpret_cast<float*>(p);
-    p += sizeof(float) * (size_t)F.cap * kRecF;
+    S.nodes = reinterpret_cast<BNode*>(p);
+    p += sizeof(BNode) * PBR_MAX_NODES;
     S.acc = reinterpret_cast<float*>(p);
-    p += sizeof(float) * (size_t)F.cap * kAcc;
-    S.flags = reinterpret_cast<uint32_t*>(p);
-    p += sizeof(uint32_t) * (size_t)F.cap;
+    p += sizeof(float) * (size_t)F.cap * ACC;
     S.list = reinterpret_cast<uint32_t*>(p);
     p += sizeof(uint32_t) * (size_t)F.cap;
     S.bitmap = reinterpret_cast<uint32_t*>(p);
@@ -385,75 +464,101 @@ __global__ __launch_bounds__(kBwdBlock) void backward_kernel(pbr_scene_desc D, B
     S.base = reinterpret_cast<uint32_t*>(p);
     p += sizeof(uint32_t) * (PBR_MAX_NODES + 1);
     S.misc = reinterpret_cast<uint32_t*>(p);
+    p += sizeof(uint32_t) * (kBwdBlock / 64);
+    S.count = reinterpret_cast<uint32_t*>(p);
+    p += sizeof(uint32_t) * (size_t)F.cap;
+    S.first = reinterpret_cast<uint32_t*>(p);
+    p += sizeof(uint32_t) * (size_t)F.cap;
+    S.order = reinterpret_cast<uint16_t*>(p);
   }
-  if (tid == 0) {
-    uint32_t acc = 0;
-    for (int j = 0; j < D.num_nodes; ++j) {
-      const pbr_node& nd = D.nodes[j];
-      int cnt = nd.instances_per_scene;
-      if (nd.counts) cnt = min(max(nd.counts[s], 0), nd.instances_per_scene);
-      S.base[j] = acc;
-      acc += (uint32_t)cnt * (uint32_t)D.meshes[nd.mesh].num_triangles;
-    }
-    S.base[D.num_nodes] = acc;
+  if (tid < D.num_nodes) {
+    const pbr_node& nd = D.nodes[tid];
+    const pbr_mesh& me = D.meshes[nd.mesh];
+    BNode e;
+    e.trans = nd.transforms;
+    e.cols = nd.colors;
+    e.gcol = G.colors[tid];
+    e.ntri = max(me.num_triangles, 1);
+    e.inv_nt = 1.0f / (float)e.ntri;
+    e.ips = nd.instances_per_scene;
+    e.voff = me.vertex_offset;
+    e.ioff = me.index_offset;
+    e.soff = F.soff[tid];
+    e.flags = (nd.shared ? 1u : 0u) | (nd.flat ? 2u : 0u);
+    e.pad = 0u;
+    S.nodes[tid] = e;
   }
   for (int i = tid; i < 16; i += kBwdBlock) S.light[i] = 0.0f;
   for (int i = tid; i < F.vtab * 6; i += kBwdBlock) S.vtab[i] = 0.0f;
   for (int i = tid; i < F.stab * 4; i += kBwdBlock) S.stab[i] = 0.0f;
+  const int segs = (W + RUN - 1) / RUN;
+  // workgroup -> (scene, band of rows [y0, y1)): the middle bands, which
+  // tend to show most, start first (static shares of a resident grid's
+  // workgroups instead: 249 against 235 us, the reduction included)
+  const int k = (int)blockIdx.x / D.num_scenes, s = (int)blockIdx.x - k * D.num_scenes;
+  const int band = F.bands / 2 + ((k & 1) ? -(k + 1) / 2 : k / 2);
+  const int y0 = band * F.band_rows;
+  const int y1 = min(H, y0 + F.band_rows);
+  const int nruns = max(0, y1 - y0) * segs;
+  const int32_t* vscene = vis + (size_t)s * plane;
+  const float* gscene = gout + (size_t)s * (size_t)NC * plane;
+  if (wave == 0) {
+    uint32_t n = 0;
+    if (lane < D.num_nodes) {
+      const pbr_node& nd = D.nodes[lane];
+      int cnt = nd.instances_per_scene;
+      if (nd.counts) cnt = min(max(nd.counts[s], 0), nd.instances_per_scene);
+      n = (uint32_t)cnt * (uint32_t)D.meshes[nd.mesh].num_triangles;
+    }
+    const uint32_t incl = (uint32_t)wave_scan_add((int)n);
+    if (lane <= D.num_nodes) S.base[lane] = incl - n;
+  }
   for (int i = tid; i < F.nwords; i += kBwdBlock) S.bitmap[i] = 0u;
   __syncthreads();
   const uint32_t total = S.base[D.num_nodes];
 
-  const int segs = (W + RUN - 1) / RUN;
-  const int nruns = max(0, y1 - y0) * segs;
-  const int32_t* vscene = vis + (size_t)s * plane;
-  const float* gscene = gout + (size_t)s * (size_t)C * plane;
-
   // phase 0: visible slots
   int nvis = (int)total;
+  const int nw = (int)((total + 31u) / 32u);
   if (F.compact) {
     for (int run = tid; run < nruns; run += kBwdBlock) {
-      const int yr = run / segs, x0 = (run - yr * segs) * RUN, y = y0 + yr;
+      const int yr = run / segs, x0 = (run - yr * segs) * RUN;
       const int n = min(RUN, W - x0);
-      const int32_t* vr = vscene + (size_t)y * W + x0;
-      int32_t prev = -1;
-      for (int i = 0; i < n; ++i) {
-        const int32_t v = vr[i];
-        if (v != prev && v >= 0 && (uint32_t)v < total)
-          atomicOr(&S.bitmap[(uint32_t)v >> 5], 1u << ((uint32_t)v & 31u));
-        prev = v;
-      }
+      const int32_t* vr = vscene + (size_t)(y0 + yr) * W + x0;
+      int32_t v[RUN];
+      load_ids<RUN>(v, vr, n, F.vec != 0);
+#pragma unroll
+      for (int i = 0; i < RUN; ++i)
+        if ((i == 0 || v[i] != v[i - 1]) && v[i] >= 0 && (uint32_t)v[i] < total)
+          atomicOr(&S.bitmap[(uint32_t)v[i] >> 5], 1u << ((uint32_t)v[i] & 31u));
     }
     __syncthreads();
     // exclusive scan of popcounts: each thread owns a contiguous chunk
-    const int nw = (int)((total + 31u) / 32u);
     const int chunk = (nw + kBwdBlock - 1) / kBwdBlock;
     const int w0 = min(nw, tid * chunk), w1 = min(nw, w0 + chunk);
     uint32_t mine = 0;
     for (int w = w0; w < w1; ++w) mine += (uint32_t)__popc(S.bitmap[w]);
-    uint32_t* scan = S.misc + 1;
-    scan[tid] = mine;
+    const uint32_t incl = (uint32_t)wave_scan_add((int)mine);
+    if (lane == 63) S.misc[wave] = incl;
     __syncthreads();
-    for (int d = 1; d < kBwdBlock; d <<= 1) {
-      const uint32_t t = tid >= d ? scan[tid - d] : 0u;
-      __syncthreads();
-      scan[tid] += t;
-      __syncthreads();
+    uint32_t run_pre = incl - mine, all = 0;
+#pragma unroll
+    for (int w = 0; w < kBwdBlock / 64; ++w) {
+      const uint32_t n = S.misc[w];
+      run_pre += w < wave ? n : 0u;
+      all += n;
     }
-    uint32_t run_pre = scan[tid] - mine;
     for (int w = w0; w < w1; ++w) {
       S.wpre[w] = run_pre;
       run_pre += (uint32_t)__popc(S.bitmap[w]);
     }
-    if (tid == kBwdBlock - 1) S.misc[0] = scan[tid];
+    nvis = (int)all;
     __syncthreads();
-    nvis = (int)S.misc[0];
   }
 
   for (int pbase = 0; pbase < nvis; pbase += F.cap) {
     const int cnt = min(F.cap, nvis - pbase);
     if (F.compact) {
-      const int nw = (int)((total + 31u) / 32u);
       for (int w = tid; w < nw; w += kBwdBlock) {
         uint32_t bits = S.bitmap[w];
         int ci = (int)S.wpre[w] - pbase;
@@ -466,281 +571,350 @@ __global__ __launch_bounds__(kBwdBlock) void backward_kernel(pbr_scene_desc D, B
       }
       __syncthreads();
     }
-    // phase 1: per-pixel factors of the pass's slots
+    // phase 1: the pass's slots
     for (int li = tid; li < cnt; li += kBwdBlock) {
       const uint32_t slot = F.compact ? S.list[li] : (uint32_t)(pbase + li);
-      float* a = S.acc + (size_t)li * kAcc;
+      int j = 0;
+      for (int k = 1; k < D.num_nodes; ++k) j = slot >= S.base[k] ? k : j;
+      S.list[li] = slot | (SMOOTH && !(S.nodes[j].flags & 2u) ? 0x80000000u : 0u);
+      S.count[li] = 0u;
+      float* a = S.acc + (size_t)li * ACC;
 #pragma unroll
-      for (int q = 0; q < kAcc; ++q) a[q] = 0.0f;
-      const int j = [&] {
-        int jj = 0;
-        while (jj + 1 < D.num_nodes && slot >= S.base[jj + 1]) ++jj;
-        return jj;
-      }();
-      const bool smooth = SMOOTH && D.nodes[j].flat == 0;
-      S.flags[li] = smooth ? 1u : 0u;
-      if (SMOOTH && smooth) {
-        BTri T;
-        bwd_fetch(D, s, S.base, slot, T);
-        float h[3][3], ox, oy;
-        local_frame(T, W, H, h, ox, oy);
-        const float w012 = T.p[0][3] * T.p[1][3] * T.p[2][3];
-        const float sg = w012 < 0.0f ? -1.0f : 1.0f;
-        float* r = S.rec + (size_t)li * kRecF;
-        r[R_O] = ox;
-        r[R_O + 1] = oy;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          float ck[3];
-          cross3(h[(k + 1) % 3], h[(k + 2) % 3], ck);
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            r[R_C + 3 * k + c] = sg * ck[c];
-            r[R_N + 3 * k + c] = T.nw[k][c];
-          }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) r[R_RGBA + c] = T.rgba[c];
-      }
+      for (int q = 0; q < ACC; ++q) a[q] = 0.0f;
     }
     __syncthreads();
 
-    // phase 2: pixel runs
-    for (int run = tid; run < nruns; run += kBwdBlock) {
-      const int yr = run / segs, x0 = (run - yr * segs) * RUN, y = y0 + yr;
-      const int n = min(RUN, W - x0);
-      const int32_t* vr = vscene + (size_t)y * W + x0;
-      const float* gr = gscene + (size_t)y * W + x0;
-      const float py = (float)(H - 1 - y) + 0.5f;
-      // the run's visibility and output gradient, loaded up front
-      int32_t vv[RUN];
-      float gg[4][RUN];
-      if (F.vec && n == RUN) {
+    // phase 2: the band's pixels, a chunk at a time, sorted by slot; then a
+    // lane per eight pixels of one slot sums them in registers and adds its
+    // sums to the slot's accumulator once.  (Lanes that walk eight pixels of
+    // a row flush at every change of slot, with few lanes active: their LDS
+    // atomics kept the LDS pipe busy half of the kernel's time.)
+    const float inv_segs = 1.0f / (float)segs;
+    for (int r0 = 0; r0 < nruns; r0 += kBwdBlock) {
+      const int run = r0 + tid;
+      int li[kPix], pos[kPix];
+      {
+        const int yr = run / segs, x0 = (run - yr * segs) * kPix;
+        const int n = run < nruns ? min(kPix, W - x0) : 0;
+        int32_t v[kPix];
+        if (n > 0) load_ids<kPix>(v, vscene + (size_t)(y0 + yr) * W + x0, n, F.vec != 0);
 #pragma unroll
-        for (int q = 0; q < RUN / 4; ++q) {
-          const int4 t = reinterpret_cast<const int4*>(vr)[q];
-          vv[4 * q] = t.x;
-          vv[4 * q + 1] = t.y;
-          vv[4 * q + 2] = t.z;
-          vv[4 * q + 3] = t.w;
+        for (int i = 0; i < kPix; ++i) {
+          if (n == 0)
+            li[i] = -1;
+          else if (i > 0 && v[i] == v[i - 1])
+            li[i] = li[i - 1];
+          else
+            li[i] = pass_index(F, S, total, v[i], pbase, cnt);
         }
+        // places within the slot: one count per stretch of equal slots
+        int len[kPix];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int i = kPix - 1; i >= 0; --i)
+          len[i] = i + 1 < kPix && li[i + 1] == li[i] ? len[i + 1] + 1 : 1;
 #pragma unroll
-          for (int q = 0; q < RUN / 4; ++q) {
-            float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (c < C) t = reinterpret_cast<const float4*>(gr + (size_t)c * plane)[q];
-            gg[c][4 * q] = t.x;
-            gg[c][4 * q + 1] = t.y;
-            gg[c][4 * q + 2] = t.z;
-            gg[c][4 * q + 3] = t.w;
+        for (int i = 0; i < kPix; ++i) {
+          if (i > 0 && li[i] == li[i - 1]) {
+            pos[i] = pos[i - 1] + 1;
+          } else {
+            pos[i] = 0;
+            if (li[i] >= 0) pos[i] = (int)atomicAdd(&S.count[li[i]], (uint32_t)len[i]);
           }
         }
-      } else {
+      }
+      __syncthreads();
+      // first place and first unit (eight pixels) of every slot: cap <= 256
+      uint32_t packed = 0;
+      if (tid < cnt) {
+        const uint32_t n = S.count[tid];
+        packed = n | ((n + kPix - 1u) / kPix) << 16;
+      }
+      const uint32_t incl = (uint32_t)wave_scan_add((int)packed);
+      if (lane == 63) S.misc[wave] = incl;
+      __syncthreads();
+      uint32_t before = incl - packed, units = 0;
 #pragma unroll
-        for (int i = 0; i < RUN; ++i) {
-          vv[i] = i < n ? vr[i] : -1;
+      for (int w = 0; w < kBwdBlock / 64; ++w) {
+        const uint32_t n = S.misc[w];
+        before += w < wave ? n : 0u;
+        units += n;
+      }
+      units >>= 16;
+      if (tid < cnt) S.first[tid] = before;
+      __syncthreads();
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            gg[c][i] = (i < n && c < C) ? gr[(size_t)c * plane + i] : 0.0f;
+      for (int i = 0; i < kPix; ++i)
+        if (li[i] >= 0)
+          S.order[(S.first[li[i]] & 0xffffu) + (uint32_t)pos[i]] = (uint16_t)(tid * kPix + i);
+      __syncthreads();
+      for (uint32_t u = (uint32_t)tid; u < units; u += kBwdBlock) {
+        // the slot: the last one whose first unit is <= u (slots without
+        // pixels share their successor's first unit)
+        int sl = 0;
+#pragma unroll
+        for (int d = 128; d > 0; d >>= 1)
+          if (sl + d < cnt && (S.first[sl + d] >> 16) <= u) sl += d;
+        const uint32_t f = S.first[sl];
+        const uint32_t p0 = (u - (f >> 16)) * kPix;
+        const int n = (int)min((uint32_t)kPix, S.count[sl] - p0);
+        const uint16_t* ord = S.order + (f & 0xffffu) + p0;
+        int px[kPix], py[kPix];  // columns and GL rows
+        float g[NC][kPix];
+#pragma unroll
+        for (int i = 0; i < kPix; ++i) {
+          const int id = ord[min(i, n - 1)];
+          const int rr = r0 + (id >> 3);
+          const int yr = (int)(((float)rr + 0.5f) * inv_segs);
+          px[i] = (rr - yr * segs) * kPix + (id & 7);
+          py[i] = H - 1 - (y0 + yr);
+          const size_t at = (size_t)(y0 + yr) * W + px[i];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) g[c][i] = ((global_cfloat*)gscene)[(size_t)c * plane + at];
+        }
+        float a[ACC];
+#pragma unroll
+        for (int q = 0; q < ACC; ++q) a[q] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kPix; ++i)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            g[c][i] = i < n ? g[c][i] : 0.0f;
+            a[A_G + c] += g[c][i];
+          }
+        float* dst = S.acc + (size_t)sl * ACC;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) atomicAdd(dst + A_G + c, a[A_G + c]);
+        if constexpr (SMOOTH) {
+          if (S.list[sl] >> 31) {
+            // the slot's per-pixel factors, made again by each of its lanes:
+            // in LDS they would take the room of every other slot
+            float r[kRecF];
+            {
+              BTri T;
+              bwd_fetch(D, s, S.nodes, S.base, S.list[sl] & 0x7fffffffu, T);
+              float h[3][3];
+              local_frame(T, W, H, h, r[R_O], r[R_O + 1]);
+              const float w012 = T.p[0][3] * T.p[1][3] * T.p[2][3];
+              const float sg = w012 < 0.0f ? -1.0f : 1.0f;
+#pragma unroll
+              for (int k = 0; k < 3; ++k) {
+                float ck[3];
+                cross3(h[(k + 1) % 3], h[(k + 2) % 3], ck);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                  r[R_C + 3 * k + c] = sg * ck[c];
+                  r[R_N + 3 * k + c] = T.nw[k][c];
+                }
+              }
+#pragma unroll
+              for (int c = 0; c < 3; ++c) r[R_W + c] = T.rgba[c] * L.s * L.col[c];
+            }
+#pragma unroll
+            for (int i = 0; i < kPix; ++i) {
+              if (i >= n) break;
+              const float x = (float)px[i] + 0.5f - r[R_O];
+              const float y = (float)py[i] + 0.5f - r[R_O + 1];
+              float u3[3], nm[3], nn[3];
+#pragma unroll
+              for (int k = 0; k < 3; ++k)
+                u3[k] = r[R_C + 3 * k] * x + r[R_C + 3 * k + 1] * y + r[R_C + 3 * k + 2];
+#pragma unroll
+              for (int c = 0; c < 3; ++c)
+                nm[c] = u3[0] * r[R_N + c] + u3[1] * r[R_N + 3 + c] + u3[2] * r[R_N + 6 + c];
+              const float len = len3(nm);
+              const float inv = len > 0.0f ? 1.0f / len : 0.0f;
+#pragma unroll
+              for (int c = 0; c < 3; ++c) nn[c] = nm[c] * inv;
+              const float raw = nn[0] * L.dir[0] + nn[1] * L.dir[1] + nn[2] * L.dir[2];
+              const float ndl = fmaxf(raw, 0.0f);
+              float Gw = 0.0f;
+#pragma unroll
+              for (int c = 0; c < NL; ++c) {
+                a[A_GD + c] += g[c][i] * ndl;
+                Gw += g[c][i] * r[R_W + c];
+              }
+              Gw = raw > 0.0f ? Gw : 0.0f;
+              const float Gi = Gw * inv;
+              float gn[3];
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                a[A_GL + c] += Gw * nn[c];
+                gn[c] = Gi * (L.dir[c] - nn[c] * ndl);
+              }
+#pragma unroll
+              for (int k = 0; k < 3; ++k) {
+                const float guk = gn[0] * r[R_N + 3 * k] + gn[1] * r[R_N + 3 * k + 1] +
+                                  gn[2] * r[R_N + 3 * k + 2];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) a[A_GN + 3 * k + c] += u3[k] * gn[c];
+                a[A_GP + 3 * k + 0] += guk * x;
+                a[A_GP + 3 * k + 1] += guk * y;
+                a[A_GP + 3 * k + 2] += guk;
+              }
+            }
+#pragma unroll
+            for (int c = 0; c < NL; ++c) atomicAdd(dst + A_GD + c, a[A_GD + c]);
+#pragma unroll
+            for (int q = A_GL; q < A_GP + 9; ++q) atomicAdd(dst + q, a[q]);
+          }
         }
       }
-      int cur = -1;
-      bool cur_smooth = false;
-      float a[kAcc];
+      __syncthreads();
+      if (r0 + kBwdBlock < nruns) {
+        if (tid < cnt) S.count[tid] = 0u;
+        __syncthreads();
+      }
+    }
+
+    // phase 3: per-slot chain to the parameters
+    // (a whole wave runs or skips a round: its light terms are summed across
+    // the lanes)
+    for (int l0 = wave * 64; l0 < cnt; l0 += kBwdBlock) {
+      const int li = l0 + lane;
+      float lsum[kLightF];
 #pragma unroll
-      for (int q = 0; q < kAcc; ++q) a[q] = 0.0f;
+      for (int q = 0; q < kLightF; ++q) lsum[q] = 0.0f;
+      float a[ACC];
+      bool any = false;
 #pragma unroll
-      for (int i = 0; i < RUN; ++i) {
-        const int li = pass_index(F, S, total, vv[i], pbase, cnt);
-        if (li != cur) {
-          if (cur >= 0) {
-            float* dst = S.acc + (size_t)cur * kAcc;
-            if (cur_smooth) {
+      for (int q = 0; q < ACC; ++q) {
+        a[q] = li < cnt ? S.acc[(size_t)li * ACC + q] : 0.0f;
+        any = any || (a[q] != 0.0f);
+      }
+      if (any) {
+        BTri T;
+        bwd_fetch(D, s, S.nodes, S.base, S.list[li] & 0x7fffffffu, T);
+        const bool smooth = SMOOTH && !T.flat;
+        float gnw[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+        float gc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float h[3][3], ox = 0.0f, oy = 0.0f, sg = 1.0f;
+        if (!smooth) {
+          // every term is linear in the summed output gradient
+          const float gs[4] = {a[0], a[1], a[2], a[3]};
+          float t[kTerms];
 #pragma unroll
-              for (int q = 0; q < kAcc; ++q) lds_add(dst + q, a[q]);
-            } else {
+          for (int q = 0; q < kTerms; ++q) t[q] = 0.0f;
+          float gn[3];
+          shade_back(T.nw[0], T.rgba, gs, NC, L, t, gn);
 #pragma unroll
-              for (int q = 0; q < 4; ++q) lds_add(dst + q, a[q]);
+          for (int c = 0; c < 3; ++c) gnw[0][c] = gn[c];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) gc[c] = t[T_COL + c];
+          gc[3] = t[T_ALPHA];
+#pragma unroll
+          for (int q = 0; q < kLightF; ++q) lsum[q] += t[T_GL + q];
+        } else if constexpr (SMOOTH) {
+#pragma unroll
+          for (int c = 0; c < NL; ++c) {
+            const float g = a[A_G + c], gd = a[A_GD + c], rs = T.rgba[c] * L.s;
+            gc[c] = ((1.0f - L.s) + L.amb[c] * L.s) * g + (L.col[c] * L.s) * gd;
+            lsum[3 + c] += rs * gd;
+            lsum[6 + c] += rs * g;
+            lsum[9] += T.rgba[c] * ((L.amb[c] - 1.0f) * g + L.col[c] * gd);
+          }
+          if (NC > 3) gc[3] = a[A_G + 3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) lsum[c] += a[A_GL + c];
+          local_frame(T, W, H, h, ox, oy);
+          const float w012 = T.p[0][3] * T.p[1][3] * T.p[2][3];
+          sg = w012 < 0.0f ? -1.0f : 1.0f;
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) gnw[k][c] = a[A_GN + 3 * k + c];
+        }
+        // instance colour
+        {
+          float* dst = nullptr;
+          const BNode& nd = S.nodes[T.node];
+          if ((nd.flags & 1u) && F.stab > 0) dst = S.stab + (size_t)(nd.soff + (int)T.row) * 4;
+          if (dst) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) lds_add(dst + c, gc[c]);
+          } else if (nd.gcol) {
+            float* gp = nd.gcol + (size_t)T.row * 4;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              if (gc[c] != 0.0f) global_add(gp + c, gc[c]);
+          }
+        }
+        // vertices: normals (through both normalisations) and, for smooth
+        // slots, positions through the homogeneous window coordinates
+        float gv[3][6];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          float gu[3];
+          normalize_back(T.nw[k], len3(T.u[k]), gnw[k], gu);
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            gv[k][3 + i] = T.M[0 * 4 + i] * gu[0] + T.M[1 * 4 + i] * gu[1] + T.M[2 * 4 + i] * gu[2];
+          gv[k][0] = gv[k][1] = gv[k][2] = 0.0f;
+        }
+        if (SMOOTH && smooth) {
+          float gh[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const int ia = (k + 1) % 3, ib = (k + 2) % 3;
+            const float gck[3] = {sg * a[A_GP + 3 * k], sg * a[A_GP + 3 * k + 1],
+                                  sg * a[A_GP + 3 * k + 2]};
+            float t0[3], t1[3];
+            cross3(h[ib], gck, t0);  // d/dh_a of (h_a x h_b) . gck
+            cross3(gck, h[ia], t1);  // d/dh_b
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              gh[ia][c] += t0[c];
+              gh[ib][c] += t1[c];
             }
           }
 #pragma unroll
-          for (int q = 0; q < kAcc; ++q) a[q] = 0.0f;
-          cur = li;
-          cur_smooth = SMOOTH && li >= 0 && (S.flags[li] & 1u);
-        }
-        if (cur < 0) continue;
-        const float g[4] = {gg[0][i], gg[1][i], gg[2][i], gg[3][i]};
-        if (!cur_smooth) {
+          for (int k = 0; k < 3; ++k) {
+            // back through the shear, then h = ((x + w) W/2, (y + w) H/2, w)
+            const float ghw = gh[k][2] - ox * gh[k][0] - oy * gh[k][1];
+            const float gx = gh[k][0] * (0.5f * (float)W), gy = gh[k][1] * (0.5f * (float)H);
+            const float gp[4] = {gx, gy, 0.0f, gx + gy + ghw};
+            float gw[4];
 #pragma unroll
-          for (int c = 0; c < 4; ++c) a[c] += g[c];
-          continue;
-        }
-        const float* r = S.rec + (size_t)cur * kRecF;
-        const float px = (float)(x0 + i) + 0.5f - r[R_O];
-        const float pyl = py - r[R_O + 1];
-        float u[3];
+            for (int r = 0; r < 4; ++r)
+              gw[r] = T.VP[0 * 4 + r] * gp[0] + T.VP[1 * 4 + r] * gp[1] + T.VP[2 * 4 + r] * gp[2] +
+                      T.VP[3 * 4 + r] * gp[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          u[k] = r[R_C + 3 * k] * px + r[R_C + 3 * k + 1] * pyl + r[R_C + 3 * k + 2];
-        float nrm[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-          nrm[c] = u[0] * r[R_N + c] + u[1] * r[R_N + 3 + c] + u[2] * r[R_N + 6 + c];
-        const float rgba[4] = {r[R_RGBA], r[R_RGBA + 1], r[R_RGBA + 2], r[R_RGBA + 3]};
-        float gn[3];
-        shade_back(nrm, rgba, g, C, L, a, gn);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const float guk = gn[0] * r[R_N + 3 * k] + gn[1] * r[R_N + 3 * k + 1] +
-                            gn[2] * r[R_N + 3 * k + 2];
-#pragma unroll
-          for (int c = 0; c < 3; ++c) a[A_GN + 3 * k + c] += u[k] * gn[c];
-          a[A_GP + 3 * k + 0] += guk * px;
-          a[A_GP + 3 * k + 1] += guk * pyl;
-          a[A_GP + 3 * k + 2] += guk;
-        }
-      }
-      if (cur >= 0) {
-        float* dst = S.acc + (size_t)cur * kAcc;
-        if (cur_smooth) {
-#pragma unroll
-          for (int q = 0; q < kAcc; ++q) lds_add(dst + q, a[q]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) lds_add(dst + q, a[q]);
-        }
-      }
-    }
-    __syncthreads();
-
-    // phase 3: per-slot chain to the parameters
-    for (int li = tid; li < cnt; li += kBwdBlock) {
-      const uint32_t slot = F.compact ? S.list[li] : (uint32_t)(pbase + li);
-      float a[kAcc];
-      const float* src = S.acc + (size_t)li * kAcc;
-#pragma unroll
-      for (int q = 0; q < kAcc; ++q) a[q] = src[q];
-      bool any = false;
-#pragma unroll
-      for (int q = 0; q < kAcc; ++q) any = any || (a[q] != 0.0f);
-      if (!any) continue;
-      BTri T;
-      bwd_fetch(D, s, S.base, slot, T);
-      float gnw[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-      float gc[4];
-      float gl[kLightF];
-      if (!SMOOTH || T.flat) {
-        // every term is linear in the summed output gradient
-        const float gs[4] = {a[0], a[1], a[2], a[3]};
-        float t[kAcc];
-#pragma unroll
-        for (int q = 0; q < kAcc; ++q) t[q] = 0.0f;
-        float gn[3];
-        shade_back(T.nw[0], T.rgba, gs, C, L, t, gn);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) gnw[0][c] = gn[c];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) gc[c] = t[A_COL + c];
-        gc[3] = t[A_ALPHA];
-#pragma unroll
-        for (int q = 0; q < kLightF; ++q) gl[q] = t[A_GL + q];
-      } else {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) gc[c] = a[A_COL + c];
-        gc[3] = a[A_ALPHA];
-#pragma unroll
-        for (int q = 0; q < kLightF; ++q) gl[q] = a[A_GL + q];
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) gnw[k][c] = a[A_GN + 3 * k + c];
-      }
-      // instance colour
-      {
-        float* dst = nullptr;
-        if (D.nodes[T.node].shared && F.stab > 0)
-          dst = S.stab + (size_t)(F.soff[T.node] + (int)T.row) * 4;
-        if (dst) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) lds_add(dst + c, gc[c]);
-        } else if (G.colors[T.node]) {
-          float* gp = G.colors[T.node] + (size_t)T.row * 4;
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (gc[c] != 0.0f) atomicAdd(gp + c, gc[c]);
-        }
-      }
-      // light
-#pragma unroll
-      for (int q = 0; q < kLightF; ++q) lds_add(S.light + q, gl[q]);
-      // vertices: normals (through both normalisations) and, for smooth
-      // slots, positions through the homogeneous window coordinates
-      float gv[3][6];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        float gu[3];
-        normalize_back(T.nw[k], len3(T.u[k]), gnw[k], gu);
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          gv[k][3 + i] = T.M[0 * 4 + i] * gu[0] + T.M[1 * 4 + i] * gu[1] + T.M[2 * 4 + i] * gu[2];
-        gv[k][0] = gv[k][1] = gv[k][2] = 0.0f;
-      }
-      if (SMOOTH && !T.flat) {
-        float h[3][3], ox, oy;
-        local_frame(T, W, H, h, ox, oy);
-        const float w012 = T.p[0][3] * T.p[1][3] * T.p[2][3];
-        const float sg = w012 < 0.0f ? -1.0f : 1.0f;
-        float gh[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const int ia = (k + 1) % 3, ib = (k + 2) % 3;
-          const float gck[3] = {sg * a[A_GP + 3 * k], sg * a[A_GP + 3 * k + 1],
-                                sg * a[A_GP + 3 * k + 2]};
-          float t0[3], t1[3];
-          cross3(h[ib], gck, t0);  // d/dh_a of (h_a x h_b) . gck
-          cross3(gck, h[ia], t1);  // d/dh_b
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            gh[ia][c] += t0[c];
-            gh[ib][c] += t1[c];
+            for (int i = 0; i < 3; ++i)
+              gv[k][i] = T.M[0 * 4 + i] * gw[0] + T.M[1 * 4 + i] * gw[1] + T.M[2 * 4 + i] * gw[2] +
+                         T.M[3 * 4 + i] * gw[3];
           }
         }
+        if (F.vtab > 0) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          // back through the shear, then h = ((x + w) W/2, (y + w) H/2, w)
-          const float ghw = gh[k][2] - ox * gh[k][0] - oy * gh[k][1];
-          const float gx = gh[k][0] * (0.5f * (float)W), gy = gh[k][1] * (0.5f * (float)H);
-          const float gp[4] = {gx, gy, 0.0f, gx + gy + ghw};
-          float gw[4];
+          for (int k = 0; k < 3; ++k)
+            if ((unsigned)T.vidx[k] < (unsigned)F.vtab) {
+              float* dst = S.vtab + (size_t)T.vidx[k] * 6;
+              if (smooth) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            gw[r] = T.VP[0 * 4 + r] * gp[0] + T.VP[1 * 4 + r] * gp[1] + T.VP[2 * 4 + r] * gp[2] +
-                    T.VP[3 * 4 + r] * gp[3];
+                for (int i = 0; i < 6; ++i) atomicAdd(dst + i, gv[k][i]);
+              } else if (k == 0) {  // only the first vertex's normal shades
 #pragma unroll
-          for (int i = 0; i < 3; ++i)
-            gv[k][i] = T.M[0 * 4 + i] * gw[0] + T.M[1 * 4 + i] * gw[1] + T.M[2 * 4 + i] * gw[2] +
-                       T.M[3 * 4 + i] * gw[3];
+                for (int i = 3; i < 6; ++i) atomicAdd(dst + i, gv[k][i]);
+              }
+            }
+        } else if (G.vertices) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+              if (gv[k][i] != 0.0f) atomicAdd(G.vertices + (size_t)T.vidx[k] * 6 + i, gv[k][i]);
         }
       }
-      if (F.vtab > 0) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if ((unsigned)T.vidx[k] < (unsigned)F.vtab)
-#pragma unroll
-            for (int i = 0; i < 6; ++i) lds_add(S.vtab + (size_t)T.vidx[k] * 6 + i, gv[k][i]);
-      } else if (G.vertices) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-          for (int i = 0; i < 6; ++i)
-            if (gv[k][i] != 0.0f) atomicAdd(G.vertices + (size_t)T.vidx[k] * 6 + i, gv[k][i]);
+      for (int q = 0; q < kLightF; ++q) {
+        const float t = wave_sum63(lsum[q]);
+        if (lane == 63) atomicAdd(S.light + q, t);
       }
     }
     __syncthreads();
   }
 
   // phase 4: this workgroup's partial row
+  __syncthreads();
   write_partial(F, L, S.light, S.vtab, S.stab, partial + (size_t)blockIdx.x * F.P, tid,
                 kBwdBlock);
 }
@@ -759,23 +933,6 @@ constexpr int kFlatBlock = 320;
 constexpr int kFlatPix = kFlatBlock - 64;
 constexpr int kMaxFlatGrid = 2048;
 constexpr int kMaxFlatTtab = 2048;  // triangles of the first-vertex table (32 KiB)
-
-// Sum of v over the 64 lanes, in lane 63 (every lane active): row-wise
-// inclusive scans by row shifts 1, 2, 4, 8, then row broadcasts of lanes 15
-// and 31; lanes without a source add 0.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_src(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ float wave_sum63(float v) {
-  v += dpp_src<0x111, 0xf>(v);  // row_shr:1
-  v += dpp_src<0x112, 0xf>(v);  // row_shr:2
-  v += dpp_src<0x114, 0xf>(v);  // row_shr:4
-  v += dpp_src<0x118, 0xf>(v);  // row_shr:8
-  v += dpp_src<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-  v += dpp_src<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
 
 // Waves 1-4: the runs of one scene into acc[cap][4] (sums of g_c per slot).
 // A run is 16 pixels down one column; run r covers column r % W of the band
@@ -913,17 +1070,6 @@ __device__ __forceinline__ FlatLds flat_lds(const BwdFrame& F, unsigned char* sm
   return S;
 }
 
-// Float atomic add through a global-address-space pointer (a generic
-// pointer would take the flat atomic's shared / private aperture checks).
-typedef __attribute__((address_space(1))) float global_float;
-typedef __attribute__((address_space(1))) const float global_cfloat;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) const f32x4 global_cfloat4;
-typedef __attribute__((address_space(1))) const int32_t global_cint;
-__device__ __forceinline__ void global_add(float* p, float v) {
-  __hip_atomic_fetch_add((global_float*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -996,13 +1142,13 @@ __device__ __forceinline__ void flat_chain(const pbr_scene_desc& D, const BwdFra
     normalize3(u, nw);
     // every term is linear in the summed output gradient
     const float gs[4] = {sum.x, sum.y, sum.z, sum.w};
-    float tacc[kAcc];
+    float tacc[kTerms];
 #pragma unroll
-    for (int q = 0; q < kAcc; ++q) tacc[q] = 0.0f;
+    for (int q = 0; q < kTerms; ++q) tacc[q] = 0.0f;
     float gn[3];
     shade_back(nw, rgba, gs, F.C, L, tacc, gn);
     // instance colour
-    const float gc[4] = {tacc[A_COL], tacc[A_COL + 1], tacc[A_COL + 2], tacc[A_ALPHA]};
+    const float gc[4] = {tacc[T_COL], tacc[T_COL + 1], tacc[T_COL + 2], tacc[T_ALPHA]};
     if (nd.shared && nd.soff >= 0) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) lds_add(S.stab + (size_t)(nd.soff + (int)row) * 4 + c, gc[c]);
@@ -1012,7 +1158,7 @@ __device__ __forceinline__ void flat_chain(const pbr_scene_desc& D, const BwdFra
         if (gc[c] != 0.0f) global_add(nd.gcol + row * 4 + c, gc[c]);
     }
 #pragma unroll
-    for (int q = 0; q < kLightF; ++q) S.glane[q * 64 + lane] += tacc[A_GL + q];
+    for (int q = 0; q < kLightF; ++q) S.glane[q * 64 + lane] += tacc[T_GL + q];
     // the first vertex's normal, through both normalisations
     float gu[3];
     normalize_back(nw, len3(u), gn, gu);
@@ -1230,12 +1376,14 @@ int plan_backward(const pbr_scene_desc* D, int channels, const pbr_grads* g, Bwd
                              PBR_MAX_NODES + kLightF * 64 + (size_t)F.vtab * 6 +
                              (size_t)F.stab * 4);
   }
-  else
-    P.lds = sizeof(float) * (size_t)F.cap * (kRecF + kAcc) +
-            sizeof(uint32_t) * (size_t)F.cap * 2 + sizeof(uint32_t) * (size_t)F.nwords * 2 +
+  else {
+    P.lds = sizeof(float) * (size_t)F.cap * (any_smooth(D) ? kAcc : kAccFlat) +
+            sizeof(uint32_t) * (size_t)F.cap + sizeof(uint32_t) * (size_t)F.nwords * 2 +
             sizeof(float) * 16 + sizeof(float) * (size_t)F.vtab * 6 +
             sizeof(float) * (size_t)F.stab * 4 + sizeof(uint32_t) * (PBR_MAX_NODES + 1) +
-            sizeof(uint32_t) * (kBwdBlock + 1);
+            sizeof(uint32_t) * (kBwdBlock / 64) + sizeof(BNode) * PBR_MAX_NODES +
+            sizeof(uint32_t) * (size_t)F.cap * 2 + sizeof(uint16_t) * kSortPixels;
+  }
   // one partial row per workgroup: per (scene, band), or per persistent flat
   // workgroup
   P.rows = P.flat ? min(D->num_scenes, kMaxFlatGrid) : D->num_scenes * F.bands;
@@ -1280,6 +1428,33 @@ hipError_t launch_flat_t(const pbr_scene_desc* D, const BwdPlan& P, const BwdLig
   hipLaunchKernelGGL(k, dim3(*grid), dim3(kFlatBlock), P.lds, st, *D, P.F, L, G, vis, gout,
                      partial);
   return hipGetLastError();
+}
+
+template <bool SMOOTH, int NC>
+hipError_t launch_bands_t(const pbr_scene_desc* D, const BwdPlan& P, const BwdLight& L,
+                          const BwdGrads& G, const int32_t* vis, const float* gout, float* partial,
+                          int grid, hipStream_t st) {
+  auto k = backward_kernel<SMOOTH, NC>;
+  if (P.lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kBwdBlock), P.lds, st, *D, P.F, L, G, vis, gout,
+                     partial);
+  return hipGetLastError();
+}
+
+template <bool SMOOTH>
+hipError_t launch_bands_nc(const pbr_scene_desc* D, const BwdPlan& P, const BwdLight& L,
+                           const BwdGrads& G, const int32_t* vis, const float* gout,
+                           float* partial, int channels, int grid, hipStream_t st) {
+  switch (channels) {
+    case 1: return launch_bands_t<SMOOTH, 1>(D, P, L, G, vis, gout, partial, grid, st);
+    case 2: return launch_bands_t<SMOOTH, 2>(D, P, L, G, vis, gout, partial, grid, st);
+    case 3: return launch_bands_t<SMOOTH, 3>(D, P, L, G, vis, gout, partial, grid, st);
+    default: return launch_bands_t<SMOOTH, 4>(D, P, L, G, vis, gout, partial, grid, st);
+  }
 }
 
 int launch_reduce(const pbr_scene_desc* D, const BwdPlan& P, const BwdGrads& G, int rows,
@@ -1382,23 +1557,13 @@ int pbr_render_backward(const pbr_scene_desc* scene, const int32_t* vis, const f
       return fail(PBR_ERR_LAUNCH, "backward launch failed: %s", hipGetErrorString(e));
     return launch_reduce(scene, P, G, grid, partial, st);
   }
-  const bool smooth = any_smooth(scene);
-  const void* kfn = smooth ? (const void*)backward_kernel<true> : (const void*)backward_kernel<false>;
-  if (P.lds > 64 * 1024) {
-    hipError_t e =
-        hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
-    if (e != hipSuccess)
-      return fail(PBR_ERR_LAUNCH, "backward LDS request failed: %s", hipGetErrorString(e));
-  }
   const uint64_t wgs = (uint64_t)scene->num_scenes * (uint64_t)P.F.bands;
   if (wgs >= 0x7fffffffull) return fail(PBR_ERR_INVALID, "too many backward workgroups");
-  if (smooth)
-    hipLaunchKernelGGL(backward_kernel<true>, dim3((uint32_t)wgs), dim3(kBwdBlock), P.lds, st,
-                       *scene, P.F, L, G, vis, grad_color, partial);
+  hipError_t e;
+  if (any_smooth(scene))
+    e = launch_bands_nc<true>(scene, P, L, G, vis, grad_color, partial, channels, (int)wgs, st);
   else
-    hipLaunchKernelGGL(backward_kernel<false>, dim3((uint32_t)wgs), dim3(kBwdBlock), P.lds, st,
-                       *scene, P.F, L, G, vis, grad_color, partial);
-  hipError_t e = hipGetLastError();
+    e = launch_bands_nc<false>(scene, P, L, G, vis, grad_color, partial, channels, (int)wgs, st);
   if (e != hipSuccess) return fail(PBR_ERR_LAUNCH, "backward launch failed: %s", hipGetErrorString(e));
   return launch_reduce(scene, P, G, P.rows, partial, st);
 }

@@ -87,17 +87,9 @@ constexpr int kOutMask = 0x3f;
 // pixels stay below 2^30.
 constexpr int kIntExtent = 1 << 14;
 
-typedef const __attribute__((address_space(4))) float const_float;
 typedef const __attribute__((address_space(1))) float global_cfloat;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) f32x4 global_cfloat4;
-
-// Sixteen floats at a wave-uniform address, by scalar loads.
-__device__ __forceinline__ void load_mat4_uniform(const float* src, float M[16]) {
-  const_float* p = (const_float*)(uintptr_t)src;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) M[q] = p[q];
-}
 
 __device__ __forceinline__ void load_mat4_global(const float* src, float M[16]) {
   global_cfloat4* q = (global_cfloat4*)(uintptr_t)src;

@@ -459,6 +459,15 @@ __device__ __forceinline__ void load_mat4(const float* src, float M[16]) {
   M[12] = d.x; M[13] = d.y; M[14] = d.z; M[15] = d.w;
 }
 
+// Sixteen floats at a wave-uniform address that nothing in the launch writes,
+// by scalar loads.
+typedef const __attribute__((address_space(4))) float const_float;
+__device__ __forceinline__ void load_mat4_uniform(const float* src, float M[16]) {
+  const_float* p = (const_float*)(uintptr_t)src;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) M[q] = p[q];
+}
+
 // Exact edge functions e_k = A*Px + B*Py + C of a snapped triangle (edge k is
 // opposite vertex k); C carries the fill-rule bias so inside <=> e >= 0.
 __device__ __forceinline__ void edges_from_fixed(const int32_t X[3], const int32_t Y[3],
