@@ -1297,9 +1297,20 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb) {
   return x < y + nb && y < x + na;
 }
 
-// Flat scenes of at most 32 slots and 64 columns run the 32-record form.
-bool rows_small(const pbr_scene_desc* D) {
+// Flat scenes of at most 32 slots and 64 columns fit the 32-record form.
+bool rows_narrow(const pbr_scene_desc* D) {
   return !any_smooth(D) && max_slots(D) <= 32 && D->width <= 64;
+}
+
+// They run it when the batch fills the chip: its two waves per workgroup keep
+// a wave per scene busy.  Up to kWideScenes scenes the 64-record form's four waves per
+// workgroup are all resident at once (four workgroups on each of 256 CUs) and
+// each has half the rows to walk.  CartPole at 64 x 64, uint8, 32- / 64-record
+// form: 64 scenes 15.9 / 11.7 us, 1000 19.2 / 14.0, 2000 20.0 / 17.5, 2500
+// 22.7 / 25.2, 4096 25.9 / 31.0.
+constexpr int kWideScenes = 2048;
+bool rows_small(const pbr_scene_desc* D) {
+  return rows_narrow(D) && D->num_scenes > kWideScenes;
 }
 
 // Whether both scenes' vertex slots fit the LDS vertex table (the vertex
@@ -1355,8 +1366,10 @@ bool match_poses(const pbr_scene_desc* D, const pbr_pose_desc* poses, int32_t co
     ++t.count;
     if (t.rows > kFusedRows) return false;
   }
-  // one pose per wave: two in the 32-record form, four in the 64-record one
-  if (t.count > (rows_small(D) ? 2 : 4)) return false;
+  // one pose per wave: two where the 32-record form may run (whatever the
+  // scene count, so that a batch's size does not change its launches), four
+  // in the 64-record one
+  if (t.count > (rows_narrow(D) ? 2 : 4)) return false;
   for (int k = 0; k < t.count; ++k) {
     const pbr_pose_desc& p = t.d[k];
     const size_t rows = (size_t)p.rows;
