@@ -162,6 +162,30 @@ typedef struct pbr_pose_desc {
   pbr_pose_component x, y, z, h, p, r, s;
 } pbr_pose_desc;
 
+/* One steering step's inputs and outputs.  Scene i reads x and y (and, with
+ * at least 4 columns, the grace time in column 3) from row i of `state`;
+ * the grace time selects color_grace (> 0.5) or color_play.  The eye is
+ * (x, y, 0) + eye_offset; the view's rows are right, up and -fwd with the
+ * translations of camera.py:201-240, the view-projection proj * view. */
+typedef struct pbr_steering_batch {
+  const float* state;         /* [num_scenes][columns], any strides         */
+  int64_t row_stride;         /* in floats                                  */
+  int64_t col_stride;         /* in floats                                  */
+  int32_t num_scenes;
+  int32_t columns;            /* >= 2                                       */
+  const float* color_play;    /* [4]                                        */
+  const float* color_grace;   /* [4]                                        */
+  const float* eye_offset;    /* [3]                                        */
+  const float* right;         /* [num_scenes][3]                            */
+  const float* up;            /* [num_scenes][3]                            */
+  const float* fwd;           /* [num_scenes][3]                            */
+  const float* proj;          /* [4][4]                                     */
+  float* colors;              /* optional [num_scenes][4] written           */
+  float* eye;                 /* [num_scenes][3] written                    */
+  float* view;                /* [num_scenes][4][4] written                 */
+  float* view_proj;           /* [num_scenes][4][4] written                 */
+} pbr_steering_batch;
+
 /* Gradient outputs of pbr_render_backward.  Every pointer is optional (NULL:
  * that gradient is not wanted); the kernels ADD into the buffers, so the
  * caller zeroes them first (torch autograd convention). */
@@ -270,6 +294,13 @@ int pbr_cartpole_step(const pbr_cartpole_params* params, const pbr_cartpole_batc
  * (envs/cartpole/env.py:95-109 _sample_initial_state, :153-176 _reset). */
 int pbr_cartpole_reset(const pbr_cartpole_params* params, const pbr_cartpole_batch* batch,
                        void* stream);
+
+/* The state mapping of one steering step (envs/steering/renderer.py:222-271)
+ * in one launch: the `npose` (<= 8) pose descriptors as pbr_set_poses writes
+ * them, the player colours, the camera eyes and the view and view-projection
+ * matrices.  Every output is written whole; none may overlap an input. */
+int pbr_steering_step(const pbr_steering_batch* batch, const pbr_pose_desc* poses,
+                      int32_t npose, void* stream);
 
 /* The kernel family pbr_render runs for this batch and launch shape: one
  * of PBR_KERNEL_CHUNKED / _SCENE / _TILES / _ROWS (AUTO resolved) in

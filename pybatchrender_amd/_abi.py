@@ -125,6 +125,27 @@ class pbr_pose_desc(C.Structure):
     ]
 
 
+class pbr_steering_batch(C.Structure):
+    _fields_ = [
+        ("state", C.c_void_p),
+        ("row_stride", C.c_int64),
+        ("col_stride", C.c_int64),
+        ("num_scenes", C.c_int32),
+        ("columns", C.c_int32),
+        ("color_play", C.c_void_p),
+        ("color_grace", C.c_void_p),
+        ("eye_offset", C.c_void_p),
+        ("right", C.c_void_p),
+        ("up", C.c_void_p),
+        ("fwd", C.c_void_p),
+        ("proj", C.c_void_p),
+        ("colors", C.c_void_p),
+        ("eye", C.c_void_p),
+        ("view", C.c_void_p),
+        ("view_proj", C.c_void_p),
+    ]
+
+
 class pbr_grads(C.Structure):
     _fields_ = [
         ("colors", C.c_void_p * PBR_MAX_NODES),
@@ -200,6 +221,8 @@ def expected_layout() -> list[int]:
         pbr_cartpole_params.seed.offset,
         C.sizeof(pbr_cartpole_batch),
         pbr_cartpole_batch.num_scenes.offset,
+        C.sizeof(pbr_steering_batch),
+        pbr_steering_batch.view_proj.offset,
     ]
 
 
@@ -214,6 +237,7 @@ EXPORTS = (
     "pbr_render_posed",
     "pbr_cartpole_step",
     "pbr_cartpole_reset",
+    "pbr_steering_step",
     "pbr_workspace_bytes",
     "pbr_choose_kernel",
     "pbr_last_error",
@@ -279,6 +303,9 @@ def declare(lib: C.CDLL) -> C.CDLL:
     lib.pbr_cartpole_reset.argtypes = [C.POINTER(pbr_cartpole_params),
                                        C.POINTER(pbr_cartpole_batch), C.c_void_p]
     lib.pbr_cartpole_reset.restype = C.c_int
+    lib.pbr_steering_step.argtypes = [C.POINTER(pbr_steering_batch), C.POINTER(pbr_pose_desc),
+                                      C.c_int32, C.c_void_p]
+    lib.pbr_steering_step.restype = C.c_int
     lib.pbr_workspace_bytes.argtypes = [
         C.POINTER(pbr_scene_desc),
         C.POINTER(pbr_render_opts),

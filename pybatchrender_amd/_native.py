@@ -134,3 +134,11 @@ def cartpole_reset(params: _abi.pbr_cartpole_params, batch: _abi.pbr_cartpole_ba
                                       ctypes.c_void_p(stream_ptr or None))
     if rc != _abi.PBR_OK:
         raise RuntimeError(f"pbr_cartpole_reset failed (status {rc}): {last_error()}")
+
+
+def steering_step(batch: _abi.pbr_steering_batch, poses: list, stream_ptr: int) -> None:
+    arr = (_abi.pbr_pose_desc * max(len(poses), 1))(*poses)
+    rc = library().pbr_steering_step(ctypes.byref(batch), arr, len(poses),
+                                     ctypes.c_void_p(stream_ptr or None))
+    if rc != _abi.PBR_OK:
+        raise RuntimeError(f"pbr_steering_step failed (status {rc}): {last_error()}")

@@ -1173,6 +1173,8 @@ int pbr_abi_layout(int64_t* out, int32_t n) {
       (int64_t)offsetof(pbr_cartpole_params, seed),
       (int64_t)sizeof(pbr_cartpole_batch),
       (int64_t)offsetof(pbr_cartpole_batch, num_scenes),
+      (int64_t)sizeof(pbr_steering_batch),
+      (int64_t)offsetof(pbr_steering_batch, view_proj),
   };
   const int32_t total = (int32_t)(sizeof(facts) / sizeof(facts[0]));
   for (int32_t i = 0; i < n && i < total; ++i) out[i] = facts[i];

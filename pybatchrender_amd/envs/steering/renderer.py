@@ -22,8 +22,10 @@ from __future__ import annotations
 
 import torch
 
+from ... import _abi, _native
 from ...config import PBRConfig
 from ...renderer import mesh as meshmod
+from ...renderer.camera import PBRCam
 from ...renderer.renderer import PBRRenderer
 
 _FALLBACK = {"models/smiley": "models/sphere", "models/cone.egg": "models/cone",
@@ -38,6 +40,13 @@ def resolve_model(path: str):
         if path in _FALLBACK:
             return meshmod.load_model(_FALLBACK[path])
         raise
+
+
+def _plain(t, shape: tuple, device: torch.device) -> bool:
+    """Whether a kernel can use t in place: a contiguous float32 tensor of
+    this shape on this device that autograd does not follow."""
+    return (type(t) is torch.Tensor and t.dtype is torch.float32 and t.device == device
+            and tuple(t.shape) == shape and t.is_contiguous() and not t.requires_grad)
 
 
 class SteeringRenderer(PBRRenderer):
@@ -129,6 +138,57 @@ class SteeringRenderer(PBRRenderer):
         elif self._geometry is None:
             self._build_geometry()
 
+    def _step_device(self, st: torch.Tensor) -> bool:
+        """The state mapping of ``_step`` in one HIP launch (pbr_steering_step);
+        False, with nothing done, for what that launch does not take: the CPU,
+        poses recorded before it, a replaced camera, and tensors it cannot
+        read or write in place."""
+        cam = self._pbr_cam
+        n = self._num_scenes
+        if (self.device.type != "cuda" or type(cam) is not PBRCam or cam.num_scenes != n
+                or cam.device != self.device or self._pending_poses or n < 1 or st.shape[1] < 2):
+            return False
+        player = self.player_node
+        col = player.colors_b4 if player.has_geometry else None
+        P = cam._get_projection()
+        reads = (cam._right, cam._up, cam._fwd, P, self._camera_eye_offset, self._color_player,
+                 self._color_crash)
+        shapes = ((n, 3), (n, 3), (n, 3), (4, 4), (1, 3), (4,), (4,))
+        if not all(_plain(t, s, self.device) for t, s in zip(reads, shapes)):
+            return False
+        if col is not None and not _plain(col, (n, 4), self.device):
+            return False
+        if type(st) is not torch.Tensor or torch._C._are_functorch_transforms_active():
+            return False
+        half = float(self.cfg.lane_width) * 0.5
+        z = float(self.cfg.rail_offset[2])
+        px, py = st[:, 0], st[:, 1]
+        poses = [node._pose_inputs(**kw)
+                 for node, kw in ((player, dict(x=px, y=py)),
+                                  (self.left_border, dict(x=-half, y=py, z=z)),
+                                  (self.right_border, dict(x=half, y=py, z=z)))]
+        poses = [p for p in poses if p is not None]
+        # nothing that the launch writes may be what another thread reads
+        written = [t for node in (player, self.left_border, self.right_border) if node.has_geometry
+                   for t in (node.transforms_b44, node.rot3_b33, node.scale_b11, node.colors_b4)]
+        src = st.untyped_storage().data_ptr()
+        if any(t.untyped_storage().data_ptr() == src for t in written):
+            return False
+        eye = torch.empty((n, 3), dtype=torch.float32, device=self.device)
+        view = torch.empty((2, n, 4, 4), dtype=torch.float32, device=self.device)
+        b = _abi.pbr_steering_batch()
+        b.state, b.row_stride, b.col_stride = st.data_ptr(), st.stride(0), st.stride(1)
+        b.num_scenes, b.columns = n, st.shape[1]
+        b.right, b.up, b.fwd, b.proj, b.eye_offset, b.color_play, b.color_grace = (
+            t.data_ptr() for t in reads)
+        b.colors = col.data_ptr() if col is not None else None
+        b.eye, b.view, b.view_proj = eye.data_ptr(), view[0].data_ptr(), view[1].data_ptr()
+        _native.steering_step(b, [d for d, _ in poses], _native.stream_ptr(self.device))
+        if col is not None and not col.is_inference():
+            torch.autograd.graph.increment_version(col)
+        cam.P_k44, cam.eye_k3, cam.V_k44, cam.VP_k44 = P, eye, view[0], view[1]
+        return True
+
     def _step(self, state_batch: torch.Tensor | None = None) -> None:
         """Observation [B, >=4] -> player, rails, player colour, camera eye."""
         if state_batch is None:
@@ -141,6 +201,8 @@ class SteeringRenderer(PBRRenderer):
         if st.shape[0] < n:
             st = torch.cat([st, st[-1:].expand(n - st.shape[0], -1)], 0)
         st = st[:n]
+        if self._step_device(st):
+            return
         px, py = st[:, 0].contiguous(), st[:, 1].contiguous()
         half = float(self.cfg.lane_width) * 0.5
         z = float(self.cfg.rail_offset[2])

@@ -10,7 +10,8 @@ import torch
 
 from pybatchrender import PBRConfig, PBRRenderer, workloads
 from pybatchrender.envs.cartpole import CartPoleConfig, CartPoleGroundRenderer, CartPoleRenderer
-from tests.test_gpu_parity import check_parity, ground_states
+from pybatchrender.envs.steering import SteeringConfig, SteeringRenderer
+from tests.test_gpu_parity import _bits, check_parity, ground_states
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +66,51 @@ def test_posed_step_record_forms(cuda, n):
                                               tile_resolution=(33, 20)))
     pix = r.step(ground_states(n, 5).cuda())
     check_parity(r, f"posed step n={n}", depth=False, vis=False, got={"pixels": pix})
+
+
+def _steering(n: int, seed: int) -> SteeringRenderer:
+    g = torch.Generator("cpu").manual_seed(seed)
+    r = SteeringRenderer(SteeringConfig(num_scenes=n, device="cuda", tile_resolution=(24, 20)))
+    obs = torch.rand(n, 3, 4, generator=g) * torch.tensor([4.0, 30.0, 1.0, 1.0])
+    r.build_obstacles(obs.cuda())
+    fwd = torch.rand(n, 3, generator=g) - torch.tensor([0.5, -1.0, 0.5])
+    r._pbr_cam.set_forward(fwd.cuda())
+    return r
+
+
+def _scene_bits(r: SteeringRenderer, pix: torch.Tensor) -> list[torch.Tensor]:
+    cam = r._pbr_cam
+    out = [pix, cam.eye_k3, cam.V_k44, cam.VP_k44]
+    for nd in (r.player_node, r.left_border, r.right_border):
+        out += [nd.transforms_b44, nd.rot3_b33, nd.scale_b11, nd.colors_b4]
+    return [_bits(t) for t in out]
+
+
+@pytest.mark.parametrize("cols", [2, 4, 7])
+@pytest.mark.parametrize("n", [1, 3, 64, 65, 257])
+def test_steering_step_launch_matches_tensor_operations(cuda, n, cols):
+    """Every tensor the one-launch steering step writes, and its frame,
+    against the same step by tensor operations: each layout of the state
+    that is read in place, states with fewer rows, on the host, of another
+    type, and in a scene's own buffer."""
+    g = torch.Generator("cpu").manual_seed(100 * n + cols)
+    a, b = _steering(n, 7), _steering(n, 7)
+    b._step_device = lambda st: False
+    base = torch.rand(n, cols, generator=g) * torch.tensor([3.0, 90.0] + [1.0] * (cols - 2))
+    base[:: 3, 0] = -0.0
+    dev = base.cuda()
+    wide = torch.zeros(n, 2 * cols, device="cuda")
+    wide[:, ::2] = dev
+    for what, st in (("contiguous", dev), ("transposed", dev.t().contiguous().t()),
+                     ("every second", wide[:, ::2]), ("host", base), ("double", dev.double()),
+                     ("half the rows", dev[: (n + 1) // 2]), ("row", dev[0])):
+        same = [x.equal(y) for x, y in zip(_scene_bits(a, a.step(st)), _scene_bits(b, b.step(st)))]
+        assert all(same), f"n={n} cols={cols} {what}: {same}"
+    if cols == 4:
+        for r in (a, b):
+            r.player_node.colors_b4.copy_(dev)
+        same = [x.equal(y) for x, y in zip(_scene_bits(a, a.step(a.player_node.colors_b4)),
+                                           _scene_bits(b, b.step(b.player_node.colors_b4)))]
+        assert all(same), f"n={n}, state in the colour buffer: {same}"
+    check_parity(a, f"steering n={n}", depth=False, vis=False,
+                 got={"pixels": a.step(dev)})
