@@ -186,6 +186,13 @@ typedef struct pbr_steering_batch {
   float* view_proj;           /* [num_scenes][4][4] written                 */
 } pbr_steering_batch;
 
+/* One buffer of pbr_copy_segments. */
+typedef struct pbr_segment {
+  void* dst;
+  const void* src;            /* NULL: dst is cleared                       */
+  int64_t bytes;
+} pbr_segment;
+
 /* Gradient outputs of pbr_render_backward.  Every pointer is optional (NULL:
  * that gradient is not wanted); the kernels ADD into the buffers, so the
  * caller zeroes them first (torch autograd convention). */
@@ -336,6 +343,13 @@ int pbr_render_backward(const pbr_scene_desc* scene, const int32_t* vis,
  * reference). */
 int pbr_backward_workspace_bytes(const pbr_scene_desc* scene, int32_t channels,
                                  const pbr_grads* grads, size_t* bytes);
+
+/* Copies (src non-NULL) or clears (src NULL) `count` (<= 32) buffers of
+ * floats in one launch on `stream`.  Every pointer is 4-byte aligned and
+ * every size a multiple of 4; no dst may overlap another segment.  No
+ * counterpart in the reference; the differentiable render snapshots its
+ * inputs and clears its gradients with it. */
+int pbr_copy_segments(const pbr_segment* segments, int32_t count, void* stream);
 
 /* Thread-local message of the last failed call ("" if none).
  * Replaces the reference's swallowed exceptions (renderer.py:340-350). */

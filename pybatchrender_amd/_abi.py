@@ -146,6 +146,14 @@ class pbr_steering_batch(C.Structure):
     ]
 
 
+class pbr_segment(C.Structure):
+    _fields_ = [
+        ("dst", C.c_void_p),
+        ("src", C.c_void_p),
+        ("bytes", C.c_int64),
+    ]
+
+
 class pbr_grads(C.Structure):
     _fields_ = [
         ("colors", C.c_void_p * PBR_MAX_NODES),
@@ -223,6 +231,7 @@ def expected_layout() -> list[int]:
         pbr_cartpole_batch.num_scenes.offset,
         C.sizeof(pbr_steering_batch),
         pbr_steering_batch.view_proj.offset,
+        C.sizeof(pbr_segment),
     ]
 
 
@@ -238,6 +247,7 @@ EXPORTS = (
     "pbr_cartpole_step",
     "pbr_cartpole_reset",
     "pbr_steering_step",
+    "pbr_copy_segments",
     "pbr_workspace_bytes",
     "pbr_choose_kernel",
     "pbr_last_error",
@@ -306,6 +316,8 @@ def declare(lib: C.CDLL) -> C.CDLL:
     lib.pbr_steering_step.argtypes = [C.POINTER(pbr_steering_batch), C.POINTER(pbr_pose_desc),
                                       C.c_int32, C.c_void_p]
     lib.pbr_steering_step.restype = C.c_int
+    lib.pbr_copy_segments.argtypes = [C.POINTER(pbr_segment), C.c_int32, C.c_void_p]
+    lib.pbr_copy_segments.restype = C.c_int
     lib.pbr_workspace_bytes.argtypes = [
         C.POINTER(pbr_scene_desc),
         C.POINTER(pbr_render_opts),

@@ -142,3 +142,12 @@ def steering_step(batch: _abi.pbr_steering_batch, poses: list, stream_ptr: int) 
                                      ctypes.c_void_p(stream_ptr or None))
     if rc != _abi.PBR_OK:
         raise RuntimeError(f"pbr_steering_step failed (status {rc}): {last_error()}")
+
+
+def copy_segments(segments: list, stream_ptr: int) -> None:
+    """One launch that copies (dst, src, bytes) or, with src 0, clears
+    (dst, 0, bytes) every buffer of floats in the list."""
+    arr = (_abi.pbr_segment * max(len(segments), 1))(*segments)
+    rc = library().pbr_copy_segments(arr, len(segments), ctypes.c_void_p(stream_ptr or None))
+    if rc != _abi.PBR_OK:
+        raise RuntimeError(f"pbr_copy_segments failed (status {rc}): {last_error()}")

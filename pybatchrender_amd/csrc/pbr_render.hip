@@ -763,6 +763,30 @@ __global__ __launch_bounds__(256) void pose_kernel(PoseBatch B) {
   write_pose(P, i);
 }
 
+// Copies or clears one segment per blockIdx.y.  Bound by its launch at the
+// sizes it is used for (a few MB): one launch for up to 32 buffers in place
+// of a tensor operation for each.  16 bytes a thread where both ends allow.
+constexpr int kMaxSegments = 32;
+struct SegmentList {
+  pbr_segment s[kMaxSegments];
+};
+
+__global__ __launch_bounds__(256) void copy_segments_kernel(SegmentList L) {
+  const pbr_segment S = L.s[blockIdx.y];
+  const uint64_t t0 = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
+  const uint64_t words = (uint64_t)S.bytes / 4;
+  uint32_t* dst = reinterpret_cast<uint32_t*>(S.dst);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(S.src);
+  uint64_t quads = 0;
+  if ((((uintptr_t)S.dst | (uintptr_t)S.src) & 15) == 0) {
+    quads = words / 4;
+    for (uint64_t i = t0; i < quads; i += step)
+      reinterpret_cast<uint4*>(dst)[i] =
+          src ? reinterpret_cast<const uint4*>(src)[i] : make_uint4(0u, 0u, 0u, 0u);
+  }
+  for (uint64_t i = quads * 4 + t0; i < words; i += step) dst[i] = src ? src[i] : 0u;
+}
+
 // Resets the persistent queue head inside the stream order (graph-safe: a
 // kernel, not a memset node).
 __global__ void reset_queue_kernel(uint32_t* q) { *q = 0u; }
@@ -1175,10 +1199,39 @@ int pbr_abi_layout(int64_t* out, int32_t n) {
       (int64_t)offsetof(pbr_cartpole_batch, num_scenes),
       (int64_t)sizeof(pbr_steering_batch),
       (int64_t)offsetof(pbr_steering_batch, view_proj),
+      (int64_t)sizeof(pbr_segment),
   };
   const int32_t total = (int32_t)(sizeof(facts) / sizeof(facts[0]));
   for (int32_t i = 0; i < n && i < total; ++i) out[i] = facts[i];
   return total;
+}
+
+int pbr_copy_segments(const pbr_segment* segments, int32_t count, void* stream) {
+  if (count < 0 || count > kMaxSegments)
+    return fail(PBR_ERR_INVALID, "segment count %d outside [0, %d]", count, kMaxSegments);
+  if (count > 0 && !segments) return fail(PBR_ERR_INVALID, "null segments");
+  SegmentList L;
+  memset(&L, 0, sizeof(L));
+  int n = 0;
+  int64_t most = 0;
+  for (int k = 0; k < count; ++k) {
+    const pbr_segment& g = segments[k];
+    if (g.bytes < 0 || (g.bytes & 3)) return fail(PBR_ERR_INVALID, "segment %d: size not a multiple of 4", k);
+    if (g.bytes == 0) continue;
+    if (!g.dst || (((uintptr_t)g.dst | (uintptr_t)g.src) & 3))
+      return fail(PBR_ERR_INVALID, "segment %d: pointers must be 4-byte aligned", k);
+    L.s[n++] = g;
+    most = g.bytes > most ? g.bytes : most;
+  }
+  g_err[0] = 0;
+  if (n == 0) return PBR_OK;
+  // four 16-byte pieces a thread, at most eight blocks per CU for one segment
+  const int64_t blocks = (most + 256 * 64 - 1) / (256 * 64);
+  const int grid = (int)(blocks < 2048 ? blocks : 2048);
+  hipLaunchKernelGGL(copy_segments_kernel, dim3(grid, n), dim3(256), 0, (hipStream_t)stream, L);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(PBR_ERR_LAUNCH, "launch failed: %s", hipGetErrorString(e));
+  return PBR_OK;
 }
 
 int pbr_set_poses(const pbr_pose_desc* poses, int32_t count, void* stream) {

@@ -31,6 +31,7 @@ keeps a copy of both for its backward.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -75,7 +76,7 @@ def scene_params(renderer, requires_grad: bool = True) -> SceneParams:
     return out
 
 
-def _descriptor(renderer, vertices, light, colors):
+def _live_descriptor(renderer, vertices, light, colors):
     desc, keep = renderer.scene_descriptor()
     g = renderer._geometry
     if vertices.shape != g["vertices"].shape or vertices.dtype != torch.float32:
@@ -101,14 +102,40 @@ def _descriptor(renderer, vertices, light, colors):
     desc.light_col[:] = lv[3:6]
     desc.ambient[:] = lv[6:9]
     desc.strength = lv[9]
-    # transforms and view-projection are read again by the backward: freeze them
-    for j in range(desc.num_nodes):
-        tr = g["nodes"][j].transforms_b44.detach().to(torch.float32).contiguous().clone()
-        desc.nodes[j].transforms = tr.data_ptr()
-        keep.append(tr)
-    vp = renderer._pbr_cam.VP_k44.detach().to(torch.float32).reshape(-1, 4, 4).contiguous().clone()
-    desc.view_proj = vp.data_ptr()
-    keep.append(vp)
+    return desc, keep
+
+
+def _freeze(renderer, desc, keep) -> None:
+    """Points the descriptor at copies of its transforms and view-projection
+    (the backward reads them again): on the GPU one buffer and one launch
+    for all of them."""
+    nodes = [desc.nodes[j] for j in range(desc.num_nodes)]
+    N = desc.num_scenes
+    src = [nd.transforms for nd in nodes] + [desc.view_proj]
+    size = [(1 if nd.shared else N) * nd.instances_per_scene * 16 for nd in nodes] + [N * 16]
+    start = [0]
+    for n in size:
+        start.append(start[-1] + (n + 63) // 64 * 64)
+    buf = torch.empty(start[-1], dtype=torch.float32, device=renderer.device)
+    base = buf.data_ptr()
+    dst = [base + 4 * o for o in start]
+    if renderer.device.type == "cuda":
+        _native.copy_segments([(d, p, 4 * n) for d, p, n in zip(dst, src, size)],
+                              _native.stream_ptr(renderer.device))
+    else:
+        for d, p, n in zip(dst, src, size):
+            ctypes.memmove(d, p, 4 * n)
+    for nd, d in zip(nodes, dst):
+        nd.transforms = d
+    desc.view_proj = dst[-2]
+    keep.append(buf)
+
+
+def _descriptor(renderer, vertices, light, colors):
+    """The scene descriptor with the parameters substituted and its
+    transforms and view-projection frozen, and the tensors it points to."""
+    desc, keep = _live_descriptor(renderer, vertices, light, colors)
+    _freeze(renderer, desc, keep)
     return desc, keep
 
 
@@ -117,18 +144,25 @@ class _DiffRender(torch.autograd.Function):
     def forward(ctx, renderer, vertices, light, *colors):
         if renderer.device.type != "cuda":
             raise RuntimeError("differentiable rendering needs the HIP renderer on a GPU device")
-        desc, keep = _descriptor(renderer, vertices, light, colors)
+        desc, keep = _live_descriptor(renderer, vertices, light, colors)
+        # the render reads aligned instance rows; others through the copies
+        aligned = not any(p & 15 for p in [desc.view_proj or 0] +
+                          [desc.nodes[j].transforms or 0 for j in range(desc.num_nodes)])
+        if not aligned:
+            _freeze(renderer, desc, keep)
         N, C, H, W = renderer.output_shape()
         out = torch.empty((N, C, H, W), dtype=torch.float32, device=renderer.device)
         vis = torch.empty((N, H, W), dtype=torch.int32, device=renderer.device)
         fo = _abi.pbr_frame_out()
         fo.color, fo.depth, fo.vis = out.data_ptr(), None, vis.data_ptr()
         fo.channels, fo.dtype = C, _abi.PBR_DTYPE_F32
-        opts = renderer.render_opts()
+        opts = renderer._cached_opts()
         ws_bytes = _native.workspace_bytes(desc, opts)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=renderer.device)
-        stream = torch.cuda.current_stream(renderer.device).cuda_stream
+        stream = _native.stream_ptr(renderer.device)
         _native.render(desc, fo, opts, ws.data_ptr() if ws_bytes else 0, ws_bytes, stream)
+        if aligned:  # behind the frame on the stream: the host gets there while it draws
+            _freeze(renderer, desc, keep)
         ctx.desc, ctx.keep, ctx.vis = desc, keep + [ws], vis
         ctx.shapes = (C, [c.shape for c in colors], vertices.shape, light.device)
         ctx.mark_non_differentiable(vis)
@@ -141,10 +175,13 @@ class _DiffRender(torch.autograd.Function):
         dev = ctx.vis.device
         need = ctx.needs_input_grad
         g = _abi.pbr_grads()
-        g_verts = torch.zeros(vshape, dtype=torch.float32, device=dev) if need[1] else None
-        g_light = torch.zeros(10, dtype=torch.float32, device=dev) if need[2] else None
-        g_cols = [torch.zeros(s, dtype=torch.float32, device=dev) if need[3 + j] else None
+        g_verts = torch.empty(vshape, dtype=torch.float32, device=dev) if need[1] else None
+        g_light = torch.empty(10, dtype=torch.float32, device=dev) if need[2] else None
+        g_cols = [torch.empty(s, dtype=torch.float32, device=dev) if need[3 + j] else None
                   for j, s in enumerate(col_shapes)]
+        stream = _native.stream_ptr(dev)
+        _native.copy_segments([(t.data_ptr(), None, 4 * t.numel())
+                               for t in (g_verts, g_light, *g_cols) if t is not None], stream)
         if g_verts is not None:
             g.vertices = g_verts.data_ptr()
         if g_light is not None:
@@ -155,7 +192,6 @@ class _DiffRender(torch.autograd.Function):
         gout = grad_out.detach().to(torch.float32).contiguous()
         ws_bytes = _native.backward_workspace_bytes(desc, C, g)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        stream = torch.cuda.current_stream(dev).cuda_stream
         _native.render_backward(desc, ctx.vis.data_ptr(), gout.data_ptr(), C, g,
                                 ws.data_ptr() if ws_bytes else 0, ws_bytes, stream)
         if g_light is not None:

@@ -8,7 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from pybatchrender import PBRConfig, PBRRenderer, workloads
+from pybatchrender import PBRConfig, PBRRenderer, _native, diff, workloads
 from pybatchrender.envs.cartpole import CartPoleConfig, CartPoleGroundRenderer, CartPoleRenderer
 from pybatchrender.envs.steering import SteeringConfig, SteeringRenderer
 from tests.test_gpu_parity import _bits, check_parity, ground_states
@@ -114,3 +114,62 @@ def test_steering_step_launch_matches_tensor_operations(cuda, n, cols):
         assert all(same), f"n={n}, state in the colour buffer: {same}"
     check_parity(a, f"steering n={n}", depth=False, vis=False,
                  got={"pixels": a.step(dev)})
+
+
+@pytest.mark.parametrize("shift_dst,shift_src", [(0, 0), (0, 1), (3, 0), (2, 2)])
+def test_copy_segments(cuda, shift_dst, shift_src):
+    """Copies and clears of 0 .. 70001 floats at aligned and odd addresses,
+    and nothing written beside them."""
+    sizes = [0, 1, 3, 4, 5, 255, 4096, 70001, 17]
+    src = [torch.randn(n + shift_src + 8, device="cuda") for n in sizes]
+    dst = [torch.full((n + shift_dst + 8,), 7.0, device="cuda") for n in sizes]
+    want = [t.clone() for t in dst]
+    segs = []
+    for k, n in enumerate(sizes):
+        clear = k % 3 == 1
+        segs.append((dst[k].data_ptr() + 4 * shift_dst,
+                     None if clear else src[k].data_ptr() + 4 * shift_src, 4 * n))
+        want[k][shift_dst:shift_dst + n] = 0.0 if clear else src[k][shift_src:shift_src + n]
+    _native.copy_segments(segs, _native.stream_ptr(src[0].device))
+    for k, n in enumerate(sizes):
+        assert torch.equal(dst[k], want[k]), f"segment {k} of {n} floats"
+    with pytest.raises(RuntimeError, match="aligned"):
+        _native.copy_segments([(dst[3].data_ptr() + 2, None, 4)], 0)
+
+
+def test_gradients_from_unaligned_transforms(cuda):
+    """Instance rows at an address that is no multiple of 16 are rendered
+    through the copies the backward reads."""
+    n = 9
+    gen = torch.Generator("cpu").manual_seed(3)
+    r = PBRRenderer(PBRConfig(num_scenes=n, tile_resolution=(33, 20), device="cuda",
+                              output_dtype="float32"))
+    node = r.add_node("models/sphere", instances_per_scene=2)
+    node.set_transforms(workloads.random_transforms(n * 2, gen, pos_range=1.0))
+    node.set_colors(torch.rand(n * 2, 4, generator=gen))
+    r.add_camera().set_positions_and_lookat(torch.tensor([0.0, -5.0, 1.0]), torch.zeros(3))
+    r.add_light()
+    r.setup_environment()
+    gout = torch.randn(n, 3, 20, 33, generator=gen).cuda()
+
+    def gradients():
+        p = diff.scene_params(r)
+        img = diff.render(r, p)
+        # what the backward reads is frozen with the frame
+        moved = node.transforms_b44
+        saved = moved.clone()
+        moved.zero_()
+        grads = torch.autograd.grad(img, p.tensors(), gout)
+        moved.copy_(saved)
+        return [img.detach()] + [g.cpu() for g in grads]
+
+    want = gradients()
+    odd = torch.empty(node.transforms_b44.numel() + 1, device="cuda")[1:]
+    odd = odd.reshape(node.transforms_b44.shape)
+    odd.copy_(node.transforms_b44)
+    node.transforms_b44 = odd
+    got = gradients()
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        # sums of float atomics in any order: a few hundred terms of 2^-24 each
+        assert (a - b).abs().max() <= 2e-5 * b.abs().max() + 1e-30
