@@ -77,9 +77,20 @@ struct NodeLds {
   uint32_t flags;         // bit 0: shared, bit 1: flat
 };
 
-// Vertex table entry: X << 6 | outcode, Y << 1 | not snapped.  |X|, |Y| <=
-// 2^24 (snap_vertex), so both shifts fit 32 bits.
-constexpr int kOutMask = 0x3f;
+// A vertex table entry is the snapped position and the depth's bits.  A vertex
+// that is outside a clip plane or did not snap (in a chunk that holds one) has
+// this NaN | kNotSnapped | its outcode for the depth, which is finite in every
+// other: a vertex inside the planes has a depth of 0 to 1.
+constexpr uint32_t kCodeTag = 0xffc00000u;
+constexpr uint32_t kOutMask = 0x3fu, kNotSnapped = 0x40u;
+__device__ __forceinline__ uint32_t vertex_code(uint32_t d) {
+  return d >= kCodeTag ? d & (kOutMask | kNotSnapped) : 0u;
+}
+
+// Lanes of m below this one.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
 
 // Snapped extents (1/256 pixel) up to which edge values are evaluated in 32
 // bits: coordinate differences are at most 2^14, their products 2^28, and
@@ -244,30 +255,30 @@ __device__ __forceinline__ void band_raster_rows(unsigned long long* pix, const 
   }
 }
 
-// The whole wave, in blocks of 8 x 8 pixels.  Every argument is uniform.
-template <typename Num>
+// The whole wave, in blocks of 8 x 8 pixels, edge values in double.  Every
+// argument is uniform.
 __device__ __forceinline__ void band_raster_wave(unsigned long long* pix, const BandCtx& t,
                                                  int lane, const FixTri& T, uint32_t rank) {
-  BandEdges<Num> E;
+  BandEdges<double> E;
   band_edges(T, T.i0, T.j0, E);
   const int li = lane & 7, lj = lane >> 3;
-  Num row[3];
+  double row[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) row[k] = E.e[k] + E.A[k] * (Num)li + E.B[k] * (Num)lj;
+  for (int k = 0; k < 3; ++k) row[k] = E.e[k] + E.A[k] * (double)li + E.B[k] * (double)lj;
   for (int jb = T.j0; jb <= T.j1; jb += 8) {
     const int j = jb + lj;
     const float tz = fmaf(T.zy, (float)j + 0.5f, T.zc);
     unsigned long long* q = pix + (t.j1 - j) * t.W + T.i0 + li;
-    Num e[3] = {row[0], row[1], row[2]};
+    double e[3] = {row[0], row[1], row[2]};
     for (int ib = T.i0; ib <= T.i1; ib += 8, q += 8) {
       const int i = ib + li;
       if (i <= T.i1 && j <= T.j1 && band_inside(e))
         band_fragment(q, clamp_depth(fmaf(T.zx, (float)i + 0.5f, tz)), rank);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) e[k] += E.A[k] * (Num)8;
+      for (int k = 0; k < 3; ++k) e[k] += E.A[k] * (double)8;
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) row[k] += E.B[k] * (Num)8;
+    for (int k = 0; k < 3; ++k) row[k] += E.B[k] * (double)8;
   }
 }
 
@@ -600,7 +611,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   int2* tables = reinterpret_cast<int2*>(pix + ((F.th * W + 1) & ~1));
   int2* vxy = tables + wave * F.verts;
   unsigned char* after = reinterpret_cast<unsigned char*>(tables + kBandWaves * F.verts);
-  float* vd = reinterpret_cast<float*>(after) + wave * F.verts;
+  uint32_t* vd = reinterpret_cast<uint32_t*>(after) + wave * F.verts;
   after += sizeof(float) * (size_t)kBandWaves * F.verts;
   uint8_t* qu = after + wave * kBandTris;
   uint32_t* tab = reinterpret_cast<uint32_t*>(after + kBandWaves * kBandTris);
@@ -664,9 +675,6 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
 
   // --- setup and raster --------------------------------------------------------
   const uint32_t chunks = __builtin_amdgcn_readfirstlane((int)total_chunks);
-  // pixel-centre limits in 1/256 pixel: a chunk wholly below / above / left /
-  // right of them touches no pixel centre of the band
-  const int ylo = 256 * t.j0 + 128, yhi = 256 * t.j1 + 128, xhi = 256 * (W - 1) + 128;
   for (;;) {
     uint32_t c = 0;
     if (lane == 0) c = atomicAdd(&next_chunk, 1u);
@@ -693,23 +701,45 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     const uint32_t n = min(g * nt, ndraw - slot0);
     const size_t row0 = nd.shared ? (size_t)i0 : (size_t)t.s * (size_t)nd.instances_per_scene + i0;
 
-    // vertices of the chunk into the wave's table; `out` gathers what all of
-    // them lie outside of (bits 0-5 clip planes, 6-9 the band's sides)
-    uint32_t out = 0x3ffu;
+    // vertices of the chunk into the wave's table.  `dirty`: some vertex is
+    // outside a clip plane or did not snap; only then are outcodes made
+    // (`out`: the planes that all vertices lie outside of) and tested.
+    bool dirty = false;
+    uint32_t out = kOutMask;
+    constexpr int kFar = 1 << 28;
+    int xmin = kFar, xmax = -kFar, ymin = kFar, ymax = -kFar;
     auto vertex = [&](uint32_t v, uint32_t k, const float* M) {
       float vv[6];
       load_vertex(D.vertices, voff + (int)k, vv);
       CVert cv;
       transform_vertex(M, VP, vv, cv);
-      SnapVert r;
-      snap_vertex(cv, W, H, r);
-      const uint32_t oc = outcode(cv, F.guard);
-      vxy[v] = make_int2((int)(((uint32_t)r.X << 6) | oc),
-                         (int)(((uint32_t)r.Y << 1) | (r.ok ? 0u : 1u)));
-      vd[v] = r.d;
-      const uint32_t side = (r.Y < ylo ? 64u : 0u) | (r.Y > yhi ? 128u : 0u) |
-                            (r.X < 128 ? 256u : 0u) | (r.X > xhi ? 512u : 0u);
-      out &= oc | (oc == 0u && r.ok ? side : 0u);
+      // plane_dist is >= 0 on both sides of an axis just when this is (a sum's
+      // sign is exact, and NaN fails in both)
+      const float w = cv.p[3], gw = F.guard * w;
+      const bool in = w - fabsf(cv.p[2]) >= 0.0f && gw - fabsf(cv.p[0]) >= 0.0f &&
+                      gw - fabsf(cv.p[1]) >= 0.0f;
+      // snap_vertex without its early returns
+      const float iw = 1.0f / w;
+      const float nx = cv.p[0] * iw, ny = cv.p[1] * iw, nz = cv.p[2] * iw;
+      const float sx = (nx + 1.0f) * (0.5f * (float)W), sy = (ny + 1.0f) * (0.5f * (float)H);
+      const bool ok = w > 0.0f && fabsf(sx) < 65536.0f && fabsf(sy) < 65536.0f;
+      int X = (int)rintf(sx * 256.0f), Y = (int)rintf(sy * 256.0f);
+      uint32_t d = __float_as_uint(nz * 0.5f + 0.5f), oc = 0u;
+      if (__ballot(!(in && ok))) {
+        dirty = true;
+        oc = outcode(cv, F.guard);
+        const uint32_t code = oc | (ok ? 0u : kNotSnapped);
+        if (code) d = kCodeTag | code;
+        X = ok ? X : 0;
+        Y = ok ? Y : 0;
+      }
+      out &= oc;
+      vxy[v] = make_int2(X, Y);
+      vd[v] = d;
+      xmin = min(xmin, X);
+      xmax = max(xmax, X);
+      ymin = min(ymin, Y);
+      ymax = max(ymax, Y);
     };
     if (group == 1u) {
       float M[16];
@@ -723,9 +753,23 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         vertex(v, v - __umul24(di, nv), M);
       }
     }
+    // A chunk is dropped when all of it lies outside one plane, beside the
+    // band, or between the same two columns or rows of pixel centres.
     bool gone = false;
+    dirty = __ballot(dirty) != 0ull;  // lanes without a vertex in the last round too
+    if (dirty) {
 #pragma unroll
-    for (int b = 0; b < 10; ++b) gone = gone || __ballot(!((out >> b) & 1u)) == 0ull;
+      for (int b = 0; b < 6; ++b) gone = gone || __ballot(!((out >> b) & 1u)) == 0ull;
+    } else {
+      // first and last centre of the lane's vertices; none where c1 < c0
+      const int cx0 = (xmin + 127) >> 8, cx1 = (xmax - 128) >> 8;
+      const int cy0 = (ymin + 127) >> 8, cy1 = (ymax - 128) >> 8;
+      const int kx = __builtin_amdgcn_readfirstlane(cx0), ky = __builtin_amdgcn_readfirstlane(cy0);
+      const bool any = xmin <= xmax;
+      gone = !__ballot(cx1 >= 0) || !__ballot(cx0 < W) || !__ballot(cy1 >= t.j0) ||
+             !__ballot(cy0 <= t.j1) || !__ballot(any && (cx0 != kx || cx1 >= kx)) ||
+             !__ballot(any && (cy0 != ky || cy1 >= ky));
+    }
     if (gone) continue;
     wave_fence();
 
@@ -736,29 +780,26 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       const uint32_t u = min(q0 + (uint32_t)lane, n - 1u);
       const uint32_t di = __umul24(u, inv_nt) >> 16;
       const uint32_t tri = mtab[u - __umul24(di, nt)];
-      const int2* vt = vxy + __umul24(di, nv);
-      const int2 a = vt[tri & 0xffu], b = vt[(tri >> 8) & 0xffu], cc = vt[tri >> 16];
-      const int32_t X0 = a.x >> 6, X1 = b.x >> 6, X2 = cc.x >> 6;
-      const int32_t Y0 = a.y >> 1, Y1 = b.y >> 1, Y2 = cc.y >> 1;
-      const double area = (double)(X1 - X0) * (double)(Y2 - Y0) -
-                          (double)(X2 - X0) * (double)(Y1 - Y0);
-      const int32_t a0 = max((min(X0, min(X1, X2)) + 127) >> 8, 0);
-      const int32_t a1 = min((max(X0, max(X1, X2)) - 128) >> 8, W - 1);
-      const int32_t b0 = max((min(Y0, min(Y1, Y2)) + 127) >> 8, t.j0);
-      const int32_t b1 = min((max(Y0, max(Y1, Y2)) - 128) >> 8, t.j1);
+      const uint32_t vb = __umul24(di, nv);
+      const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu), ic = vb + (tri >> 16);
+      const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
+      const int32_t X[3] = {a.x, b.x, cc.x}, Y[3] = {a.y, b.y, cc.y};
+      FixTri T;
+      snapped_box(X, Y, W, t.j0, t.j1, T);
       const bool here = q0 + (uint32_t)lane < n;
-      const uint32_t any = (uint32_t)(a.x | b.x | cc.x) & (uint32_t)kOutMask;
-      const bool clip = here && any != 0u && (a.x & b.x & cc.x & kOutMask) == 0;
-      const bool live = here && any == 0u && ((a.y | b.y | cc.y) & 1) == 0 && area > 0.0 &&
-                        a0 <= a1 && b0 <= b1;
-      const uint64_t ml = __ballot(live), mc = __ballot(clip);
-      const uint64_t below = (1ull << lane) - 1ull;
-      if (live) qu[live_n + (uint32_t)__popcll(ml & below)] = (uint8_t)u;
-      live_n += (uint32_t)__popcll(ml);
-      if (mc) {
-        if (clip) qu[kBandTris - 1u - (clip_n + (uint32_t)__popcll(mc & below))] = (uint8_t)u;
+      bool live = here && T.i0 <= T.i1 && T.j0 <= T.j1 && snapped_area(X, Y) > 0.0;
+      if (dirty) {
+        const uint32_t ca = vertex_code(vd[ia]), cb = vertex_code(vd[ib]), c3 = vertex_code(vd[ic]);
+        const uint32_t some = ca | cb | c3;
+        const bool clip = here && (some & kOutMask) && !(ca & cb & c3 & kOutMask);
+        live = live && some == 0u;
+        const uint64_t mc = __ballot(clip);
+        if (clip) qu[kBandTris - 1u - (clip_n + lanes_below(mc))] = (uint8_t)u;
         clip_n += (uint32_t)__popcll(mc);
       }
+      const uint64_t ml = __ballot(live);
+      if (live) qu[live_n + lanes_below(ml)] = (uint8_t)u;
+      live_n += (uint32_t)__popcll(ml);
     }
     wave_fence();
 
@@ -777,10 +818,12 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu),
                          ic = vb + (tri >> 16);
           const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
-          const SnapVert sa = {a.x >> 6, a.y >> 1, vd[ia], 0.0f, true};
-          const SnapVert sb = {b.x >> 6, b.y >> 1, vd[ib], 0.0f, true};
-          const SnapVert sc = {cc.x >> 6, cc.y >> 1, vd[ic], 0.0f, true};
-          has = setup_snapped(sa, sb, sc, W, H, t.j0, t.j1, T);
+          const int32_t X[3] = {a.x, b.x, cc.x}, Y[3] = {a.y, b.y, cc.y};
+          const float d[3] = {__uint_as_float(vd[ia]), __uint_as_float(vd[ib]),
+                              __uint_as_float(vd[ic])};
+          snapped_box(X, Y, W, t.j0, t.j1, T);
+          snapped_planes(X, Y, d, T);
+          has = true;
           rank = (slot0 + u) << 3;
         }
         k0 = min(k0 + 64u, live_n);
@@ -840,7 +883,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         U.j0 = rl(T.j0, l);
         U.j1 = rl(T.j1, l);
         U.bias = (uint32_t)rl((int)T.bias, l);
-        band_raster_wave<double>(pix, t, lane, U, (uint32_t)rl((int)rank, l));
+        band_raster_wave(pix, t, lane, U, (uint32_t)rl((int)rank, l));
       }
     }
     wave_fence();  // the next chunk rewrites the table

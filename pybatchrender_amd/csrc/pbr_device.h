@@ -300,36 +300,32 @@ __device__ __forceinline__ void snap_vertex(const CVert& v, int W, int H, SnapVe
   S.ok = true;
 }
 
-// The per-triangle rest of (b) on three snapped vertices: cull, bound,
-// fill-rule bias and depth plane; false if the triangle yields no fragment
-// in GL rows [jr0, jr1].
-__device__ __forceinline__ bool setup_snapped(const SnapVert& s0, const SnapVert& s1,
-                                              const SnapVert& s2, int W, int H, int jr0, int jr1,
-                                              FixTri& T) {
-  if (!(s0.ok && s1.ok && s2.ok)) return false;
-  // Snapped positions satisfy |X|, |Y| <= 2^24 (snap_vertex rejects larger
-  // ones), so coordinate differences fit 25 bits, their products are below
-  // 2^50 and exact in double, and so is the difference of two products:
-  // 32-bit integer and double arithmetic give the exact integer results of
-  // the 64-bit integer forms, at a fraction of their instructions.
-  const int32_t X[3] = {s0.X, s1.X, s2.X}, Y[3] = {s0.Y, s1.Y, s2.Y};
-  const float d[3] = {s0.d, s1.d, s2.d};
-  T.invw[0] = s0.invw;
-  T.invw[1] = s1.invw;
-  T.invw[2] = s2.invw;
-  const double area = (double)(X[1] - X[0]) * (double)(Y[2] - Y[0]) -
-                      (double)(X[2] - X[0]) * (double)(Y[1] - Y[0]);
-  if (!(area > 0.0)) return false;
+// Twice the signed area of a snapped triangle.  Snapped positions satisfy
+// |X|, |Y| <= 2^24 (snap_vertex rejects larger ones), so coordinate
+// differences fit 25 bits, their products are below 2^50 and exact in double,
+// and so is the difference of two products: 32-bit integer and double
+// arithmetic give the exact integer results of the 64-bit integer forms, at a
+// fraction of their instructions.
+__device__ __forceinline__ double snapped_area(const int32_t X[3], const int32_t Y[3]) {
+  return (double)(X[1] - X[0]) * (double)(Y[2] - Y[0]) -
+         (double)(X[2] - X[0]) * (double)(Y[1] - Y[0]);
+}
+
+// Its box of pixels within GL rows [jr0, jr1] (empty: i0 > i1 or j0 > j1).
+__device__ __forceinline__ void snapped_box(const int32_t X[3], const int32_t Y[3], int W, int jr0,
+                                            int jr1, FixTri& T) {
   const int32_t xmin = min(X[0], min(X[1], X[2])), xmax = max(X[0], max(X[1], X[2]));
   const int32_t ymin = min(Y[0], min(Y[1], Y[2])), ymax = max(Y[0], max(Y[1], Y[2]));
   // pixel centres 256 i + 128 inside [min, max]: floor division by 256
-  const int32_t i0 = max((xmin - 128 + 255) >> 8, 0), i1 = min((xmax - 128) >> 8, W - 1);
-  const int32_t j0 = max((ymin - 128 + 255) >> 8, jr0), j1 = min((ymax - 128) >> 8, jr1);
-  if (i0 > i1 || j0 > j1) return false;
-  T.i0 = i0;
-  T.i1 = i1;
-  T.j0 = j0;
-  T.j1 = j1;
+  T.i0 = max((xmin - 128 + 255) >> 8, 0);
+  T.i1 = min((xmax - 128) >> 8, W - 1);
+  T.j0 = max((ymin - 128 + 255) >> 8, jr0);
+  T.j1 = min((ymax - 128) >> 8, jr1);
+}
+
+// Fill-rule bias and depth plane of a snapped triangle of positive area.
+__device__ __forceinline__ void snapped_planes(const int32_t X[3], const int32_t Y[3],
+                                               const float d[3], FixTri& T) {
   uint32_t bias = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -353,6 +349,24 @@ __device__ __forceinline__ bool setup_snapped(const SnapVert& s0, const SnapVert
   T.zx = (float)zxd;
   T.zy = (float)zyd;
   T.zc = (float)zcd;
+}
+
+// The per-triangle rest of (b) on three snapped vertices: cull, bound,
+// fill-rule bias and depth plane; false if the triangle yields no fragment
+// in GL rows [jr0, jr1].
+__device__ __forceinline__ bool setup_snapped(const SnapVert& s0, const SnapVert& s1,
+                                              const SnapVert& s2, int W, int H, int jr0, int jr1,
+                                              FixTri& T) {
+  if (!(s0.ok && s1.ok && s2.ok)) return false;
+  const int32_t X[3] = {s0.X, s1.X, s2.X}, Y[3] = {s0.Y, s1.Y, s2.Y};
+  const float d[3] = {s0.d, s1.d, s2.d};
+  T.invw[0] = s0.invw;
+  T.invw[1] = s1.invw;
+  T.invw[2] = s2.invw;
+  if (!(snapped_area(X, Y) > 0.0)) return false;
+  snapped_box(X, Y, W, jr0, jr1, T);
+  if (T.i0 > T.i1 || T.j0 > T.j1) return false;
+  snapped_planes(X, Y, d, T);
   return true;
 }
 
