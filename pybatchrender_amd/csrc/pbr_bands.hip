@@ -46,6 +46,9 @@ constexpr int kBandPixels = 8192;
 constexpr int kBandLds = 80 * 1024;  // half a CU's LDS: two workgroups share a CU
 constexpr int kSmallPixels = 12;  // box pixels one lane rasterises alone
 constexpr uint32_t kDepthOne = 0x3f800000u;
+// Sub-triangle number of a triangle that no plane clips (a clipped polygon has
+// at most seven, 0 to 6), so that shading knows it without testing vertices.
+constexpr uint32_t kUnclipped = 7;
 
 // Per-node launch constants.
 struct BandNode {
@@ -439,7 +442,7 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
   const int runs = __popcll(hm);
   int32_t X[3] = {0, 0, 0}, Y[3] = {0, 0, 0};
   float iw[3] = {0.0f, 0.0f, 0.0f}, n[3][3] = {}, base[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  uint32_t code = 0;  // outcodes; bit 6: flat
+  uint32_t fl = 0;  // the winner's node flags
   if (runs <= kShadeRuns) {
     const int run = __popcll(hm & ((2ull << lane) - 1ull)) - 1;
     if (head) heads[run] = (uint8_t)lane;
@@ -447,7 +450,7 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
     const int u = (lane * 86) >> 8, k = lane - 3 * u;
     CVert cv = {};
     SnapVert sv = {};
-    uint32_t fl = 0;
+    uint32_t vf = 0;
     float rgba[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     // every lane takes part in the reads of other lanes' slots
     const uint32_t vslot = (uint32_t)from_lane(u < runs ? (int)heads[u] : 0, (int)slot);
@@ -464,7 +467,7 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
       load_vertex(D.vertices, R.voff + (int)id, vv);
       transform_vertex(M, VP, vv, cv);
       snap_vertex(cv, F.W, F.H, sv);
-      fl = outcode(cv, F.guard) | ((R.flags & 2u) << 5);
+      vf = R.flags;
     }
     const int src = mine ? 3 * run : 0;
 #pragma unroll
@@ -472,12 +475,12 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
       X[v] = from_lane(src + v, sv.X);
       Y[v] = from_lane(src + v, sv.Y);
       iw[v] = from_lane(src + v, sv.invw);
-      code |= (uint32_t)from_lane(src + v, (int)fl);
 #pragma unroll
       for (int c = 0; c < 3; ++c) n[v][c] = from_lane(src + v, cv.n[c]);
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) base[c] = from_lane(src, rgba[c]);
+    fl = (uint32_t)from_lane(src, (int)vf);
   } else if (mine) {
     const SlotRef R = band_slot(s, nodes, nn, tab, slot);
     const f32x4 c4 = ((global_cfloat4*)(uintptr_t)R.cols)[R.row];
@@ -487,7 +490,7 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
     base[3] = c4.w;
     float M[16];
     load_mat4_global(R.trans + R.row * 16, M);
-    code = (R.flags & 2u) << 5;
+    fl = R.flags;
 #pragma unroll
     for (int v = 0; v < 3; ++v) {
       float vv[6];
@@ -496,7 +499,6 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
       SnapVert sv;
       transform_vertex(M, VP, vv, cv);
       snap_vertex(cv, F.W, F.H, sv);
-      code |= outcode(cv, F.guard);
       X[v] = sv.X;
       Y[v] = sv.Y;
       iw[v] = sv.invw;
@@ -504,10 +506,10 @@ __device__ __forceinline__ void band_shade_smooth(const pbr_scene_desc& D, const
       for (int c = 0; c < 3; ++c) n[v][c] = cv.n[c];
     }
   }
-  const bool flat = (code & 64u) != 0u;
+  const bool flat = (fl & 2u) != 0u;
 
   // winners that straddle a clip plane: their polygons, four slots at a time
-  bool clipped = mine && !flat && (code & (uint32_t)kOutMask) != 0u;
+  bool clipped = mine && !flat && q != (int)kUnclipped;
   for (uint64_t cm = __ballot(clipped); cm; cm = __ballot(clipped)) {
     uint32_t gs = 0;
     int group = -1, count = 0;
@@ -803,61 +805,8 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     }
     wave_fence();
 
-    // 64 live triangles are set up at a time, then clipped ones four at a
-    // time (a lane per sub-triangle); each set is rasterised at once
-    for (uint32_t k0 = 0; k0 < live_n + clip_n;) {
-      FixTri T;
-      bool has = false;
-      uint32_t rank = 0;
-      if (k0 < live_n) {
-        if (k0 + (uint32_t)lane < live_n) {
-          const uint32_t u = qu[k0 + (uint32_t)lane];
-          const uint32_t di = __umul24(u, inv_nt) >> 16;
-          const uint32_t tri = mtab[u - __umul24(di, nt)];
-          const uint32_t vb = __umul24(di, nv);
-          const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu),
-                         ic = vb + (tri >> 16);
-          const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
-          const int32_t X[3] = {a.x, b.x, cc.x}, Y[3] = {a.y, b.y, cc.y};
-          const float d[3] = {__uint_as_float(vd[ia]), __uint_as_float(vd[ib]),
-                              __uint_as_float(vd[ic])};
-          snapped_box(X, Y, W, t.j0, t.j1, T);
-          snapped_planes(X, Y, d, T);
-          has = true;
-          rank = (slot0 + u) << 3;
-        }
-        k0 = min(k0 + 64u, live_n);
-      } else {
-        const uint32_t k = k0 - live_n + (uint32_t)(lane >> 4);
-        int pn = k < clip_n ? 3 : 0;
-        const uint32_t u = qu[kBandTris - 1u - min(k, clip_n - 1u)];
-        CVert cv = {};
-        if (pn && (lane & 15) < 3) {
-          const uint32_t di = __umul24(u, inv_nt) >> 16;
-          group_vertex(D, trans, row0 + di, voff, mtab[u - __umul24(di, nt)], VP, lane, cv);
-        }
-        clip_groups<4>(cv.p, pn, F.guard, lane);
-        SnapVert S;
-        snap_vertex(cv, W, H, S);
-        const int lost = 0x7fffffff;  // X of a vertex that did not snap
-        const int X = S.ok ? S.X : lost;
-        const int at = lane & 48, q = lane & 15;
-        const bool sub = q + 2 < pn;
-        const int f1 = sub ? at + q + 1 : at, f2 = sub ? at + q + 2 : at;
-        SnapVert V[3];
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-          const int f = e == 0 ? at : (e == 1 ? f1 : f2);
-          V[e].X = from_lane(f, X);
-          V[e].Y = from_lane(f, S.Y);
-          V[e].d = from_lane(f, S.d);
-          V[e].invw = 0.0f;
-          V[e].ok = V[e].X != lost;
-        }
-        has = sub && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
-        rank = ((slot0 + u) << 3) | (uint32_t)q;
-        k0 += 4u;
-      }
+    // set-up triangles of the lanes (`has`) into the band's pixels
+    auto draw = [&](bool has, const FixTri& T, uint32_t rank) {
       const bool fits =  // edge values fit 32 bits
           has &&
           max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
@@ -885,6 +834,62 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         U.bias = (uint32_t)rl((int)T.bias, l);
         band_raster_wave(pix, t, lane, U, (uint32_t)rl((int)rank, l));
       }
+    };
+    // 64 live triangles are set up at a time, then clipped ones four at a time
+    // (a lane per sub-triangle); each set is rasterised at once
+    for (uint32_t k0 = 0; k0 < live_n; k0 += 64u) {
+      FixTri T;
+      bool has = false;
+      uint32_t rank = 0;
+      if (k0 + (uint32_t)lane < live_n) {
+        const uint32_t u = qu[k0 + (uint32_t)lane];
+        const uint32_t di = __umul24(u, inv_nt) >> 16;
+        const uint32_t tri = mtab[u - __umul24(di, nt)];
+        const uint32_t vb = __umul24(di, nv);
+        const uint32_t ia = vb + (tri & 0xffu), ib = vb + ((tri >> 8) & 0xffu),
+                       ic = vb + (tri >> 16);
+        const int2 a = vxy[ia], b = vxy[ib], cc = vxy[ic];
+        const int32_t X[3] = {a.x, b.x, cc.x}, Y[3] = {a.y, b.y, cc.y};
+        const float d[3] = {__uint_as_float(vd[ia]), __uint_as_float(vd[ib]),
+                            __uint_as_float(vd[ic])};
+        snapped_box(X, Y, W, t.j0, t.j1, T);
+        snapped_planes(X, Y, d, T);
+        has = true;
+        rank = ((slot0 + u) << 3) | kUnclipped;
+      }
+      draw(has, T, rank);
+    }
+    for (uint32_t k0 = 0; k0 < clip_n; k0 += 4u) {
+      FixTri T;
+      const uint32_t k = k0 + (uint32_t)(lane >> 4);
+      int pn = k < clip_n ? 3 : 0;
+      const uint32_t u = qu[kBandTris - 1u - min(k, clip_n - 1u)];
+      CVert cv = {};
+      if (pn && (lane & 15) < 3) {
+        const uint32_t di = __umul24(u, inv_nt) >> 16;
+        group_vertex(D, trans, row0 + di, voff, mtab[u - __umul24(di, nt)], VP, lane, cv);
+      }
+      clip_groups<4>(cv.p, pn, F.guard, lane);
+      SnapVert S;
+      snap_vertex(cv, W, H, S);
+      const int lost = 0x7fffffff;  // X of a vertex that did not snap
+      const int X = S.ok ? S.X : lost;
+      const int at = lane & 48, q = lane & 15;
+      const bool sub = q + 2 < pn;
+      const int f1 = sub ? at + q + 1 : at, f2 = sub ? at + q + 2 : at;
+      SnapVert V[3];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        const int f = e == 0 ? at : (e == 1 ? f1 : f2);
+        V[e].X = from_lane(f, X);
+        V[e].Y = from_lane(f, S.Y);
+        V[e].d = from_lane(f, S.d);
+        V[e].invw = 0.0f;
+        V[e].ok = V[e].X != lost;
+      }
+      const bool has = sub && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
+      const uint32_t rank = ((slot0 + u) << 3) | (uint32_t)q;
+      draw(has, T, rank);
     }
     wave_fence();  // the next chunk rewrites the table
   }

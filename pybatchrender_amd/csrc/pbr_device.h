@@ -323,6 +323,21 @@ __device__ __forceinline__ void snapped_box(const int32_t X[3], const int32_t Y[
   T.j1 = min((ymax - 128) >> 8, jr1);
 }
 
+// n / ar for several n: Newton's iteration for the reciprocal from the
+// hardware's estimate, then the quotient with one correction by its exact
+// remainder, which rounds it correctly (Markstein).  The steps of a double
+// division without its range scaling: ar is a whole number of 1 to 2^51, |n| 0
+// or 2^-210 to 2^27.
+__device__ __forceinline__ double plane_rcp(double ar) {
+  double r = __builtin_amdgcn_rcp(ar);
+  r = __builtin_fma(r, __builtin_fma(-ar, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-ar, r, 1.0), r);
+}
+__device__ __forceinline__ double plane_div(double n, double ar, double r) {
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-ar, q, n), r, q);
+}
+
 // Fill-rule bias and depth plane of a snapped triangle of positive area.
 __device__ __forceinline__ void snapped_planes(const int32_t X[3], const int32_t Y[3],
                                                const float d[3], FixTri& T) {
@@ -337,17 +352,19 @@ __device__ __forceinline__ void snapped_planes(const int32_t X[3], const int32_t
     T.Y[k] = Y[k];
   }
   T.bias = bias;
-  double x0 = (double)X[0] * (1.0 / 256.0), y0 = (double)Y[0] * (1.0 / 256.0);
-  double ax = (double)X[1] * (1.0 / 256.0) - x0, ay = (double)Y[1] * (1.0 / 256.0) - y0;
-  double bx = (double)X[2] * (1.0 / 256.0) - x0, by = (double)Y[2] * (1.0 / 256.0) - y0;
-  double ar = ax * by - bx * ay;
-  double dz1 = (double)d[1] - (double)d[0], dz2 = (double)d[2] - (double)d[0];
-  double zxd = (dz1 * by - dz2 * ay) / ar;
-  double zyd = (dz2 * ax - dz1 * bx) / ar;
-  double zcd = (double)d[0] - zxd * x0;
-  zcd = zcd - zyd * y0;
-  T.zx = (float)zxd;
-  T.zy = (float)zyd;
+  // The depth plane in units of 1/256 pixel: every scale is a power of two,
+  // so each rounding is that of the plane in pixels.
+  const double ax = (double)(X[1] - X[0]), ay = (double)(Y[1] - Y[0]);
+  const double bx = (double)(X[2] - X[0]), by = (double)(Y[2] - Y[0]);
+  const double ar = ax * by - bx * ay;
+  const double dz1 = (double)d[1] - (double)d[0], dz2 = (double)d[2] - (double)d[0];
+  const double r = plane_rcp(ar);
+  const double zxd = plane_div(dz1 * by - dz2 * ay, ar, r);
+  const double zyd = plane_div(dz2 * ax - dz1 * bx, ar, r);
+  double zcd = (double)d[0] - zxd * (double)X[0];
+  zcd = zcd - zyd * (double)Y[0];
+  T.zx = (float)(zxd * 256.0);
+  T.zy = (float)(zyd * 256.0);
   T.zc = (float)zcd;
 }
 
