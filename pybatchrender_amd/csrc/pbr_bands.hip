@@ -36,8 +36,9 @@ using namespace pbr_host;
 
 namespace {
 
-constexpr int kBandBlock = 512;
-constexpr int kBandWaves = kBandBlock / 64;
+constexpr int kBandWaves = 8;     // waves of a workgroup, two workgroups on a CU
+constexpr int kWideWaves = 16;    // or one workgroup with all the waves of a CU
+constexpr int kWideItems = 256;   // for at most this many workgroups (see bands_plan)
 constexpr int kBandVerts = 136;   // vertices a wave's table holds at most
 constexpr int kBandTris = 256;    // triangles of one chunk (8-bit queue entries)
 constexpr int kBandTable = 512;   // triangles of all meshes (LDS index table) at most
@@ -63,6 +64,7 @@ struct BandFrame {
   uint32_t max_slots;  // slots of the largest scene
   uint32_t budget;     // slots drawn of the whole batch at most
   int uniform;         // 1: no node has per-scene counts
+  int waves;           // of a workgroup
   int verts;           // entries of a wave's vertex table
   int ntab;            // triangles in the LDS index table
   int vec;             // 1: four pixels of a plane are whole aligned dwords / float4s
@@ -184,9 +186,6 @@ __device__ __forceinline__ void band_edges(const FixTri& T, int i, int j, BandEd
 }
 
 __device__ __forceinline__ bool band_inside(const int32_t e[3]) { return (e[0] | e[1] | e[2]) >= 0; }
-__device__ __forceinline__ bool band_inside(const double e[3]) {
-  return e[0] >= 0.0 && e[1] >= 0.0 && e[2] >= 0.0;
-}
 
 // One lane, the whole box.
 __device__ __forceinline__ void band_raster_lane(unsigned long long* pix, const BandCtx& t,
@@ -214,11 +213,35 @@ __device__ __forceinline__ void band_raster_lane(unsigned long long* pix, const 
   }
 }
 
-// The rows of the lanes' triangles (`has`, extents within kIntExtent) dealt to
-// the lanes of the wave, 64 rows at a time: a lane finds its triangle by a
-// binary search of the running row counts and walks the row.  Triangles of
-// more than a few pixels keep the whole wave busy this way, where a lane per
-// triangle would walk as long as the largest box.
+// Pixels lo .. hi of a row of w + 1 that lie inside the three edges (e at the
+// row's first pixel): each edge's crossing from a reciprocal estimate, off by
+// less than a pixel's half, and one exact evaluation at the nearest pixel.
+__device__ __forceinline__ void row_span(const BandEdges<double>& E, int w, int& lo, int& hi) {
+  lo = 0;
+  hi = w;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double A = E.A[k], e = E.e[k];
+    const double q = rint(-e * __builtin_amdgcn_rcp(A));
+    // in range before it becomes an integer (A = 0: any value)
+    const double c = fmin(fmax(q, -1.0), (double)(w + 1));
+    const bool out = __builtin_fma(A, c, e) < 0.0;
+    const int i = (int)c;
+    if (A > 0.0) lo = max(lo, out ? i + 1 : i);
+    else if (A < 0.0) hi = min(hi, out ? i - 1 : i);
+    else if (e < 0.0) hi = -1;
+  }
+}
+
+// The rows of the lanes' triangles (`has`) dealt to the lanes of the wave, 64
+// rows at a time: a lane finds its triangle by a binary search of the running
+// row counts and walks the row.  Triangles of more than a few pixels keep the
+// whole wave busy this way, where a lane per triangle would walk as long as
+// the largest box.  Num int32_t (extents within kIntExtent) tests each pixel
+// of the box's row; double, for the long thin triangles that reach out of the
+// frame, walks the row's span: in blocks of 8 x 8 pixels of the box they took
+// a steering scene's wave longest of all.
+template <typename Num>
 __device__ __forceinline__ void band_raster_rows(unsigned long long* pix, const BandCtx& t,
                                                  int lane, bool has, const FixTri& T,
                                                  uint32_t rank) {
@@ -243,51 +266,29 @@ __device__ __forceinline__ void band_raster_rows(unsigned long long* pix, const 
     const uint32_t ur = (uint32_t)from_lane(l, (int)rank);
     U.bias = (uint32_t)b >> 26;
     const int i0 = b & 0x1fff, w = ((b >> 13) & 0x1fff) - i0;
-    BandEdges<int32_t> E;
+    BandEdges<Num> E;
     band_edges(U, i0, j, E);
     const float tz = fmaf(zy, (float)j + 0.5f, zc);
-    float x = (float)i0 + 0.5f;
     unsigned long long* q = pix + (t.j1 - j) * t.W + i0;
-    if (r0 + lane < total)
+    if (r0 + lane >= total) continue;
+    if constexpr (sizeof(Num) == 4) {
+      float x = (float)i0 + 0.5f;
       for (int i = 0; i <= w; ++i) {
         if (band_inside(E.e)) band_fragment(q + i, clamp_depth(fmaf(zx, x, tz)), ur);
 #pragma unroll
         for (int k = 0; k < 3; ++k) E.e[k] += E.A[k];
         x += 1.0f;
       }
-  }
-}
-
-// The whole wave, in blocks of 8 x 8 pixels, edge values in double.  Every
-// argument is uniform.
-__device__ __forceinline__ void band_raster_wave(unsigned long long* pix, const BandCtx& t,
-                                                 int lane, const FixTri& T, uint32_t rank) {
-  BandEdges<double> E;
-  band_edges(T, T.i0, T.j0, E);
-  const int li = lane & 7, lj = lane >> 3;
-  double row[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) row[k] = E.e[k] + E.A[k] * (double)li + E.B[k] * (double)lj;
-  for (int jb = T.j0; jb <= T.j1; jb += 8) {
-    const int j = jb + lj;
-    const float tz = fmaf(T.zy, (float)j + 0.5f, T.zc);
-    unsigned long long* q = pix + (t.j1 - j) * t.W + T.i0 + li;
-    double e[3] = {row[0], row[1], row[2]};
-    for (int ib = T.i0; ib <= T.i1; ib += 8, q += 8) {
-      const int i = ib + li;
-      if (i <= T.i1 && j <= T.j1 && band_inside(e))
-        band_fragment(q, clamp_depth(fmaf(T.zx, (float)i + 0.5f, tz)), rank);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) e[k] += E.A[k] * (double)8;
+    } else {
+      int lo, hi;
+      row_span(E, w, lo, hi);
+      float x = (float)(i0 + lo) + 0.5f;
+      for (int i = lo; i <= hi; ++i) {
+        band_fragment(q + i, clamp_depth(fmaf(zx, x, tz)), ur);
+        x += 1.0f;
+      }
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) row[k] += E.B[k] * (double)8;
   }
-}
-
-__device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-__device__ __forceinline__ float rlf(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
 // Bit p: not inside clip plane p (NaN distances count as outside, as the
@@ -591,7 +592,7 @@ __device__ __forceinline__ uint32_t band_gather(uint32_t p0, uint32_t p1, uint32
 // [th][W], the waves' vertex tables (int2 [verts], float depth [verts]) and
 // triangle queues, then the index table.
 template <bool SMOOTH, int OM>
-__global__ __launch_bounds__(kBandBlock)
+__global__ __launch_bounds__(kWideWaves * 64)
 __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_frame_out O,
                                                           BandFrame F, const uint32_t* scene_off,
                                                           const uint32_t* order, uint32_t* hdr, Light lt, float4 bg) {
@@ -601,6 +602,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   const int tid = (int)threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = F.W, H = F.H, nn = D.num_nodes;
+  const int waves = F.waves, block = waves * 64;
   BandCtx t;
   const uint32_t at = blockIdx.x / (uint32_t)F.bands;
   const int band = (int)(blockIdx.x - at * (uint32_t)F.bands);
@@ -612,11 +614,11 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   const int npx = rows * W;
   int2* tables = reinterpret_cast<int2*>(pix + ((F.th * W + 1) & ~1));
   int2* vxy = tables + wave * F.verts;
-  unsigned char* after = reinterpret_cast<unsigned char*>(tables + kBandWaves * F.verts);
+  unsigned char* after = reinterpret_cast<unsigned char*>(tables + waves * F.verts);
   uint32_t* vd = reinterpret_cast<uint32_t*>(after) + wave * F.verts;
-  after += sizeof(float) * (size_t)kBandWaves * F.verts;
+  after += sizeof(float) * (size_t)waves * F.verts;
   uint8_t* qu = after + wave * kBandTris;
-  uint32_t* tab = reinterpret_cast<uint32_t*>(after + kBandWaves * kBandTris);
+  uint32_t* tab = reinterpret_cast<uint32_t*>(after + waves * kBandTris);
 
   if (F.uniform && blockIdx.x == 0 && tid == 0) hdr[0] = 0u;  // no overflow
   // slots of this scene that are drawn (all, unless the batch exceeds its
@@ -630,9 +632,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     ndraw = e > o ? e - o : 0u;
   }
   // two keys per store (the key area is padded to an even count)
-  for (int p = tid; p < (npx + 1) / 2; p += kBandBlock)
+  for (int p = tid; p < (npx + 1) / 2; p += block)
     reinterpret_cast<uint4*>(pix)[p] = make_uint4(0u, kDepthOne, 0u, kDepthOne);
-  for (int q = tid; q < F.ntab; q += kBandBlock) tab[q] = pool_triangle(D, q);
+  for (int q = tid; q < F.ntab; q += block) tab[q] = pool_triangle(D, q);
   if (wave == 0) {
     uint32_t cnt = 0, nslot = 0, nchunk = 0;
     if (lane < nn) {
@@ -815,25 +817,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       const bool small = fits && w * h <= kSmallPixels;
       if (small) band_raster_lane(pix, t, T, rank);
       const bool rows = fits && !small;
-      if (__ballot(rows)) band_raster_rows(pix, t, lane, rows, T, rank);
-      for (uint64_t m = __ballot(has && !fits); m; m &= m - 1ull) {
-        const int l = __ffsll((unsigned long long)m) - 1;
-        FixTri U;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          U.X[k] = rl(T.X[k], l);
-          U.Y[k] = rl(T.Y[k], l);
-        }
-        U.zx = rlf(T.zx, l);
-        U.zy = rlf(T.zy, l);
-        U.zc = rlf(T.zc, l);
-        U.i0 = rl(T.i0, l);
-        U.i1 = rl(T.i1, l);
-        U.j0 = rl(T.j0, l);
-        U.j1 = rl(T.j1, l);
-        U.bias = (uint32_t)rl((int)T.bias, l);
-        band_raster_wave(pix, t, lane, U, (uint32_t)rl((int)rank, l));
-      }
+      if (__ballot(rows)) band_raster_rows<int32_t>(pix, t, lane, rows, T, rank);
+      const bool far = has && !fits;
+      if (__ballot(far)) band_raster_rows<double>(pix, t, lane, far, T, rank);
     };
     // 64 live triangles are set up at a time, then clipped ones four at a time
     // (a lane per sub-triangle); each set is rasterised at once
@@ -987,7 +973,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       if ((cov >> k) & 1u) *q++ = (uint16_t)(p0 + lane * step + k);
   };
   // Shades the pixels q[0 .. take) (take <= 64).
-  uint8_t* heads = reinterpret_cast<uint8_t*>(tab) - 64 * kBandWaves + 64 * wave;
+  uint8_t* heads = reinterpret_cast<uint8_t*>(tab) - 64 * waves + 64 * wave;
   auto shade_batch = [&](const uint16_t* q, uint32_t take) {
     const int p = q[min((uint32_t)lane, take - 1u)];
     const uint32_t rank = (uint32_t)pix[p];
@@ -1026,10 +1012,10 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     // triangle queues), so that only one batch per block of pixels is not
     // full; a block is what the queue holds
     uint16_t* pq = reinterpret_cast<uint16_t*>(tables);
-    const int hold = (kBandWaves * (12 * F.verts + kBandTris - 64) / 2) & ~255;
+    const int hold = (waves * (12 * F.verts + kBandTris - 64) / 2) & ~255;
     for (int b0 = 0; b0 < npx; b0 += hold) {
       const int bend = min(npx, b0 + hold);
-      for (int p0 = b0 + wave * 64 * step; p0 < bend; p0 += kBandBlock * step) {
+      for (int p0 = b0 + wave * 64 * step; p0 < bend; p0 += block * step) {
         uint32_t sum;
         const uint32_t cov = scan(p0, bend), at = place(cov, sum);
         if (sum) {
@@ -1041,7 +1027,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       }
       __syncthreads();
       const uint32_t total = (uint32_t)__builtin_amdgcn_readfirstlane((int)covered_n);
-      for (uint32_t k0 = (uint32_t)wave * 64u; k0 < total; k0 += (uint32_t)kBandBlock)
+      for (uint32_t k0 = (uint32_t)wave * 64u; k0 < total; k0 += (uint32_t)block)
         shade_batch(pq + k0, min(total - k0, 64u));
       __syncthreads();
       if (bend < npx) {  // the next block starts with an empty queue
@@ -1060,7 +1046,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
         const uint32_t cov = scan(p0, npx), at = place(cov, sum);
         push(pq + pend + at, cov, p0);
         pend += sum;
-        p0 += kBandBlock * step;
+        p0 += block * step;
       }
       wave_fence();
       uint32_t done = 0;
@@ -1090,7 +1076,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   };
   if (F.vec) {
     // four pixels of every channel from one read of their keys
-    for (int p = tid * 4; p < npx; p += kBandBlock * 4) {
+    for (int p = tid * 4; p < npx; p += block * 4) {
       const ulonglong2 ka = *reinterpret_cast<const ulonglong2*>(pix + p);
       const ulonglong2 kb = *reinterpret_cast<const ulonglong2*>(pix + p + 2);
       const auto v0 = pixel(ka.x), v1 = pixel(ka.y), v2 = pixel(kb.x), v3 = pixel(kb.y);
@@ -1117,7 +1103,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
   for (int ch = 0; ch < C; ++ch) {
     unsigned char* dst = cout + (size_t)ch * plane * ES;
     const int mis = (int)(((uintptr_t)dst & 3u) / ES);
-    for (int k = tid; k * PER - mis < npx; k += kBandBlock) {
+    for (int k = tid; k * PER - mis < npx; k += block) {
       const int p = k * PER - mis;
       if (p >= 0 && p + PER <= npx) {
         uint32_t v;
@@ -1184,15 +1170,32 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   if (ntab > kBandTable) return false;
   F.ntab = ntab;
   const size_t stat = sizeof(NodeLds) * PBR_MAX_NODES + 64;
-  const size_t rest = (size_t)kBandWaves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)ntab;
-  const int px = std::min((int)((kBandLds - stat - rest) / 8), kBandPixels);
+  const auto rest = [&](int waves) {
+    return (size_t)waves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)ntab;
+  };
+  const auto split = [&](int waves, int most, int bands) {
+    F.waves = waves;
+    F.bands = std::max((D->height + most - 1) / most, bands);
+    F.th = (D->height + F.bands - 1) / F.bands;
+    F.bands = (D->height + F.th - 1) / F.th;
+    P.lds = (size_t)8 * ((F.th * F.W + 1) & ~1) + rest(waves);
+  };
+  const int px = std::min((int)((kBandLds - stat - rest(kBandWaves)) / 8), kBandPixels);
   if (D->width > px) return false;
-  const int most = px / D->width;
-  F.bands = (D->height + most - 1) / most;
+  split(kBandWaves, px / D->width, 1);
   if (F.bands > kMaxBands) return false;
-  F.th = (D->height + F.bands - 1) / F.bands;
-  F.bands = (D->height + F.th - 1) / F.th;
-  P.lds = (size_t)8 * ((F.th * F.W + 1) & ~1) + rest;
+  // A batch that leaves CUs without a workgroup runs workgroups of twice the
+  // waves and, while CUs are left, more bands.  Kernel time in us (8 waves /
+  // 16 / 16 and bands): 64 scenes of 84 x 84 with up to 256 instances 99 / 68 /
+  // 50, of 128 x 128 with 64 boxes 26 / 26 / 18, of 64 x 64 steering 50 / 47 /
+  // 45; 512 steering scenes in one workgroup per CU at a time 96, not 73.
+  const int64_t n = D->num_scenes;
+  if (n * F.bands <= kWideItems) {
+    const int wide = (int)((2 * kBandLds - stat - rest(kWideWaves)) / 8);
+    int bands = 1;
+    while (bands < kMaxBands && 2 * n * bands <= kWideItems && D->height / bands >= 16) bands *= 2;
+    split(kWideWaves, std::min(wide, 2 * kBandPixels) / D->width, bands);
+  }
   return true;
 }
 
@@ -1206,7 +1209,7 @@ hipError_t launch_bands_t(const pbr_scene_desc* D, const pbr_frame_out* O, const
         (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k, dim3(grid), dim3(kBandBlock), P.lds, st, *D, *O, P.F, scene_off, order, hdr, lt,
+  hipLaunchKernelGGL(k, dim3(grid), dim3(P.F.waves * 64), P.lds, st, *D, *O, P.F, scene_off, order, hdr, lt,
                      bg);
   return hipGetLastError();
 }

@@ -11,6 +11,7 @@ import torch
 from pybatchrender import PBRConfig, PBRRenderer, _native, diff, workloads
 from pybatchrender.envs.cartpole import CartPoleConfig, CartPoleGroundRenderer, CartPoleRenderer
 from pybatchrender.envs.steering import SteeringConfig, SteeringRenderer
+from pybatchrender.renderer.mesh import Mesh
 from tests.test_gpu_parity import _bits, check_parity, ground_states
 
 pytestmark = pytest.mark.gpu
@@ -173,3 +174,63 @@ def test_gradients_from_unaligned_transforms(cuda):
     for a, b in zip(got[1:], want[1:]):
         # sums of float atomics in any order: a few hundred terms of 2^-24 each
         assert (a - b).abs().max() <= 2e-5 * b.abs().max() + 1e-30
+
+
+def _strip_mesh(verts: int, tris: int, gen) -> Mesh:
+    """A closed-looking blob of `tris` triangles on exactly `verts` vertices."""
+    pos = torch.nn.functional.normalize(torch.randn(verts, 3, generator=gen), dim=1)
+    tri = torch.stack([torch.randperm(verts, generator=gen)[:3] for _ in range(tris)])
+    tri[0] = torch.tensor([0, verts // 2, verts - 1])
+    return Mesh(pos.numpy(), pos.numpy(), tri.numpy())
+
+
+@pytest.mark.parametrize("verts,tris", [(3, 1), (64, 63), (65, 64), (136, 256), (137, 256),
+                                        (136, 257)])
+@pytest.mark.parametrize("flat", [False, True])
+def test_band_kernel_mesh_sizes(cuda, verts, tris, flat):
+    """Meshes on both sides of what a wave's vertex table and triangle queue
+    hold (beyond them the tile kernels draw), several instances a chunk."""
+    gen = torch.Generator("cpu").manual_seed(verts + tris)
+    n, k = 5, 7
+    mesh = _strip_mesh(verts, tris, gen)
+    if flat:
+        mesh.normals[:] = mesh.normals[:1]
+    r = PBRRenderer(PBRConfig(num_scenes=n, tile_resolution=(45, 37), device="cuda",
+                              kernel="tiles"))
+    node = r.add_node(mesh, instances_per_scene=k)
+    node.set_transforms(workloads.random_transforms(n * k, gen, pos_range=2.0,
+                                                    scale_range=(0.2, 1.5)))
+    node.set_colors(torch.rand(n * k, 4, generator=gen))
+    node.set_instance_counts(torch.tensor([k, 0, 3, 1, k]))
+    r.add_camera().set_positions_and_lookat(torch.tensor([0.0, -5.0, 1.0]), torch.zeros(3))
+    r.add_light()
+    r.setup_environment()
+    check_parity(r, f"{verts} vertices, {tris} triangles")
+
+
+@pytest.mark.parametrize("dtype", ["uint8", "bfloat16", "float32"])
+@pytest.mark.parametrize("n,res", [(3, (33, 130)), (64, (40, 64)), (256, (21, 9)), (257, (21, 9)),
+                                   (258, (20, 12)), (65, (128, 128))])
+def test_band_kernel_forms(cuda, n, res, dtype):
+    """Scene counts on both sides of the wide form and of its numbers of
+    bands, frames of odd and of whole groups of four pixels: smooth and flat
+    nodes, near-plane crossings of more triangles than the clip queue holds,
+    long triangles beyond the frame, empty scenes."""
+    gen = torch.Generator("cpu").manual_seed(n + res[0])
+    r = PBRRenderer(PBRConfig(num_scenes=n, tile_resolution=res, device="cuda", kernel="tiles",
+                              output_dtype=dtype))
+    for model, k, lo, hi in (("models/sphere", 3, 0.2, 1.0), ("models/cylinder", 3, 2.0, 9.0),
+                             ("models/box", 9, 0.1, 30.0)):
+        node = r.add_node(model, instances_per_scene=k)
+        node.set_transforms(workloads.random_transforms(n * k, gen, pos_range=2.5,
+                                                        scale_range=(lo, hi)))
+        node.set_colors(torch.rand(n * k, 4, generator=gen))
+        node.set_instance_counts(torch.randint(0, k + 1, (n,), generator=gen))
+    r.add_camera(z_near=0.4)
+    eye = torch.stack([torch.rand(n, generator=gen) * 4 - 2, torch.full((n,), -4.0),
+                       torch.rand(n, generator=gen) * 3], 1)
+    r._pbr_cam.set_positions_and_lookat(eye, torch.zeros(3))
+    r.add_light()
+    r.setup_environment()
+    check_parity(r, f"band form n={n} {res} {dtype}")
+    check_parity(r, f"band form n={n} {res} {dtype}, colour only", depth=False, vis=False)
