@@ -45,6 +45,7 @@ constexpr int kBandTable = 512;   // triangles of all meshes (LDS index table) a
 constexpr int kMaxBands = 4;      // bands per scene at most: each repeats the vertex work
 constexpr int kBandPixels = 8192;
 constexpr int kBandLds = 80 * 1024;  // half a CU's LDS: two workgroups share a CU
+constexpr int kClipQueue = 128;   // clipped triangles that wait for the whole workgroup
 constexpr int kSmallPixels = 12;  // box pixels one lane rasterises alone
 constexpr uint32_t kDepthOne = 0x3f800000u;
 // Sub-triangle number of a triangle that no plane clips (a clipped polygon has
@@ -598,7 +599,8 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
                                                           const uint32_t* order, uint32_t* hdr, Light lt, float4 bg) {
   extern __shared__ __align__(16) unsigned long long pix[];
   __shared__ NodeLds nodes[PBR_MAX_NODES];
-  __shared__ uint32_t next_chunk, total_chunks, covered_n;
+  __shared__ uint32_t next_chunk, total_chunks, covered_n, clip_total;
+  __shared__ uint32_t clip_queue[kClipQueue];
   const int tid = (int)threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = F.W, H = F.H, nn = D.num_nodes;
@@ -669,6 +671,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     if (lane == 63) {
       next_chunk = 0u;
       covered_n = 0u;
+      clip_total = 0u;
       total_chunks = ic;
     }
   }
@@ -679,6 +682,52 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
 
   // --- setup and raster --------------------------------------------------------
   const uint32_t chunks = __builtin_amdgcn_readfirstlane((int)total_chunks);
+  // set-up triangles of the lanes (`has`) into the band's pixels
+  auto draw = [&](bool has, const FixTri& T, uint32_t rank) {
+    const bool fits =  // edge values fit 32 bits
+        has &&
+        max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
+        max(T.Y[0], max(T.Y[1], T.Y[2])) - min(T.Y[0], min(T.Y[1], T.Y[2])) <= kIntExtent;
+    const int w = T.i1 - T.i0 + 1, h = T.j1 - T.j0 + 1;
+    const bool small = fits && w * h <= kSmallPixels;
+    if (small) band_raster_lane(pix, t, T, rank);
+    const bool rows = fits && !small;
+    if (__ballot(rows)) band_raster_rows<int32_t>(pix, t, lane, rows, T, rank);
+    const bool far = has && !fits;
+    if (__ballot(far)) band_raster_rows<double>(pix, t, lane, far, T, rank);
+  };
+  // four triangles that straddle a clip plane, one per group of 16 lanes, a
+  // lane per sub-triangle
+  auto draw_clipped = [&](uint32_t slot, bool some) {
+    FixTri T;
+    CVert cv = {};
+    int pn = some ? 3 : 0;
+    if (some && (lane & 15) < 3) {
+      const SlotRef R = band_slot(t.s, nodes, nn, tab, slot);
+      group_vertex(D, R.trans, R.row, R.voff, R.tri, VP, lane, cv);
+    }
+    clip_groups<4>(cv.p, pn, F.guard, lane);
+    SnapVert S;
+    snap_vertex(cv, W, H, S);
+    const int lost = 0x7fffffff;  // X of a vertex that did not snap
+    const int X = S.ok ? S.X : lost;
+    const int at = lane & 48, q = lane & 15;
+    const bool sub = q + 2 < pn;
+    const int f1 = sub ? at + q + 1 : at, f2 = sub ? at + q + 2 : at;
+    SnapVert V[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      const int f = e == 0 ? at : (e == 1 ? f1 : f2);
+      V[e].X = from_lane(f, X);
+      V[e].Y = from_lane(f, S.Y);
+      V[e].d = from_lane(f, S.d);
+      V[e].invw = 0.0f;
+      V[e].ok = V[e].X != lost;
+    }
+    const bool has = sub && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
+    const uint32_t rank = (slot << 3) | (uint32_t)q;
+    draw(has, T, rank);
+  };
   for (;;) {
     uint32_t c = 0;
     if (lane == 0) c = atomicAdd(&next_chunk, 1u);
@@ -807,22 +856,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
     }
     wave_fence();
 
-    // set-up triangles of the lanes (`has`) into the band's pixels
-    auto draw = [&](bool has, const FixTri& T, uint32_t rank) {
-      const bool fits =  // edge values fit 32 bits
-          has &&
-          max(T.X[0], max(T.X[1], T.X[2])) - min(T.X[0], min(T.X[1], T.X[2])) <= kIntExtent &&
-          max(T.Y[0], max(T.Y[1], T.Y[2])) - min(T.Y[0], min(T.Y[1], T.Y[2])) <= kIntExtent;
-      const int w = T.i1 - T.i0 + 1, h = T.j1 - T.j0 + 1;
-      const bool small = fits && w * h <= kSmallPixels;
-      if (small) band_raster_lane(pix, t, T, rank);
-      const bool rows = fits && !small;
-      if (__ballot(rows)) band_raster_rows<int32_t>(pix, t, lane, rows, T, rank);
-      const bool far = has && !fits;
-      if (__ballot(far)) band_raster_rows<double>(pix, t, lane, far, T, rank);
-    };
-    // 64 live triangles are set up at a time, then clipped ones four at a time
-    // (a lane per sub-triangle); each set is rasterised at once
+    // 64 live triangles are set up at a time and rasterised at once
     for (uint32_t k0 = 0; k0 < live_n; k0 += 64u) {
       FixTri T;
       bool has = false;
@@ -845,41 +879,33 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       }
       draw(has, T, rank);
     }
-    for (uint32_t k0 = 0; k0 < clip_n; k0 += 4u) {
-      FixTri T;
-      const uint32_t k = k0 + (uint32_t)(lane >> 4);
-      int pn = k < clip_n ? 3 : 0;
-      const uint32_t u = qu[kBandTris - 1u - min(k, clip_n - 1u)];
-      CVert cv = {};
-      if (pn && (lane & 15) < 3) {
-        const uint32_t di = __umul24(u, inv_nt) >> 16;
-        group_vertex(D, trans, row0 + di, voff, mtab[u - __umul24(di, nt)], VP, lane, cv);
+    // clipped ones go to the workgroup's queue, so that a mesh which crosses
+    // the near plane does not keep one wave while the others run out of
+    // chunks; what does not fit is drawn at once
+    if (clip_n) {
+      uint32_t first = 0;
+      if (lane == 0) first = atomicAdd(&clip_total, clip_n);
+      first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+      const uint32_t room = first < (uint32_t)kClipQueue ? kClipQueue - first : 0u;
+      for (uint32_t k = (uint32_t)lane; k < min(clip_n, room); k += 64u)
+        clip_queue[first + k] = slot0 + qu[kBandTris - 1u - k];
+      for (uint32_t k0 = room; k0 < clip_n; k0 += 4u) {
+        const uint32_t k = k0 + (uint32_t)(lane >> 4);
+        draw_clipped(slot0 + qu[kBandTris - 1u - min(k, clip_n - 1u)], k < clip_n);
       }
-      clip_groups<4>(cv.p, pn, F.guard, lane);
-      SnapVert S;
-      snap_vertex(cv, W, H, S);
-      const int lost = 0x7fffffff;  // X of a vertex that did not snap
-      const int X = S.ok ? S.X : lost;
-      const int at = lane & 48, q = lane & 15;
-      const bool sub = q + 2 < pn;
-      const int f1 = sub ? at + q + 1 : at, f2 = sub ? at + q + 2 : at;
-      SnapVert V[3];
-#pragma unroll
-      for (int e = 0; e < 3; ++e) {
-        const int f = e == 0 ? at : (e == 1 ? f1 : f2);
-        V[e].X = from_lane(f, X);
-        V[e].Y = from_lane(f, S.Y);
-        V[e].d = from_lane(f, S.d);
-        V[e].invw = 0.0f;
-        V[e].ok = V[e].X != lost;
-      }
-      const bool has = sub && setup_snapped(V[0], V[1], V[2], W, H, t.j0, t.j1, T);
-      const uint32_t rank = ((slot0 + u) << 3) | (uint32_t)q;
-      draw(has, T, rank);
     }
     wave_fence();  // the next chunk rewrites the table
   }
   __syncthreads();
+  const uint32_t clips =
+      min((uint32_t)__builtin_amdgcn_readfirstlane((int)clip_total), (uint32_t)kClipQueue);
+  if (clips) {
+    for (uint32_t k0 = (uint32_t)wave * 4u; k0 < clips; k0 += (uint32_t)waves * 4u) {
+      const uint32_t k = k0 + (uint32_t)(lane >> 4);
+      draw_clipped(clip_queue[min(k, clips - 1u)], k < clips);
+    }
+    __syncthreads();
+  }
 
   // --- resolve -----------------------------------------------------------------
   const int C = O.channels;
@@ -1169,7 +1195,7 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   F.verts = verts;
   if (ntab > kBandTable) return false;
   F.ntab = ntab;
-  const size_t stat = sizeof(NodeLds) * PBR_MAX_NODES + 64;
+  const size_t stat = sizeof(NodeLds) * PBR_MAX_NODES + 4 * kClipQueue + 64;
   const auto rest = [&](int waves) {
     return (size_t)waves * ((size_t)verts * 12 + kBandTris) + 4 * (size_t)ntab;
   };
