@@ -941,13 +941,13 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
 #pragma unroll
         for (int k = 0; k < 4; ++k)
           z[k] = (cov >> k) & 1u ? __uint_as_float((uint32_t)(key[k] >> 32)) : 1.0f;
-        *reinterpret_cast<float4*>(dep + p) = make_float4(z[0], z[1], z[2], z[3]);
+        store_stream(dep + p, make_float4(z[0], z[1], z[2], z[3]));
       }
       if (vis) {
         int v[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = (cov >> k) & 1u ? (int)((uint32_t)key[k] >> 3) : -1;
-        *reinterpret_cast<int4*>(vis + p) = make_int4(v[0], v[1], v[2], v[3]);
+        store_stream(vis + p, make_int4(v[0], v[1], v[2], v[3]));
       }
       if constexpr (OM == 1) {
 #pragma unroll
@@ -956,8 +956,8 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
       } else if constexpr (OM == 2) {
         if (cov == 0u) {
           for (int ch = 0; ch < C; ++ch)
-            *reinterpret_cast<float4*>(fout + (size_t)ch * plane + p) =
-                make_float4(bgc[ch], bgc[ch], bgc[ch], bgc[ch]);
+            store_stream(fout + (size_t)ch * plane + p,
+                         make_float4(bgc[ch], bgc[ch], bgc[ch], bgc[ch]));
         } else if (cov != 15u) {
           for (int ch = 0; ch < C; ++ch)
 #pragma unroll
@@ -1110,13 +1110,13 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
 #pragma unroll 1
       for (int ch = 0; ch < C; ++ch) {
         if constexpr (OM == 0) {
-          *reinterpret_cast<uint32_t*>(dst + (size_t)ch * plane) =
-              band_gather((uint32_t)v0, (uint32_t)v1, (uint32_t)v2, (uint32_t)v3, ch);
+          store_stream(dst + (size_t)ch * plane,
+                       band_gather((uint32_t)v0, (uint32_t)v1, (uint32_t)v2, (uint32_t)v3, ch));
         } else {
           const int sh = 16 * ch;
-          *reinterpret_cast<uint2*>(dst + (size_t)ch * plane * 2) = make_uint2(
-              ((uint32_t)(v0 >> sh) & 0xffffu) | ((uint32_t)(v1 >> sh) << 16),
-              ((uint32_t)(v2 >> sh) & 0xffffu) | ((uint32_t)(v3 >> sh) << 16));
+          store_stream(dst + (size_t)ch * plane * 2,
+                       make_uint2(((uint32_t)(v0 >> sh) & 0xffffu) | ((uint32_t)(v1 >> sh) << 16),
+                                  ((uint32_t)(v2 >> sh) & 0xffffu) | ((uint32_t)(v3 >> sh) << 16)));
         }
       }
     }
@@ -1140,7 +1140,7 @@ __attribute__((amdgpu_waves_per_eu(4))) void bands_kernel(pbr_scene_desc D, pbr_
           v = ((uint32_t)(pix[p] >> (16 * ch)) & 0xffffu) |
               ((uint32_t)(pix[p + 1] >> (16 * ch)) << 16);
         }
-        *reinterpret_cast<uint32_t*>(dst + (size_t)p * ES) = v;
+        store_stream(dst + (size_t)p * ES, v);
       } else {
 #pragma unroll
         for (int b = 0; b < PER; ++b) {

@@ -490,6 +490,33 @@ __device__ __forceinline__ void load_mat4(const float* src, float M[16]) {
   M[12] = d.x; M[13] = d.y; M[14] = d.z; M[15] = d.w;
 }
 
+// Stores of a frame in whole pieces of 4, 8 or 16 bytes at any address (global
+// stores of any width take any byte address in the unaligned access mode that
+// ROCm runs compute with), past the caches: no lane reads a frame back, and
+// its dirty lines make later kernels wait.  Ordinary / streaming stores, us
+// per call with two frames in turn: 1024 scenes of 128 x 128 float32 + depth
+// 134 / 109, 8192 of 84 x 84 uint8 560 / 533, 16384 of 64 x 64 bf16 + depth
+// 155 / 149, 4096 uint8 26.5 / 24.6.  Single pixels that a lane scatters
+// (float colours of the band path) stay ordinary: they meet their line's other
+// pixels in the cache (1024 scenes: 212 with streaming stores).
+template <int N> struct StreamWord;
+template <> struct StreamWord<4> {
+  typedef uint32_t T __attribute__((aligned(1)));
+};
+template <> struct StreamWord<8> {
+  typedef uint32_t T __attribute__((ext_vector_type(2), aligned(1)));
+};
+template <> struct StreamWord<16> {
+  typedef uint32_t T __attribute__((ext_vector_type(4), aligned(1)));
+};
+template <typename T, typename E>
+__device__ __forceinline__ void store_stream(E* dst, const T& v) {
+  typedef typename StreamWord<sizeof(T)>::T W;
+  W w;
+  __builtin_memcpy(&w, &v, sizeof(T));
+  __builtin_nontemporal_store(w, reinterpret_cast<W*>(dst));
+}
+
 // Sixteen floats at a wave-uniform address that nothing in the launch writes,
 // by scalar loads.
 typedef const __attribute__((address_space(4))) float const_float;

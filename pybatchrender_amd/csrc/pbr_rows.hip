@@ -868,14 +868,6 @@ __device__ __forceinline__ uint32_t gather_byte(uint32_t p0, uint32_t p1, uint32
   return __builtin_amdgcn_perm(t23, t01, 0x05040100u);
 }
 
-// One store of T at an address aligned only to its elements (global stores
-// of any width take any byte address in the unaligned access mode that
-// ROCm runs compute with; the compiler picks the instruction from the copy).
-template <typename T, typename E>
-__device__ __forceinline__ void store_at(E* dst, const T& v) {
-  __builtin_memcpy(dst, &v, sizeof(T));
-}
-
 // The output planes of one scene: every offset within them fits 32 bits.
 struct SceneOut {
   void* color;     // [C][H][W] of the output dtype
@@ -930,7 +922,7 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
       for (int c = 0; c < so.C; ++c, dst += so.plane) {
 #pragma unroll
         for (int h = 0; h < PXL; h += 4)
-          store_at(dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
+          store_stream(dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
       }
     } else if constexpr (OM == 1) {
       uint16_t* dst = reinterpret_cast<uint16_t*>(so.color);
@@ -939,10 +931,13 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
         if (c >= so.C) break;
         const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
 #pragma unroll
-        for (int h = 0; h < PXL; h += 2) {
-          const uint32_t a = (c < 2) ? cv[h].x : cv[h].y;
-          const uint32_t b = (c < 2) ? cv[h + 1].x : cv[h + 1].y;
-          store_at(dst + (size_t)c * so.plane + pix0 + h, __builtin_amdgcn_perm(b, a, sel));
+        for (int h = 0; h < PXL; h += 4) {
+          uint32_t v[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] = (c < 2) ? cv[h + k].x : cv[h + k].y;
+          store_stream(dst + (size_t)c * so.plane + pix0 + h,
+                       make_uint2(__builtin_amdgcn_perm(v[1], v[0], sel),
+                                  __builtin_amdgcn_perm(v[3], v[2], sel)));
         }
       }
     } else {
@@ -956,14 +951,14 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
 #pragma unroll
           for (int k = 0; k < 4; ++k)
             v[k] = c == 0 ? cv[h + k].x : (c == 1 ? cv[h + k].y : (c == 2 ? cv[h + k].z : cv[h + k].w));
-          store_at(dst + (size_t)c * so.plane + pix0 + h, make_float4(v[0], v[1], v[2], v[3]));
+          store_stream(dst + (size_t)c * so.plane + pix0 + h, make_float4(v[0], v[1], v[2], v[3]));
         }
       }
     }
     if (so.depth) {
 #pragma unroll
       for (int h = 0; h < PXL; h += 4)
-        store_at(so.depth + pix0 + h, make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f,
+        store_stream(so.depth + pix0 + h, make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f,
                                                   S.z[h + 2] + 0.0f, S.z[h + 3] + 0.0f));
     }
     if (so.vis) {
@@ -972,7 +967,7 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
       for (int i = 0; i < PXL; ++i) v[i] = S.z[i] < 1.0f ? (int32_t)(S.ref[i] >> 3) : -1;
 #pragma unroll
       for (int h = 0; h < PXL; h += 4)
-        store_at(so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
+        store_stream(so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
     }
     return;
   }
