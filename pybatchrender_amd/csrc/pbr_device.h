@@ -490,15 +490,15 @@ __device__ __forceinline__ void load_mat4(const float* src, float M[16]) {
   M[12] = d.x; M[13] = d.y; M[14] = d.z; M[15] = d.w;
 }
 
-// Stores of a frame in whole pieces of 4, 8 or 16 bytes at any address (global
-// stores of any width take any byte address in the unaligned access mode that
-// ROCm runs compute with), past the caches: no lane reads a frame back, and
-// its dirty lines make later kernels wait.  Ordinary / streaming stores, us
-// per call with two frames in turn: 1024 scenes of 128 x 128 float32 + depth
-// 134 / 109, 8192 of 84 x 84 uint8 560 / 533, 16384 of 64 x 64 bf16 + depth
-// 155 / 149, 4096 uint8 26.5 / 24.6.  Single pixels that a lane scatters
-// (float colours of the band path) stay ordinary: they meet their line's other
-// pixels in the cache (1024 scenes: 212 with streaming stores).
+// A store of 4, 8 or 16 bytes at any address (global stores of any width take
+// any byte address in the unaligned access mode that ROCm runs compute with),
+// past the caches: for frames, which no lane reads back and whose dirty lines
+// make later kernels wait.  Ordinary / streaming, us per call with two frames
+// in turn: 1024 scenes of 128 x 128 float32 + depth (band path) 134 / 109,
+// 8192 of 84 x 84 uint8 560 / 533, 4096 of 64 x 64 uint8 (row-span kernel)
+// 26.5 / 24.6.  Only for stores in which a wave writes one contiguous piece:
+// lines that several stores fill, each at its own time, are better put
+// together in the cache (single pixels that lanes scatter: 1024 scenes 212).
 template <int N> struct StreamWord;
 template <> struct StreamWord<4> {
   typedef uint32_t T __attribute__((aligned(1)));

@@ -71,6 +71,7 @@ struct RowsFrame {
   int seg;  // setup lanes per scene (power of two >= slots, <= 64)
   int cap;  // row-list entries per band (8..kCap)
   int vphase;  // 1: vertices transformed once into an LDS table (they fit)
+  int stream;  // 1: frame stores are streaming (see launch_rows)
 };
 
 // Instance poses a launch applies itself (pbr_render_posed).  Pose d[k]
@@ -868,6 +869,17 @@ __device__ __forceinline__ uint32_t gather_byte(uint32_t p0, uint32_t p1, uint32
   return __builtin_amdgcn_perm(t23, t01, 0x05040100u);
 }
 
+// A store of the frame, streaming (store_stream) in frames where a wave's store
+// covers whole cache lines: RowsFrame::stream, never with eight pixels a lane
+// (each store instruction writes every second half then).
+template <int PXL, typename T, typename E>
+__device__ __forceinline__ void store_frame(int stream, E* dst, const T& v) {
+  if (PXL == 4 && stream)
+    store_stream(dst, v);
+  else
+    __builtin_memcpy(dst, &v, sizeof(T));
+}
+
 // The output planes of one scene: every offset within them fits 32 bits.
 struct SceneOut {
   void* color;     // [C][H][W] of the output dtype
@@ -922,7 +934,7 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
       for (int c = 0; c < so.C; ++c, dst += so.plane) {
 #pragma unroll
         for (int h = 0; h < PXL; h += 4)
-          store_stream(dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
+          store_frame<PXL>(F.stream, dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
       }
     } else if constexpr (OM == 1) {
       uint16_t* dst = reinterpret_cast<uint16_t*>(so.color);
@@ -935,7 +947,7 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
           uint32_t v[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k) v[k] = (c < 2) ? cv[h + k].x : cv[h + k].y;
-          store_stream(dst + (size_t)c * so.plane + pix0 + h,
+          store_frame<PXL>(F.stream, dst + (size_t)c * so.plane + pix0 + h,
                        make_uint2(__builtin_amdgcn_perm(v[1], v[0], sel),
                                   __builtin_amdgcn_perm(v[3], v[2], sel)));
         }
@@ -951,14 +963,14 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
 #pragma unroll
           for (int k = 0; k < 4; ++k)
             v[k] = c == 0 ? cv[h + k].x : (c == 1 ? cv[h + k].y : (c == 2 ? cv[h + k].z : cv[h + k].w));
-          store_stream(dst + (size_t)c * so.plane + pix0 + h, make_float4(v[0], v[1], v[2], v[3]));
+          store_frame<PXL>(F.stream, dst + (size_t)c * so.plane + pix0 + h, make_float4(v[0], v[1], v[2], v[3]));
         }
       }
     }
     if (so.depth) {
 #pragma unroll
       for (int h = 0; h < PXL; h += 4)
-        store_stream(so.depth + pix0 + h, make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f,
+        store_frame<PXL>(F.stream, so.depth + pix0 + h, make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f,
                                                   S.z[h + 2] + 0.0f, S.z[h + 3] + 0.0f));
     }
     if (so.vis) {
@@ -967,7 +979,7 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
       for (int i = 0; i < PXL; ++i) v[i] = S.z[i] < 1.0f ? (int32_t)(S.ref[i] >> 3) : -1;
 #pragma unroll
       for (int h = 0; h < PXL; h += 4)
-        store_stream(so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
+        store_frame<PXL>(F.stream, so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
     }
     return;
   }
@@ -1430,6 +1442,13 @@ int launch_rows(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rende
   const bool small = rows_small(D);
   F.cap = cap ? cap : kCap;
   F.vphase = rows_vphase(D) ? 1 : 0;
+  // A wave stores four rows of at most 64 columns, one piece of 4 W pixels.
+  // Streaming stores pay where the pieces are whole 128-byte lines and cost
+  // where they cut lines (us per call, ordinary / streaming: 4096 scenes of 64
+  // x 64 uint8 26.5 / 24.6, float32 + depth 72 / 66; of 47 x 64 63 / 76; of
+  // 84 x 84 128 / 266).
+  const int elem = O->dtype == PBR_DTYPE_U8 ? 1 : (O->dtype == PBR_DTYPE_BF16 ? 2 : 4);
+  F.stream = D->width <= 64 && (4 * D->width * elem) % 128 == 0 ? 1 : 0;
   const Light lt = host_light(D);
   const float4 bg = make_float4(D->background[0], D->background[1], D->background[2],
                                 D->background[3]);
