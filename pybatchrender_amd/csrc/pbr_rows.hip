@@ -869,12 +869,10 @@ __device__ __forceinline__ uint32_t gather_byte(uint32_t p0, uint32_t p1, uint32
   return __builtin_amdgcn_perm(t23, t01, 0x05040100u);
 }
 
-// A store of the frame, streaming (store_stream) in frames where a wave's store
-// covers whole cache lines: RowsFrame::stream, never with eight pixels a lane
-// (each store instruction writes every second half then).
-template <int PXL, typename T, typename E>
-__device__ __forceinline__ void store_frame(int stream, E* dst, const T& v) {
-  if (PXL == 4 && stream)
+// A store of the frame, streaming (store_stream) or ordinary.
+template <bool STREAM, typename T, typename E>
+__device__ __forceinline__ void store_frame(E* dst, const T& v) {
+  if constexpr (STREAM)
     store_stream(dst, v);
   else
     __builtin_memcpy(dst, &v, sizeof(T));
@@ -900,6 +898,72 @@ __device__ __forceinline__ int lane_x0(int lane, int W) {
   return W >= PXL ? min(x, W - PXL) : x;
 }
 
+// Stores a lane's whole pixels (lane_x0), the first of them pix0 of the planes:
+// one dword (or wider) store per channel, whatever the row's alignment.
+template <int OM, int PXL, bool STREAM>
+__device__ __forceinline__ void store_lane(const SceneOut& so, uint32_t pix0,
+                                           const typename ColOf<OM>::T* cv,
+                                           const PixState<PXL>& S) {
+  if constexpr (OM == 0) {
+    // a uniform loop over the channels (its counter and byte selector stay
+    // scalar; unrolled, the per-channel conditions were kept in spilled
+    // scalar registers)
+    uint8_t* dst = reinterpret_cast<uint8_t*>(so.color) + pix0;
+#pragma unroll 1
+    for (int c = 0; c < so.C; ++c, dst += so.plane) {
+#pragma unroll
+      for (int h = 0; h < PXL; h += 4)
+        store_frame<STREAM>(dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
+    }
+  } else if constexpr (OM == 1) {
+    uint16_t* dst = reinterpret_cast<uint16_t*>(so.color);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (c >= so.C) break;
+      const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+      for (int h = 0; h < PXL; h += 4) {
+        uint32_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = (c < 2) ? cv[h + k].x : cv[h + k].y;
+        store_frame<STREAM>(dst + (size_t)c * so.plane + pix0 + h,
+                            make_uint2(__builtin_amdgcn_perm(v[1], v[0], sel),
+                                       __builtin_amdgcn_perm(v[3], v[2], sel)));
+      }
+    }
+  } else {
+    float* dst = reinterpret_cast<float*>(so.color);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (c >= so.C) break;
+#pragma unroll
+      for (int h = 0; h < PXL; h += 4) {
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          v[k] = c == 0 ? cv[h + k].x : (c == 1 ? cv[h + k].y : (c == 2 ? cv[h + k].z : cv[h + k].w));
+        store_frame<STREAM>(dst + (size_t)c * so.plane + pix0 + h,
+                            make_float4(v[0], v[1], v[2], v[3]));
+      }
+    }
+  }
+  if (so.depth) {
+#pragma unroll
+    for (int h = 0; h < PXL; h += 4)
+      store_frame<STREAM>(so.depth + pix0 + h,
+                          make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f, S.z[h + 2] + 0.0f,
+                                      S.z[h + 3] + 0.0f));
+  }
+  if (so.vis) {
+    int32_t v[PXL];
+#pragma unroll
+    for (int i = 0; i < PXL; ++i) v[i] = S.z[i] < 1.0f ? (int32_t)(S.ref[i] >> 3) : -1;
+#pragma unroll
+    for (int h = 0; h < PXL; h += 4)
+      store_frame<STREAM>(so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
+  }
+}
+
 // Writes the lane's PXL pixels of GL row j (x0 .. x0 + PXL - 1, those < W).
 template <bool SMOOTH, int OM, int PXL, int RECS>
 __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const SceneOut& so,
@@ -923,64 +987,12 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
     }
   }
   if (F.W >= PXL) {
-    // whole lane pixels (lane_x0): one dword (or wider) store per channel,
-    // whatever the row's alignment
-    if constexpr (OM == 0) {
-      // a uniform loop over the channels (its counter and byte selector stay
-      // scalar; unrolled, the per-channel conditions were kept in spilled
-      // scalar registers)
-      uint8_t* dst = reinterpret_cast<uint8_t*>(so.color) + pix0;
-#pragma unroll 1
-      for (int c = 0; c < so.C; ++c, dst += so.plane) {
-#pragma unroll
-        for (int h = 0; h < PXL; h += 4)
-          store_frame<PXL>(F.stream, dst + h, gather_byte(cv[h], cv[h + 1], cv[h + 2], cv[h + 3], c));
-      }
-    } else if constexpr (OM == 1) {
-      uint16_t* dst = reinterpret_cast<uint16_t*>(so.color);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c >= so.C) break;
-        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
-#pragma unroll
-        for (int h = 0; h < PXL; h += 4) {
-          uint32_t v[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) v[k] = (c < 2) ? cv[h + k].x : cv[h + k].y;
-          store_frame<PXL>(F.stream, dst + (size_t)c * so.plane + pix0 + h,
-                       make_uint2(__builtin_amdgcn_perm(v[1], v[0], sel),
-                                  __builtin_amdgcn_perm(v[3], v[2], sel)));
-        }
-      }
-    } else {
-      float* dst = reinterpret_cast<float*>(so.color);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c >= so.C) break;
-#pragma unroll
-        for (int h = 0; h < PXL; h += 4) {
-          float v[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            v[k] = c == 0 ? cv[h + k].x : (c == 1 ? cv[h + k].y : (c == 2 ? cv[h + k].z : cv[h + k].w));
-          store_frame<PXL>(F.stream, dst + (size_t)c * so.plane + pix0 + h, make_float4(v[0], v[1], v[2], v[3]));
-        }
-      }
-    }
-    if (so.depth) {
-#pragma unroll
-      for (int h = 0; h < PXL; h += 4)
-        store_frame<PXL>(F.stream, so.depth + pix0 + h, make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f,
-                                                  S.z[h + 2] + 0.0f, S.z[h + 3] + 0.0f));
-    }
-    if (so.vis) {
-      int32_t v[PXL];
-#pragma unroll
-      for (int i = 0; i < PXL; ++i) v[i] = S.z[i] < 1.0f ? (int32_t)(S.ref[i] >> 3) : -1;
-#pragma unroll
-      for (int h = 0; h < PXL; h += 4)
-        store_frame<PXL>(F.stream, so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
-    }
+    // never streaming with eight pixels a lane: each store instruction writes
+    // every second half then
+    if (PXL == 4 && F.stream)
+      store_lane<OM, PXL, true>(so, pix0, cv, S);
+    else
+      store_lane<OM, PXL, false>(so, pix0, cv, S);
     return;
   }
   // a tile narrower than a lane: pixel by pixel
