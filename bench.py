@@ -468,7 +468,7 @@ def render_kernel_name(r) -> str:
 
 KERNEL_LABEL = {"rows": "rows_kernel (setup + lists + row walk, one launch)",
                 "scene": "setup_kernel + raster_kernel",
-                "tiles": "tile_prep_kernel + tile_setup_kernel + tile_raster_kernel",
+                "tiles": "bands_kernel (after tile_prep_kernel with instance counts)",
                 "chunked": "chunked_kernel"}
 
 

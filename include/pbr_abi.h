@@ -122,14 +122,18 @@ enum pbr_kernel {
 
 typedef struct pbr_render_opts {
   int32_t region_rows;        /* chunked: output rows per work item (x8)    */
-  int32_t persistent;         /* chunked, tiles: persistent work queue      */
+  int32_t persistent;         /* chunked, tiles with a tile_size or a
+                                 bin_capacity: persistent work queue        */
   int32_t workgroups;         /* persistent launch size, 0 = 8 per CU       */
   int32_t kernel;             /* enum pbr_kernel                            */
   int32_t bin_width;          /* scene: 16, 32 or 64 pixel-wide bins        */
   int32_t bins_per_item;      /* scene: bins one work item walks, 0 = auto  */
   int32_t lane_pixels;        /* scene: 4 or 8 pixels per lane, 0 = auto    */
   int32_t tile_size;          /* tiles: 8, 16, 32 or 64 pixel square tiles,
-                                 0 = full-width bands of <= 8192 pixels     */
+                                 0 = full-width bands; with bin_capacity 0
+                                 too and meshes of at most 136 vertices and
+                                 256 triangles these are drawn straight from
+                                 the instances, without records             */
   int64_t slot_budget;        /* tiles: upper bound of the batch's triangle
                                  slots (sum over scenes of active instances
                                  x triangles); 0 = num_scenes x the largest

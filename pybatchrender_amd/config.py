@@ -10,7 +10,8 @@ New fields (defaults keep the reference's behaviour):
     output_dtype   'uint8' (reference), 'bfloat16' or 'float32' colour output
     output_depth   also produce a [N, H, W] float32 window-depth tensor
     region_rows    chunked kernel: output rows per work item (0 = automatic)
-    persistent     chunked kernel over a persistent (scene, region) work queue
+    persistent     chunked kernel over a persistent (scene, region) work queue,
+                   tile kernels with a tile_size or bin_capacity likewise
     kernel         'auto', 'rows' (setup and exact per-row spans in one
                    launch: at most 64 triangle slots per scene and tiles at
                    most 128 pixels wide), 'scene' (one wave per scene, at most
@@ -18,7 +19,9 @@ New fields (defaults keep the reference's behaviour):
                    one setup pass, then one workgroup per scene tile) or
                    'chunked' (any triangle count, setup repeated per row strip)
     tile_size      tile kernels: 8, 16, 32 or 64 pixel square tiles (0 =
-                   full-width bands of at most 8192 pixels)
+                   full-width bands; with bin_capacity 0 and meshes of at most
+                   136 vertices and 256 triangles each band is drawn straight
+                   from the scene's instances)
     bin_capacity   tile kernels: entries of each LDS bin of a tile before it
                    is rasterised and emptied, 1024..16384 (0 = 1904)
     row_list_cap   rows kernel: row-list entries per band, 8..256 (0 = 256)

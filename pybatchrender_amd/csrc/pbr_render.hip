@@ -1216,7 +1216,8 @@ int pbr_copy_segments(const pbr_segment* segments, int32_t count, void* stream) 
   int64_t most = 0;
   for (int k = 0; k < count; ++k) {
     const pbr_segment& g = segments[k];
-    if (g.bytes < 0 || (g.bytes & 3)) return fail(PBR_ERR_INVALID, "segment %d: size not a multiple of 4", k);
+    if (g.bytes < 0 || (g.bytes & 3))
+      return fail(PBR_ERR_INVALID, "segment %d: size not a multiple of 4", k);
     if (g.bytes == 0) continue;
     if (!g.dst || (((uintptr_t)g.dst | (uintptr_t)g.src) & 3))
       return fail(PBR_ERR_INVALID, "segment %d: pointers must be 4-byte aligned", k);

@@ -1,5 +1,7 @@
 // pbr_tiles.hip - the tile path: any triangle count per scene, each triangle
-// set up exactly once.
+// set up exactly once.  Launches at default tile options whose meshes fit go
+// to the band path instead (pbr_bands.hip), after tile_prep_kernel if there
+// are instance counts.
 //
 //   tile_prep_kernel    zeroes the per-scene visible counts and the work
 //                       queue; with per-scene instance counts, the
