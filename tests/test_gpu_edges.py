@@ -1,7 +1,7 @@
-"""Edge sizes of the row-span and band kernels, bit for bit against the oracle.
+"""Edge sizes of the row-span, band, backward, steering and copy kernels.
 
-Both kernels repeat the oracle's operations in its order, so the tolerance is
-zero for every output.
+Frames repeat the oracle's operations in its order, so their tolerance is
+zero; gradients are held to bounds of their float32 sums.
 """
 from __future__ import annotations
 
@@ -234,3 +234,42 @@ def test_band_kernel_forms(cuda, n, res, dtype):
     r.setup_environment()
     check_parity(r, f"band form n={n} {res} {dtype}")
     check_parity(r, f"band form n={n} {res} {dtype}, colour only", depth=False, vis=False)
+
+
+@pytest.mark.parametrize("res,spheres", [((7, 40), 1), ((50, 17), 3), ((130, 33), 3),
+                                         ((300, 16), 2), ((1000, 9), 2), ((64, 15), 8)])
+def test_smooth_backward_pixel_sums(cuda, res, spheres):
+    """The sorted smooth backward where a row is no whole run of eight pixels,
+    a band takes several chunks of runs, the last band is short, and the
+    visible slots take one pass or several.  Unlit, an instance's colour
+    gradient is the sum of the output gradient over its pixels, so every
+    pixel has to reach its own slot; a float32 sum of n terms in any order is
+    within n 2^-24 of the sum of their magnitudes."""
+    gen = torch.Generator("cpu").manual_seed(res[0])
+    n, (W, H) = 2, res
+    r = PBRRenderer(PBRConfig(num_scenes=n, tile_resolution=res, device="cuda",
+                              output_dtype="float32"))
+    counts = (2, spheres)
+    for model, k in zip(("models/box", "models/sphere"), counts):
+        node = r.add_node(model, instances_per_scene=k)
+        node.set_transforms(workloads.random_transforms(n * k, gen, pos_range=1.2,
+                                                        scale_range=(0.5, 1.2)))
+        node.set_colors(torch.rand(n * k, 4, generator=gen))
+    r.add_camera().set_positions_and_lookat(torch.tensor([0.0, -5.0, 1.5]), torch.zeros(3))
+    r.add_light(strength=0.0)
+    r.setup_environment()
+    gout = torch.randn(n, 3, H, W, generator=gen)
+    p = diff.scene_params(r)
+    grads = torch.autograd.grad(diff.render(r, p), p.colors, gout.cuda())
+    vis = r.render(vis=True)["vis"].cpu()
+    first = 0
+    for got, k, ntri in zip(grads, counts, (12, 224)):
+        for s in range(n):
+            for i in range(k):
+                lo = first + i * ntri
+                mine = (vis[s] >= lo) & (vis[s] < lo + ntri)
+                g = gout[s][:, mine].double()
+                bound = mine.sum() * 2.0 ** -24 * g.abs().sum(1)
+                err = (got[s * k + i, :3].cpu().double() - g.sum(1)).abs()
+                assert (err <= bound).all(), (res, ntri, s, i, err, bound)
+        first += k * ntri
