@@ -44,9 +44,11 @@ def resolve_model(path: str):
 
 def _plain(t, shape: tuple, device: torch.device) -> bool:
     """Whether a kernel can use t in place: a contiguous float32 tensor of
-    this shape on this device that autograd does not follow."""
+    this shape on this device that autograd does not follow and whose memory
+    holds its values (not their negatives, see torch's negative bit)."""
     return (type(t) is torch.Tensor and t.dtype is torch.float32 and t.device == device
-            and tuple(t.shape) == shape and t.is_contiguous() and not t.requires_grad)
+            and tuple(t.shape) == shape and t.is_contiguous() and not t.requires_grad
+            and not t.is_neg())
 
 
 class SteeringRenderer(PBRRenderer):
@@ -158,7 +160,9 @@ class SteeringRenderer(PBRRenderer):
             return False
         if col is not None and not _plain(col, (n, 4), self.device):
             return False
-        if type(st) is not torch.Tensor or torch._C._are_functorch_transforms_active():
+        # the memory of a state with the negative bit holds other signs
+        if (type(st) is not torch.Tensor or st.is_neg()
+                or torch._C._are_functorch_transforms_active()):
             return False
         half = float(self.cfg.lane_width) * 0.5
         z = float(self.cfg.rail_offset[2])

@@ -117,6 +117,26 @@ def test_steering_step_launch_matches_tensor_operations(cuda, n, cols):
                  got={"pixels": a.step(dev)})
 
 
+@pytest.mark.parametrize("cols", [2, 4])
+def test_steering_step_of_negated_memory(cuda, cols):
+    """A state, or a tensor the step reads, whose memory holds the negatives
+    of its values (torch's negative bit)."""
+    g = torch.Generator("cpu").manual_seed(cols)
+    a, b = _steering(65, 7), _steering(65, 7)
+    b._step_device = lambda st: False
+    z = torch.complex(torch.rand(65, cols, generator=g), torch.randn(65, cols, generator=g) * 2.0)
+    state = z.cuda().conj().imag
+    assert state.is_neg()
+    same = [x.equal(y) for x, y in zip(_scene_bits(a, a.step(state)),
+                                       _scene_bits(b, b.step(state.resolve_neg())))]
+    assert all(same), same
+    for r in (a, b):
+        r._camera_eye_offset = torch._neg_view(r._camera_eye_offset)
+    state = state.resolve_neg()
+    same = [x.equal(y) for x, y in zip(_scene_bits(a, a.step(state)), _scene_bits(b, b.step(state)))]
+    assert all(same), same
+
+
 @pytest.mark.parametrize("shift_dst,shift_src", [(0, 0), (0, 1), (3, 0), (2, 2)])
 def test_copy_segments(cuda, shift_dst, shift_src):
     """Copies and clears of 0 .. 70001 floats at aligned and odd addresses,
