@@ -26,6 +26,7 @@ from ... import _abi, _native
 from ...config import PBRConfig
 from ...renderer import mesh as meshmod
 from ...renderer.camera import PBRCam
+from ...renderer.node import PBRNode
 from ...renderer.renderer import PBRRenderer
 
 _FALLBACK = {"models/smiley": "models/sphere", "models/cone.egg": "models/cone",
@@ -49,6 +50,13 @@ def _plain(t, shape: tuple, device: torch.device) -> bool:
     return (type(t) is torch.Tensor and t.dtype is torch.float32 and t.device == device
             and tuple(t.shape) == shape and t.is_contiguous() and not t.requires_grad
             and not t.is_neg())
+
+
+def _replaced(obj, base: type, *names: str) -> bool:
+    """Whether obj's class or obj itself has its own version of one of these
+    methods of base."""
+    own, cls = obj.__dict__, type(obj)
+    return any(n in own or getattr(cls, n) is not getattr(base, n) for n in names)
 
 
 class SteeringRenderer(PBRRenderer):
@@ -143,14 +151,20 @@ class SteeringRenderer(PBRRenderer):
     def _step_device(self, st: torch.Tensor) -> bool:
         """The state mapping of ``_step`` in one HIP launch (pbr_steering_step);
         False, with nothing done, for what that launch does not take: the CPU,
-        poses recorded before it, a replaced camera, and tensors it cannot
-        read or write in place."""
+        poses recorded before it, a replaced camera, methods of the renderer,
+        the player or the camera that it would pass by although a subclass or
+        the object itself has its own, and tensors it cannot read or write in
+        place."""
         cam = self._pbr_cam
         n = self._num_scenes
         if (self.device.type != "cuda" or type(cam) is not PBRCam or cam.num_scenes != n
                 or cam.device != self.device or self._pending_poses or n < 1 or st.shape[1] < 2):
             return False
         player = self.player_node
+        if (_replaced(self, PBRRenderer, "set_poses") or _replaced(player, PBRNode, "set_colors")
+                or _replaced(cam, PBRCam, "set_positions", "set_eye", "_update_view",
+                             "_compose_view", "_refresh", "_update_vp")):
+            return False
         col = player.colors_b4 if player.has_geometry else None
         P = cam._get_projection()
         reads = (cam._right, cam._up, cam._fwd, P, self._camera_eye_offset, self._color_player,

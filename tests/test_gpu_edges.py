@@ -137,6 +137,42 @@ def test_steering_step_of_negated_memory(cuda, cols):
     assert all(same), same
 
 
+@pytest.mark.parametrize("what", ["subclass", "instance"])
+def test_steering_step_calls_replaced_methods(cuda, what):
+    """A subclass's or an object's own set_poses, set_colors and camera
+    methods see the step's poses, colours and eye."""
+    calls = []
+
+    class Logged(SteeringRenderer):
+        def set_poses(self, poses):
+            calls.append("poses")
+            super().set_poses(poses)
+
+    def logged(obj, name):
+        inner = getattr(obj, name)
+
+        def method(*args, **kw):
+            calls.append(name)
+            return inner(*args, **kw)
+        setattr(obj, name, method)
+
+    r = _steering(5, 7)
+    state = torch.rand(5, 4).cuda()
+    r.step(state)
+    if what == "subclass":
+        r.__class__ = Logged
+        r.step(state)
+        assert calls == ["poses"]
+        return
+    for obj, name in ((r, "set_poses"), (r.player_node, "set_colors"),
+                      (r._pbr_cam, "set_positions")):
+        calls.clear()
+        logged(obj, name)
+        r.step(state)
+        assert name in calls, name
+        delattr(obj, name)
+
+
 @pytest.mark.parametrize("shift_dst,shift_src", [(0, 0), (0, 1), (3, 0), (2, 2)])
 def test_copy_segments(cuda, shift_dst, shift_src):
     """Copies and clears of 0 .. 70001 floats at aligned and odd addresses,
