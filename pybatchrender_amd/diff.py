@@ -102,7 +102,26 @@ def _live_descriptor(renderer, vertices, light, colors):
     desc.light_col[:] = lv[3:6]
     desc.ambient[:] = lv[6:9]
     desc.strength = lv[9]
+    # transforms and a view-projection that a kernel cannot read in place: the
+    # renderer's descriptor may hold a copy made before their last change
+    for j, node in enumerate(g["nodes"]):
+        t = _readable(node.transforms_b44)
+        if t is not node.transforms_b44:
+            desc.nodes[j].transforms = t.data_ptr()
+            keep.append(t)
+    vp = renderer._pbr_cam.VP_k44
+    t = _readable(vp)
+    if t is not vp:
+        desc.view_proj = t.data_ptr()
+        keep.append(t)
     return desc, keep
+
+
+def _readable(t: torch.Tensor) -> torch.Tensor:
+    """t if its memory holds its values as contiguous float32, else a copy."""
+    if t.dtype is torch.float32 and t.is_contiguous() and not t.is_neg():
+        return t
+    return t.detach().to(torch.float32).contiguous().resolve_neg()
 
 
 def _freeze(renderer, desc, keep) -> None:

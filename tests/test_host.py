@@ -345,3 +345,47 @@ def test_atlas_layout_errors():
     from pybatchrender.envs.cartpole import CartPoleConfig
     cc = PBRConfig.from_config(CartPoleConfig(num_scenes=2, device="cpu"), max_steps=7)
     assert type(cc) is CartPoleConfig and cc.max_steps == 7 and cc.num_scenes == 2
+
+
+@pytest.mark.parametrize("what", ["float64", "strided", "negated"])
+def test_differentiable_render_reads_current_transforms(what):
+    """The descriptor of a differentiable render holds the values its
+    transforms and view-projection have at the call, also where they are not
+    float32 rows that a kernel can read in place and were edited in place since
+    the last call."""
+    import ctypes
+
+    import numpy as np
+
+    import pybatchrender as pbr
+    from pybatchrender import diff
+
+    n = 3
+    r = pbr.PBRRenderer(pbr.PBRConfig(num_scenes=n, tile_resolution=(8, 8), device="cpu"))
+    node = r.add_node("models/box", instances_per_scene=2)
+    r.add_camera()
+    r.setup_environment()
+
+    def odd(t):
+        if what == "float64":
+            return t.double()
+        if what == "strided":
+            return t.transpose(1, 2).contiguous().transpose(1, 2)
+        return torch._neg_view(-t)
+
+    def floats(p, count):
+        return torch.from_numpy(np.ctypeslib.as_array(
+            ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (count,)).copy())
+
+    node.transforms_b44 = odd(torch.randn(n * 2, 4, 4))
+    r._pbr_cam.VP_k44 = odd(torch.randn(n, 4, 4))
+    p = diff.scene_params(r)
+    for k in range(2):
+        desc, keep = diff._descriptor(r, p.vertices, p.light, p.colors)
+        for ptr, t in ((desc.nodes[0].transforms, node.transforms_b44),
+                       (desc.view_proj, r._pbr_cam.VP_k44)):
+            want = t.to(torch.float32).resolve_neg().reshape(-1)
+            assert torch.equal(floats(ptr, t.numel()), want), (what, k)
+        node.transforms_b44.mul_(2.0)
+        r._pbr_cam.VP_k44.add_(1.0)
+        del keep
