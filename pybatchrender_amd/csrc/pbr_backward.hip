@@ -56,6 +56,7 @@
 #include "../../include/pbr_abi.h"
 #include "pbr_device.h"
 #include "pbr_host.h"
+#include "pbr_slot.h"
 
 using namespace pbr_host;
 
@@ -172,17 +173,9 @@ __device__ __forceinline__ void bwd_fetch(const pbr_scene_desc& D, int s, const 
   for (int k = 1; k < D.num_nodes; ++k) j = slot >= base[k] ? k : j;
   const BNode& nd = nodes[j];
   const uint32_t local = slot - base[j];
-  // local / ntri from a float reciprocal: below 2^17, so the truncated product
-  // is off by at most one and one step corrects it
-  uint32_t i = (uint32_t)((float)local * nd.inv_nt);
-  int32_t t = (int32_t)(local - i * (uint32_t)nd.ntri);
-  if (t < 0) {
-    --i;
-    t += nd.ntri;
-  } else if (t >= nd.ntri) {
-    ++i;
-    t -= nd.ntri;
-  }
+  uint32_t i;
+  int32_t t;
+  pbr_slot::split(local, nd.ntri, nd.inv_nt, i, t);  // below kMaxBitmapSlots
   const size_t row = (nd.flags & 1u) ? (size_t)i : (size_t)s * (size_t)nd.ips + i;
   T.node = j;
   T.row = (uint32_t)row;

@@ -38,6 +38,7 @@
 #include "../../include/pbr_abi.h"
 #include "pbr_device.h"
 #include "pbr_host.h"
+#include "pbr_slot.h"
 
 using namespace pbr_host;
 
@@ -387,17 +388,9 @@ __device__ __forceinline__ SlotRef band_slot(int s, const NodeLds* nodes, int nn
   for (int k = 1; k < nn; ++k) nj = slot >= nodes[k].base ? k : nj;
   const NodeLds& nd = nodes[nj];
   const uint32_t local = slot - nd.base;
-  // local / ntri from a float reciprocal: the quotient is below 2^24, so the
-  // truncated product is off by at most one and one step corrects it
-  uint32_t i = (uint32_t)((float)local * nd.inv_nt);
-  int32_t t = (int32_t)(local - i * (uint32_t)nd.ntri);
-  if (t < 0) {
-    --i;
-    t += nd.ntri;
-  } else if (t >= nd.ntri) {
-    ++i;
-    t -= nd.ntri;
-  }
+  uint32_t i;
+  int32_t t;
+  pbr_slot::split(local, nd.ntri, nd.inv_nt, i, t);
   SlotRef R;
   R.trans = nd.trans;
   R.cols = nd.cols;
@@ -1186,6 +1179,8 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
     if (D->nodes[j].instances_per_scene == 0 || me.num_triangles == 0) continue;
     if (me.num_vertices < 1 || me.num_vertices > kBandVerts || me.num_triangles > kBandTris)
       return false;
+    // shading finds a slot's instance by pbr_slot::split
+    if (D->nodes[j].instances_per_scene > (int32_t)pbr_slot::kMaxInstances) return false;
     verts = std::max(verts, me.num_vertices);
     ntab = std::max(ntab, me.index_offset + me.num_triangles);
   }
