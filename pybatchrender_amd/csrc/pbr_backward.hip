@@ -67,6 +67,15 @@ constexpr int kRun = 16;   // flat kernel: pixels of one column walked by a lane
 constexpr int kPix = 8;    // per-scene kernel: pixels of one row a thread sorts, and of
                            // one slot a lane then sums
 constexpr int kSortPixels = kBwdBlock * kPix;  // pixels sorted at a time
+// lanes of a wave that hold their neighbour's slot from which on the slots' sums
+// are joined across lanes before the atomics: 64 atomics on one address take
+// their turns, the joins about eight instructions a sum.  Kernel in us, never /
+// from 44 / 32 / 16 lanes: 512 scenes of 128 x 128 with a plane of 2 smooth
+// triangles over the frame 273 / 114 / 114 / 114, of 128 triangles 290 / 142 / 142 /
+// 142, 4096 of 48 x 48 with one of 2 329 / 173 / 173 / 162, 256 of 256 x 256
+// with 8 boxes and 8 spheres 220 / 216 / 209 / 199, 512 of 128 x 128 with 16 and
+// 16 231 / 231 / 230 / 228.
+constexpr int kJoin = 16;
 constexpr int kAcc = 29;   // accumulator floats per slot (28, odd to spread LDS banks)
 constexpr int kRecF = 23;  // per-pixel factors per slot
 constexpr int kLightF = 10;
@@ -378,6 +387,40 @@ __device__ __forceinline__ float wave_sum63(float v) {
   return v;
 }
 
+// Lanes of a wave ordered by slot: which of the lanes 1, 2, 4 and 8 before
+// this one in its row of 16 hold the same slot, and whether the next one does
+// not.
+struct SlotRuns {
+  bool same[4];
+  bool last;
+};
+template <int CTRL>
+__device__ __forceinline__ int dpp_slot(int slot) {
+  return __builtin_amdgcn_update_dpp(-1, slot, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ SlotRuns slot_runs(int slot) {
+  SlotRuns R;
+  R.same[0] = dpp_slot<0x111>(slot) == slot;  // row_shr:1
+  R.same[1] = dpp_slot<0x112>(slot) == slot;
+  R.same[2] = dpp_slot<0x114>(slot) == slot;
+  R.same[3] = dpp_slot<0x118>(slot) == slot;
+  R.last = dpp_slot<0x101>(slot) != slot;  // row_shl:1
+  return R;
+}
+// Sum of v over the slot's lanes in the row up to this one (lanes of other
+// slots are left out by selection: theirs may be infinite).
+__device__ __forceinline__ float slot_sum(float v, const SlotRuns& R) {
+  const float a = dpp_src<0x111, 0xf>(v);
+  v += R.same[0] ? a : 0.0f;
+  const float b = dpp_src<0x112, 0xf>(v);
+  v += R.same[1] ? b : 0.0f;
+  const float c = dpp_src<0x114, 0xf>(v);
+  v += R.same[2] ? c : 0.0f;
+  const float d = dpp_src<0x118, 0xf>(v);
+  v += R.same[3] ? d : 0.0f;
+  return v;
+}
+
 // The light, vertex and shared-colour sums of one workgroup as its partial
 // row (layout: light[10], then F.off_v, then F.off_s).
 __device__ __forceinline__ void write_partial(const BwdFrame& F, const BwdLight& L,
@@ -651,6 +694,9 @@ __attribute__((amdgpu_waves_per_eu(4))) void backward_kernel(pbr_scene_desc D, B
         const uint32_t p0 = (u - (f >> 16)) * kPix;
         const int n = (int)min((uint32_t)kPix, S.count[sl] - p0);
         const uint16_t* ord = S.order + (f & 0xffffu) + p0;
+        // units of a slot sit in neighbouring lanes
+        const SlotRuns runs = slot_runs(sl);
+        const bool join = __popcll(__ballot(runs.same[0])) >= kJoin;
         int px[kPix], py[kPix];  // columns and GL rows
         float g[NC][kPix];
 #pragma unroll
@@ -675,8 +721,14 @@ __attribute__((amdgpu_waves_per_eu(4))) void backward_kernel(pbr_scene_desc D, B
             a[A_G + c] += g[c][i];
           }
         float* dst = S.acc + (size_t)sl * ACC;
+        if (join) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) atomicAdd(dst + A_G + c, a[A_G + c]);
+          for (int c = 0; c < NC; ++c) a[A_G + c] = slot_sum(a[A_G + c], runs);
+        }
+        if (!join || runs.last) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) atomicAdd(dst + A_G + c, a[A_G + c]);
+        }
         if constexpr (SMOOTH) {
           if (S.list[sl] >> 31) {
             // the slot's per-pixel factors, made again by each of its lanes:
@@ -745,10 +797,17 @@ __attribute__((amdgpu_waves_per_eu(4))) void backward_kernel(pbr_scene_desc D, B
                 a[A_GP + 3 * k + 2] += guk;
               }
             }
+            if (join) {
 #pragma unroll
-            for (int c = 0; c < NL; ++c) atomicAdd(dst + A_GD + c, a[A_GD + c]);
+              for (int q = A_GD; q < A_GP + 9; ++q)
+                if (q < A_GD + NL || q >= A_GL) a[q] = slot_sum(a[q], runs);
+            }
+            if (!join || runs.last) {
 #pragma unroll
-            for (int q = A_GL; q < A_GP + 9; ++q) atomicAdd(dst + q, a[q]);
+              for (int c = 0; c < NL; ++c) atomicAdd(dst + A_GD + c, a[A_GD + c]);
+#pragma unroll
+              for (int q = A_GL; q < A_GP + 9; ++q) atomicAdd(dst + q, a[q]);
+            }
           }
         }
       }

@@ -329,3 +329,74 @@ def test_smooth_backward_pixel_sums(cuda, res, spheres):
                 err = (got[s * k + i, :3].cpu().double() - g.sum(1)).abs()
                 assert (err <= bound).all(), (res, ntri, s, i, err, bound)
         first += k * ntri
+
+
+@pytest.mark.parametrize("mesh", [1, 2, 5])
+@pytest.mark.parametrize("res", [(64, 64), (50, 17), (130, 33), (300, 100)])
+def test_smooth_backward_large_triangles(cuda, res, mesh):
+    """Smooth triangles of many units of eight pixels each, whose sums are
+    joined across a wave's lanes: one slot for whole waves, slots that change
+    within a row of lanes, a last wave that is not full.  Unlit, a node's
+    colour gradient is the sum of the output gradient over its pixels (bound as
+    in test_smooth_backward_pixel_sums), also where one instance's gradient is
+    infinite and its neighbour's is not."""
+    W, H = res
+    gen = torch.Generator("cpu").manual_seed(W + mesh)
+    t = torch.linspace(-3.0, 3.0, mesh + 1)
+    x, z = torch.meshgrid(t, t, indexing="ij")
+    pos = torch.stack([x, 0.1 * x * z, z], -1).reshape(-1, 3)
+    nrm = torch.stack([0.1 * x, -torch.ones_like(x), 0.1 * z], -1).reshape(-1, 3)
+    a = (torch.arange(mesh)[:, None] * (mesh + 1) + torch.arange(mesh)).reshape(-1)
+    b = a + mesh + 1
+    tri = torch.cat([torch.stack([a, b, b + 1], 1), torch.stack([a, b + 1, a + 1], 1)])
+    n = 3
+    r = PBRRenderer(PBRConfig(num_scenes=n, tile_resolution=res, device="cuda",
+                              output_dtype="float32"))
+    node = r.add_node(Mesh(pos.numpy(), nrm.numpy(), tri.numpy()), instances_per_scene=2)
+    eye = torch.eye(4).repeat(n * 2, 1, 1)
+    eye[1::2, 0, 3] = 1.5  # the second plane covers the right part of the frame
+    eye[1::2, 1, 3] = -0.7
+    node.set_transforms(eye)
+    node.set_colors(torch.rand(n * 2, 4, generator=gen))
+    r.add_camera().set_positions_and_lookat(torch.tensor([0.0, -4.0, 0.3]), torch.zeros(3))
+    r.add_light(strength=0.0)
+    r.setup_environment()
+    vis = r.render(vis=True)["vis"].cpu()
+    inst = torch.where(vis >= 0, vis // len(tri), -1)
+    assert all((inst[s] == i).sum() > W * H // 20 for s in range(n) for i in (0, 1))
+    gout = torch.randn(n, 3, H, W, generator=gen)
+    gout[2][:, inst[2] == 0] = float("inf")
+    p = diff.scene_params(r)
+    got = torch.autograd.grad(diff.render(r, p), p.colors, gout.cuda())[0].cpu()
+    for s in range(n):
+        for i in range(2):
+            if (s, i) == (2, 0):
+                assert not torch.isfinite(got[s * 2 + i, :3]).any()
+                continue
+            g = gout[s][:, inst[s] == i].double()
+            bound = g.shape[1] * 2.0 ** -24 * g.abs().sum(1)
+            err = (got[s * 2 + i, :3].double() - g.sum(1)).abs()
+            assert (err <= bound).all(), (res, mesh, s, i, err, bound)
+
+
+@pytest.mark.parametrize("mesh", [1, 5])
+def test_smooth_backward_large_triangles_match_reference(cuda, mesh):
+    """All gradients of lit smooth planes against the float64 reference."""
+    from tests.test_diff import _assert_close, _kernel_and_reference
+
+    t = torch.linspace(-3.0, 3.0, mesh + 1)
+    x, z = torch.meshgrid(t, t, indexing="ij")
+    pos = torch.stack([x, 0.1 * x * z, z], -1).reshape(-1, 3)
+    nrm = torch.stack([0.1 * x, -torch.ones_like(x), 0.1 * z], -1).reshape(-1, 3)
+    a = (torch.arange(mesh)[:, None] * (mesh + 1) + torch.arange(mesh)).reshape(-1)
+    b = a + mesh + 1
+    tri = torch.cat([torch.stack([a, b, b + 1], 1), torch.stack([a, b + 1, a + 1], 1)])
+    r = PBRRenderer(PBRConfig(num_scenes=2, tile_resolution=(96, 96), device="cuda",
+                              output_dtype="float32"))
+    node = r.add_node(Mesh(pos.numpy(), nrm.numpy(), tri.numpy()), instances_per_scene=1)
+    node.set_colors(torch.tensor([[0.3, 0.6, 0.5, 0.9], [0.8, 0.2, 0.4, 0.7]]))
+    r.add_camera().set_positions_and_lookat(torch.tensor([0.2, -4.0, 0.3]), torch.zeros(3))
+    r.add_light(ambient=(0.2, 0.2, 0.25), dir_dir=(0.1, 0.9, -0.3), dir_col=(0.9, 0.8, 0.7),
+                strength=0.9)
+    r.setup_environment()
+    _assert_close(*_kernel_and_reference(r)[:2])
