@@ -71,7 +71,7 @@ struct RowsFrame {
   int seg;  // setup lanes per scene (power of two >= slots, <= 64)
   int cap;  // row-list entries per band (8..kCap)
   int vphase;  // 1: vertices transformed once into an LDS table (they fit)
-  int stream;  // 1: frame stores are streaming (see launch_rows)
+  int stream;  // 1: frame stores are streaming (see streams_frame)
 };
 
 // Instance poses a launch applies itself (pbr_render_posed).  Pose d[k]
@@ -1332,6 +1332,42 @@ bool rows_small(const pbr_scene_desc* D) {
   return rows_narrow(D) && D->num_scenes > kWideScenes;
 }
 
+// Whether the frame's stores are streaming.  A wave stores four rows of at most 64
+// columns, one piece of 4 W pixels; streaming stores of pieces that are no whole
+// 128-byte lines cost (4096 scenes of 47 x 64 float32 + depth, ordinary /
+// streaming: 63 / 76 us).  For the others the caches decide: outputs of up to
+// kL2Bytes leave the L2s sooner, uint8 colours alone always do; of what is larger
+// the 256 MiB last-level cache keeps enough until the same buffers are written
+// again (or read) up to the limits below, with depth or ids at any size that was
+// measured.  Kernel in us for scenes of 64 x 64, ordinary / streaming, one output
+// buffer (two in turn):
+//   uint8 + depth    1024  28 MiB  15.8 / 14.8 (15.7 / 14.7)
+//   uint8            4096  48      26.8 / 24.9 (26.2 / 24.4)
+//   uint8            8192  96      46.8 / 44.4 (45.7 / 43.7)
+//   uint8 + depth    4096 112      30.0 / 34.0 (29.9 / 33.7)
+//   uint8 + d + ids  8192 352      79.2 / 82.9 (78.7 / 84.1)
+//   bf16             8192 192      49.2 / 51.6 (53.1 / 51.1)
+//   bf16            12288 288      75.5 / 71.9 (75.3 / 70.7)
+//   bf16 + d + ids   5200 284      54.5 / 69.8 (68.5 / 69.2)
+//   bf16 + depth    16384 640       138 / 137  (138 / 139)
+//   float32          1024  48      17.5 / 17.0 (17.3 / 16.9)
+//   float32 + depth  1024  64      19.4 / 20.6 (19.2 / 20.4)
+//   float32          2048  96      25.0 / 27.2 (24.9 / 27.1)
+//   float32          4096 192      40.0 / 47.7 (49.4 / 48.0)
+//   float32          6656 312      65.5 / 73.8 (75.2 / 73.0)
+//   float32          8192 384      87.8 / 85.9 (88.9 / 86.4)
+//   float32 + depth  4096 256      49.4 / 61.5 (60.6 / 61.0)
+bool streams_frame(const pbr_scene_desc* D, const pbr_frame_out* O) {
+  constexpr uint64_t kL2Bytes = 64ull << 20, kKeptF32 = 320ull << 20, kKeptBf16 = 256ull << 20;
+  const uint64_t elem = O->dtype == PBR_DTYPE_U8 ? 1 : (O->dtype == PBR_DTYPE_BF16 ? 2 : 4);
+  if (D->width > 64 || (4 * D->width * elem) % 128 != 0) return false;
+  const uint64_t bytes = (uint64_t)D->num_scenes * D->width * D->height *
+                         (O->channels * elem + (O->depth ? 4 : 0) + (O->vis ? 4 : 0));
+  if (bytes <= kL2Bytes) return true;
+  if (O->depth || O->vis) return false;
+  return elem == 1 || bytes > (elem == 2 ? kKeptBf16 : kKeptF32);
+}
+
 // Whether both scenes' vertex slots fit the LDS vertex table (the vertex
 // phase transforms each vertex once).
 bool rows_vphase(const pbr_scene_desc* D) {
@@ -1454,13 +1490,7 @@ int launch_rows(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rende
   const bool small = rows_small(D);
   F.cap = cap ? cap : kCap;
   F.vphase = rows_vphase(D) ? 1 : 0;
-  // A wave stores four rows of at most 64 columns, one piece of 4 W pixels.
-  // Streaming stores pay where the pieces are whole 128-byte lines and cost
-  // where they cut lines (us per call, ordinary / streaming: 4096 scenes of 64
-  // x 64 uint8 26.5 / 24.6, float32 + depth 72 / 66; of 47 x 64 63 / 76; of
-  // 84 x 84 128 / 266).
-  const int elem = O->dtype == PBR_DTYPE_U8 ? 1 : (O->dtype == PBR_DTYPE_BF16 ? 2 : 4);
-  F.stream = D->width <= 64 && (4 * D->width * elem) % 128 == 0 ? 1 : 0;
+  F.stream = streams_frame(D, O) ? 1 : 0;
   const Light lt = host_light(D);
   const float4 bg = make_float4(D->background[0], D->background[1], D->background[2],
                                 D->background[3]);

@@ -30,6 +30,31 @@ def test_rows_kernel_ragged_widths(cuda, width, dtype):
         check_parity(r, f"rows width {width} {cls.__name__}, colour only", depth=False, vis=False)
 
 
+@pytest.mark.parametrize("n,dtype", [(7168, "float32"), (11264, "bfloat16")])
+def test_rows_kernel_store_forms(cuda, n, dtype):
+    """Frames larger than the last-level cache leave by streaming stores: the
+    same pixels as the scenes give in smaller batches, alone and with depth and
+    ids (by ordinary stores)."""
+    st = ground_states(n, 3).cuda()
+    vp = None  # the whole batch's: a view's aspect follows the batch's tile grid
+
+    def frames(a, b):
+        nonlocal vp
+        r = CartPoleGroundRenderer(CartPoleConfig(num_scenes=b - a, device="cuda", kernel="rows",
+                                                  output_dtype=dtype))
+        r._step(st[a:b])
+        if vp is None:
+            vp = r._pbr_cam.VP_k44
+        r._pbr_cam.VP_k44 = vp[a:b].clone()
+        full = r.render(depth=True, vis=True)
+        return r.render()["pixels"], full["pixels"], full["depth"], full["vis"]
+
+    whole = frames(0, n)
+    for a in range(0, n, 1024):
+        for x, y in zip(whole, frames(a, a + 1024)):
+            assert _bits(x[a:a + 1024]).equal(_bits(y)), (a, x.dtype)
+
+
 @pytest.mark.parametrize("cap", [0, 8])
 @pytest.mark.parametrize("dtype", ["uint8", "bfloat16", "float32"])
 @pytest.mark.parametrize("n", [2048, 2049])
