@@ -45,8 +45,8 @@ using namespace pbr_host;
 namespace {
 
 constexpr int kBandWaves = 8;     // waves of a workgroup, two workgroups on a CU
-constexpr int kWideWaves = 16;    // or one workgroup with all the waves of a CU
-constexpr int kWideItems = 256;   // for at most this many workgroups (see bands_plan)
+constexpr int kWideWaves = 16;    // or one workgroup with all the waves of a CU, for
+                                  // at most one workgroup a CU (see bands_plan)
 constexpr int kBandVerts = 136;   // vertices a wave's table holds at most
 constexpr int kBandTris = 256;    // triangles of one chunk (8-bit queue entries)
 constexpr int kBandTable = 512;   // triangles of all meshes (LDS index table) at most
@@ -1217,11 +1217,11 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   // 16 / 16 and bands): 64 scenes of 84 x 84 with up to 256 instances 99 / 68 /
   // 50, of 128 x 128 with 64 boxes 26 / 26 / 18, of 64 x 64 steering 50 / 47 /
   // 45; 512 steering scenes in one workgroup per CU at a time 96, not 73.
-  const int64_t n = D->num_scenes;
-  if (n * F.bands <= kWideItems) {
+  const int64_t n = D->num_scenes, cus = device_cus();
+  if (n * F.bands <= cus) {
     const int wide = (int)((2 * kBandLds - stat - rest(kWideWaves)) / 8);
     int bands = 1;
-    while (bands < kMaxBands && 2 * n * bands <= kWideItems && D->height / bands >= 16) bands *= 2;
+    while (bands < kMaxBands && 2 * n * bands <= cus && D->height / bands >= 16) bands *= 2;
     split(kWideWaves, std::min(wide, 2 * kBandPixels) / D->width, bands);
   }
   return true;

@@ -1322,14 +1322,14 @@ bool rows_narrow(const pbr_scene_desc* D) {
 }
 
 // They run it when the batch fills the chip: its two waves per workgroup keep
-// a wave per scene busy.  Up to kWideScenes scenes the 64-record form's four waves per
-// workgroup are all resident at once (four workgroups on each of 256 CUs) and
-// each has half the rows to walk.  CartPole at 64 x 64, uint8, 32- / 64-record
-// form: 64 scenes 15.9 / 11.7 us, 1000 19.2 / 14.0, 2000 20.0 / 17.5, 2500
-// 22.7 / 25.2, 4096 25.9 / 31.0.
-constexpr int kWideScenes = 2048;
+// a wave per scene busy.  Up to eight scenes a CU the 64-record form's four waves
+// per workgroup are all resident at once (four workgroups on each CU) and each
+// has half the rows to walk.  CartPole at 64 x 64, uint8, 32- / 64-record form, 256
+// CUs: 64 scenes 15.9 / 11.7 us, 1000 19.2 / 14.0, 2000 20.0 / 17.5, 2500 22.7 /
+// 25.2, 4096 25.9 / 31.0; at 32 x 32 to 64 x 160, uint8 and float32, 2000 scenes
+// 0.96 to 1.26 of the speed, fewer always faster.
 bool rows_small(const pbr_scene_desc* D) {
-  return rows_narrow(D) && D->num_scenes > kWideScenes;
+  return rows_narrow(D) && D->num_scenes > 8 * device_cus();
 }
 
 // Whether the frame's stores are streaming.  A wave stores four rows of at most 64
