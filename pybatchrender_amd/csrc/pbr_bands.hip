@@ -1162,12 +1162,50 @@ struct BandPlan {
   size_t lds;
 };
 
+// Whether the scenes are few and each is much work.  A scene has at most kMaxBands
+// workgroups, which each transform all its vertices, where the tile path spreads
+// the scene's setup over the chip.  Which path draws sooner then depends on what is
+// left after setup, which the host does not know: tile path's time over the band
+// path's for objects of usual size / smaller than a pixel, frames of 32 x 32 to 160 x
+// 160 (geometric means, boxes, UV spheres and cylinders):
+//   vertices of a scene  1 scene      4            8            16           32
+//   10 to 15 thousand    1.51 / 1.13  1.86 / 1.23  2.22 / 1.34  2.99 / 1.54  4.10 / 1.91
+//   30 to 60             1.15 / 0.52  1.48 / 0.65  1.86 / 0.80  2.58 / 1.08  2.92 / 1.34
+//   60 to 150            1.04 / 0.28  1.42 / 0.41  1.61 / 0.50  1.97 / 0.66  2.41 / 0.87
+//   150 to 400           0.96 / 0.15  1.17 / 0.23  1.33 / 0.30  1.75 / 0.46  2.47 / 0.74
+//   400 to 2000          1.07 / 0.10  1.23 / 0.18  1.47 / 0.29  1.92 / 0.49  2.57 / 0.82
+// The line is where the mean over both is about one.  From 128 scenes on it is 1.8
+// to 2.3, the lowest 0.74 (1024 scenes of 160 x 160 with 500 boxes below a pixel).
+bool few_large_scenes(const pbr_scene_desc* D, const pbr_render_opts* opts) {
+  const int64_t n = D->num_scenes;
+  if (n < 1 || 16 * n > device_cus()) return false;
+  double verts = 0.0;
+  bool counts = false;
+  for (int j = 0; j < D->num_nodes; ++j) {
+    const pbr_node& nd = D->nodes[j];
+    const pbr_mesh& me = D->meshes[nd.mesh];
+    if (me.num_triangles > 0) verts += (double)nd.instances_per_scene * me.num_vertices;
+    counts = counts || nd.counts;
+  }
+  // of a batch with instance counts the slot budget tells the mean scene's share
+  const double most = (double)n * (double)max_slots(D);
+  if (counts && opts && opts->slot_budget > 0 && (double)opts->slot_budget < most)
+    verts *= (double)opts->slot_budget / most;
+  return verts > 24576.0 + 6144.0 * (double)n;
+}
+
 // Whether the band path draws the batch, and its launch shape: default tile
-// options (a tile size or bin capacity asks for the tile path), meshes the
-// wave tables hold, and few enough bands that repeating the scene's vertex
-// work per band stays below what the tile path's records cost.
+// options (a tile size or bin capacity asks for the tile path), meshes that the
+// wave tables hold, scenes whose setup its workgroups share out well, and frames of
+// at most kMaxBands bands and kBandTable triangles.  Tile path's time over the band
+// path's at three and four bands (160 x 160 and 176 x 176), 300 to 1024 scenes: 1.2
+// to 2.9 for objects of usual size, 0.74 to 2.5 for objects smaller than a pixel.
+// The two limits bound what was tested, they are no crossing: with both raised,
+// five to fourteen bands (200 x 200 to 320 x 320) gave 1.04 to 4.2 and 0.62 to 2.4,
+// and three to eight nodes with a sphere of 224 triangles each 1.3 to 4.5.
 bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& P) {
   if (opts && (opts->tile_size > 0 || opts->bin_capacity > 0)) return false;
+  if (few_large_scenes(D, opts)) return false;
   memset(&P, 0, sizeof(P));
   BandFrame& F = P.F;
   F.W = D->width;

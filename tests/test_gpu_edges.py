@@ -13,6 +13,7 @@ from pybatchrender.envs.cartpole import CartPoleConfig, CartPoleGroundRenderer, 
 from pybatchrender.envs.steering import SteeringConfig, SteeringRenderer
 from pybatchrender.renderer.mesh import Mesh
 from tests.test_gpu_parity import _bits, check_parity, ground_states
+from tests.test_gpu_posed import _kernel_names
 
 pytestmark = pytest.mark.gpu
 
@@ -315,6 +316,30 @@ def test_band_kernel_forms(cuda, n, res, dtype):
     r.setup_environment()
     check_parity(r, f"band form n={n} {res} {dtype}")
     check_parity(r, f"band form n={n} {res} {dtype}, colour only", depth=False, vis=False)
+
+
+@pytest.mark.parametrize("counts", [False, True])
+@pytest.mark.parametrize("n", [1, 4, 16])
+def test_band_kernel_few_scenes(cuda, n, counts):
+    """Few scenes on both sides of the vertices per scene from which the tile
+    kernels draw them (box: 24 vertices): the same frames as the oracle's, from
+    the expected kernels; with instance counts it is the mean scene's vertices
+    that decide."""
+    line = (24576 + 6144 * n) // 24
+    for k, band in ((line, True), (line + 1, False)):
+        ips = 2 * k if counts else k
+        r = workloads.many_cubes(num_scenes=n, resolution=33, instances=ips, seed=n, kernel="tiles",
+                                 output_dtype="uint8", output_depth=False)
+        if counts:  # k in the mean
+            c = torch.full((n,), k)
+            if n > 1:
+                c[0], c[1] = 2 * k, 0
+            r._drawn_nodes()[0].set_instance_counts(c)
+        check_parity(r, f"n={n}, {k} of {ips} boxes", vis=False)
+        names = _kernel_names(lambda: r.render())
+        if names:
+            assert any("bands_kernel" in s for s in names) == band, names
+            assert any("tile_raster_kernel" in s for s in names) != band, names
 
 
 @pytest.mark.parametrize("res,spheres", [((7, 40), 1), ((50, 17), 3), ((130, 33), 3),
