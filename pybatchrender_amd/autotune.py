@@ -11,7 +11,8 @@ renderer's config and returns the measurements:
       4 or 8 pixels per lane, bins per work item 0 (auto) / 1 / 2 / 4
   tile kernels: tile 0 (full-width bands) / 8 / 16 / 32 / 64 pixels (8 only
       for scenes of at most 2048 triangle slots: every tile tests every
-      slot's box), LDS bin capacity 1024 / 1904 / 4096 entries, and the
+      slot's box), LDS bin capacity 1024 / default / 4096 entries (tile 0 at the
+      default capacity is the band path where it draws the batch), and the
       persistent (scene, tile) queue at 4 / 8 / 16 workgroups per CU
 
 Results are cached per batch signature in memory (and in ``cache_path`` as
@@ -66,8 +67,10 @@ def candidates(renderer) -> list[dict]:
             out.append({"kernel": "tiles", "tile_size": ts, "persistent": False,
                         "bin_capacity": cap})
         for wpc in (4, 8, 16):
+            # a bin capacity (the default one) keeps full-width tiles with the
+            # tile kernels: the band path has no queue
             out.append({"kernel": "tiles", "tile_size": ts, "persistent": True,
-                        "workgroups_per_cu": wpc})
+                        "bin_capacity": 0 if ts else 1904, "workgroups_per_cu": wpc})
     return out
 
 

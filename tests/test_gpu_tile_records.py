@@ -8,7 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from pybatchrender import PBRConfig, PBRRenderer, workloads
+from pybatchrender import PBRConfig, PBRRenderer, autotune, workloads
 from tests.test_gpu_parity import _bits, check_parity
 from tests.test_gpu_posed import _kernel_names
 from tests.test_zz_no_alloc import _render, _same
@@ -105,3 +105,18 @@ def test_tile_records_noalloc(cuda, persistent):
         r = workloads.uneven_batch(num_scenes=n, resolution=84, max_instances=48, seed=n,
                                    kernel="tiles", bin_capacity=1904, persistent=persistent)
         _same(_render(r, noalloc=True), _render(r, noalloc=False), f"N={n}")
+
+
+def test_autotune_persistent_candidates_reach_the_queue(cuda):
+    """Every persistent tile candidate runs the tile kernels, not the band
+    path, which ignores the queue and its size."""
+    r = workloads.uneven_batch(num_scenes=24, resolution=48, max_instances=16, seed=1)
+    want = r.render()["pixels"].cpu()
+    seen = 0
+    for cand in autotune.candidates(r):
+        if cand["kernel"] == "tiles" and cand["persistent"]:
+            autotune._apply(r, cand)
+            assert torch.equal(r.render()["pixels"].cpu(), want), cand
+            _draws_records(r)
+            seen += 1
+    assert seen >= 12

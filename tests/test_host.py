@@ -389,3 +389,15 @@ def test_differentiable_render_reads_current_transforms(what):
         node.transforms_b44.mul_(2.0)
         r._pbr_cam.VP_k44.add_(1.0)
         del keep
+
+
+def test_autotune_candidates_are_different_launches():
+    """At default tile options the band path draws and ignores the persistent
+    queue, so persistent candidates name a tile size or a bin capacity."""
+    from pybatchrender import autotune, workloads
+
+    r = workloads.uneven_batch(num_scenes=4, resolution=32, max_instances=8, device="cpu")
+    tiles = [c for c in autotune.candidates(r) if c["kernel"] == "tiles"]
+    assert all(c["tile_size"] or c["bin_capacity"] for c in tiles if c["persistent"])
+    assert {c["workgroups_per_cu"] for c in tiles if c["persistent"] and not c["tile_size"]} == {
+        4, 8, 16}
