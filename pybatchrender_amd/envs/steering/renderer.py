@@ -52,11 +52,9 @@ def _plain(t, shape: tuple, device: torch.device) -> bool:
             and not t.is_neg())
 
 
-def _replaced(obj, base: type, *names: str) -> bool:
-    """Whether obj's class or obj itself has its own version of one of these
-    methods of base."""
-    own, cls = obj.__dict__, type(obj)
-    return any(n in own or getattr(cls, n) is not getattr(base, n) for n in names)
+# what the tensor operations of a step call (PBRCam.set_positions)
+_CAM_METHODS = frozenset(("set_positions", "set_eye", "_update_view", "_compose_view", "_refresh",
+                          "_update_vp"))
 
 
 class SteeringRenderer(PBRRenderer):
@@ -161,9 +159,9 @@ class SteeringRenderer(PBRRenderer):
                 or cam.device != self.device or self._pending_poses or n < 1 or st.shape[1] < 2):
             return False
         player = self.player_node
-        if (_replaced(self, PBRRenderer, "set_poses") or _replaced(player, PBRNode, "set_colors")
-                or _replaced(cam, PBRCam, "set_positions", "set_eye", "_update_view",
-                             "_compose_view", "_refresh", "_update_vp")):
+        if (type(self).set_poses is not PBRRenderer.set_poses or "set_poses" in self.__dict__
+                or type(player).set_colors is not PBRNode.set_colors
+                or "set_colors" in player.__dict__ or not _CAM_METHODS.isdisjoint(cam.__dict__)):
             return False
         col = player.colors_b4 if player.has_geometry else None
         P = cam._get_projection()
