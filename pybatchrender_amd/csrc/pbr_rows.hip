@@ -71,7 +71,7 @@ struct RowsFrame {
   int seg;  // setup lanes per scene (power of two >= slots, <= 64)
   int cap;  // row-list entries per band (8..kCap)
   int vphase;  // 1: vertices transformed once into an LDS table (they fit)
-  int stream;  // 1: frame stores are streaming (see streams_frame)
+  int stream;  // streaming stores: 1 colours, 2 depth and ids too (frame_stores)
 };
 
 // Instance poses a launch applies itself (pbr_render_posed).  Pose d[k]
@@ -899,11 +899,12 @@ __device__ __forceinline__ int lane_x0(int lane, int W) {
 }
 
 // Stores a lane's whole pixels (lane_x0), the first of them pix0 of the planes:
-// one dword (or wider) store per channel, whatever the row's alignment.
+// one dword (or wider) store per channel, whatever the row's alignment.  With
+// STREAM the colours' stores are streaming, with `planes` depth's and ids' too.
 template <int OM, int PXL, bool STREAM>
 __device__ __forceinline__ void store_lane(const SceneOut& so, uint32_t pix0,
                                            const typename ColOf<OM>::T* cv,
-                                           const PixState<PXL>& S) {
+                                           const PixState<PXL>& S, bool planes) {
   if constexpr (OM == 0) {
     // a uniform loop over the channels (its counter and byte selector stay
     // scalar; unrolled, the per-channel conditions were kept in spilled
@@ -949,18 +950,27 @@ __device__ __forceinline__ void store_lane(const SceneOut& so, uint32_t pix0,
   }
   if (so.depth) {
 #pragma unroll
-    for (int h = 0; h < PXL; h += 4)
-      store_frame<STREAM>(so.depth + pix0 + h,
-                          make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f, S.z[h + 2] + 0.0f,
-                                      S.z[h + 3] + 0.0f));
+    for (int h = 0; h < PXL; h += 4) {
+      const float4 z = make_float4(S.z[h] + 0.0f, S.z[h + 1] + 0.0f, S.z[h + 2] + 0.0f,
+                                   S.z[h + 3] + 0.0f);
+      if (STREAM && planes)
+        store_stream(so.depth + pix0 + h, z);
+      else
+        store_frame<false>(so.depth + pix0 + h, z);
+    }
   }
   if (so.vis) {
     int32_t v[PXL];
 #pragma unroll
     for (int i = 0; i < PXL; ++i) v[i] = S.z[i] < 1.0f ? (int32_t)(S.ref[i] >> 3) : -1;
 #pragma unroll
-    for (int h = 0; h < PXL; h += 4)
-      store_frame<STREAM>(so.vis + pix0 + h, make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]));
+    for (int h = 0; h < PXL; h += 4) {
+      const int4 id = make_int4(v[h], v[h + 1], v[h + 2], v[h + 3]);
+      if (STREAM && planes)
+        store_stream(so.vis + pix0 + h, id);
+      else
+        store_frame<false>(so.vis + pix0 + h, id);
+    }
   }
 }
 
@@ -990,9 +1000,9 @@ __device__ __forceinline__ void resolve_lane(const pbr_scene_desc& D, const Scen
     // never streaming with eight pixels a lane: each store instruction writes
     // every second half then
     if (PXL == 4 && F.stream)
-      store_lane<OM, PXL, true>(so, pix0, cv, S);
+      store_lane<OM, PXL, true>(so, pix0, cv, S, F.stream == 2);
     else
-      store_lane<OM, PXL, false>(so, pix0, cv, S);
+      store_lane<OM, PXL, false>(so, pix0, cv, S, false);
     return;
   }
   // a tile narrower than a lane: pixel by pixel
@@ -1332,40 +1342,43 @@ bool rows_small(const pbr_scene_desc* D) {
   return rows_narrow(D) && D->num_scenes > 8 * device_cus();
 }
 
-// Whether the frame's stores are streaming.  A wave stores four rows of at most 64
-// columns, one piece of 4 W pixels; streaming stores of pieces that are no whole
-// 128-byte lines cost (4096 scenes of 47 x 64 float32 + depth, ordinary /
+// Which stores of the frame are streaming: 0 none, 1 the colours, 2 depth and ids
+// too.  A wave stores four rows of
+// at most 64 columns, one piece of 4 W pixels; streaming stores of pieces that are
+// no whole 128-byte lines cost (4096 scenes of 47 x 64 float32 + depth, ordinary /
 // streaming: 63 / 76 us).  For the others the caches decide: outputs of up to
-// kL2Bytes leave the L2s sooner, uint8 colours alone always do; of what is larger
-// the 256 MiB last-level cache keeps enough until the same buffers are written
-// again (or read) up to the limits below, with depth or ids at any size that was
-// measured.  Kernel in us for scenes of 64 x 64, ordinary / streaming, one output
-// buffer (two in turn):
-//   uint8 + depth    1024  28 MiB  15.8 / 14.8 (15.7 / 14.7)
-//   uint8            4096  48      26.8 / 24.9 (26.2 / 24.4)
-//   uint8            8192  96      46.8 / 44.4 (45.7 / 43.7)
-//   uint8 + depth    4096 112      30.0 / 34.0 (29.9 / 33.7)
-//   uint8 + d + ids  8192 352      79.2 / 82.9 (78.7 / 84.1)
-//   bf16             8192 192      49.2 / 51.6 (53.1 / 51.1)
-//   bf16            12288 288      75.5 / 71.9 (75.3 / 70.7)
-//   bf16 + d + ids   5200 284      54.5 / 69.8 (68.5 / 69.2)
-//   bf16 + depth    16384 640       138 / 137  (138 / 139)
-//   float32          1024  48      17.5 / 17.0 (17.3 / 16.9)
-//   float32 + depth  1024  64      19.4 / 20.6 (19.2 / 20.4)
-//   float32          2048  96      25.0 / 27.2 (24.9 / 27.1)
-//   float32          4096 192      40.0 / 47.7 (49.4 / 48.0)
-//   float32          6656 312      65.5 / 73.8 (75.2 / 73.0)
-//   float32          8192 384      87.8 / 85.9 (88.9 / 86.4)
-//   float32 + depth  4096 256      49.4 / 61.5 (60.6 / 61.0)
-bool streams_frame(const pbr_scene_desc* D, const pbr_frame_out* O) {
-  constexpr uint64_t kL2Bytes = 64ull << 20, kKeptF32 = 320ull << 20, kKeptBf16 = 256ull << 20;
+// kL2Bytes leave the L2s sooner; of what is larger the 256 MiB last-level cache
+// keeps enough until the same buffers are written again, or read, for ordinary
+// stores to pay up to the limits below, except for uint8 colours, and for colours
+// beside depth or ids, which stay there better without them.  Kernel in us for
+// scenes of 64 x 64, none / colours / all streaming, one output buffer (two in
+// turn; d depth, i ids):
+//   uint8 d      1024  28 MiB  15.8 / 15.8 / 14.8 (15.7 / 15.6 / 14.7)
+//   uint8        4096  48      26.8 / 24.9        (26.2 / 24.4)
+//   uint8        8192  96      46.8 / 44.4        (45.7 / 43.7)
+//   uint8 d      4096 112      30.0 / 29.7 / 34.0 (29.9 / 29.7 / 33.7)
+//   bf16         8192 192      49.2 / 51.6        (53.1 / 51.1)
+//   bf16        12288 288      75.5 / 71.9        (75.3 / 70.7)
+//   bf16 d i     5200 284      54.5 / 53.5 / 69.8 (68.5 / 62.8 / 69.2)
+//   float32      1024  48      17.5 / 17.0        (17.3 / 16.9)
+//   float32      2048  96      25.0 / 27.2        (24.9 / 27.1)
+//   float32      4096 192      40.0 / 47.7        (49.4 / 48.0)
+//   float32      6656 312      65.5 / 73.8        (75.2 / 73.0)
+//   float32      8192 384      87.8 / 85.9        (88.9 / 86.4)
+//   float32 d    4096 256      49.4 / 50.2 / 61.5 (60.6 / 50.1 / 61.0)
+// Beyond kKeptPlanes three captured steps with depth in turn lose by depth's
+// ordinary stores, one alone gains (colours / all streaming, one - three: uint8
+// 12288, 336 MiB, 91 / 101 - 108 / 100; bf16 16384, 640 MiB, 129 / 150 - 155 / 150).
+int frame_stores(const pbr_scene_desc* D, const pbr_frame_out* O) {
+  constexpr uint64_t kL2Bytes = 64ull << 20, kKeptF32 = 320ull << 20, kKeptBf16 = 256ull << 20,
+                     kKeptPlanes = 328ull << 20;
   const uint64_t elem = O->dtype == PBR_DTYPE_U8 ? 1 : (O->dtype == PBR_DTYPE_BF16 ? 2 : 4);
-  if (D->width > 64 || (4 * D->width * elem) % 128 != 0) return false;
+  if (D->width > 64 || (4 * D->width * elem) % 128 != 0) return 0;
   const uint64_t bytes = (uint64_t)D->num_scenes * D->width * D->height *
                          (O->channels * elem + (O->depth ? 4 : 0) + (O->vis ? 4 : 0));
-  if (bytes <= kL2Bytes) return true;
-  if (O->depth || O->vis) return false;
-  return elem == 1 || bytes > (elem == 2 ? kKeptBf16 : kKeptF32);
+  if (bytes <= kL2Bytes) return 2;
+  if (O->depth || O->vis) return bytes > kKeptPlanes ? 2 : 1;
+  return elem == 1 || bytes > (elem == 2 ? kKeptBf16 : kKeptF32) ? 1 : 0;
 }
 
 // Whether both scenes' vertex slots fit the LDS vertex table (the vertex
@@ -1490,7 +1503,7 @@ int launch_rows(const pbr_scene_desc* D, const pbr_frame_out* O, const pbr_rende
   const bool small = rows_small(D);
   F.cap = cap ? cap : kCap;
   F.vphase = rows_vphase(D) ? 1 : 0;
-  F.stream = streams_frame(D, O) ? 1 : 0;
+  F.stream = frame_stores(D, O);
   const Light lt = host_light(D);
   const float4 bg = make_float4(D->background[0], D->background[1], D->background[2],
                                 D->background[3]);

@@ -31,11 +31,11 @@ def test_rows_kernel_ragged_widths(cuda, width, dtype):
         check_parity(r, f"rows width {width} {cls.__name__}, colour only", depth=False, vis=False)
 
 
-@pytest.mark.parametrize("n,dtype", [(7168, "float32"), (11264, "bfloat16")])
+@pytest.mark.parametrize("n,dtype", [(7168, "float32"), (11264, "bfloat16"), (1536, "float32"),
+                                     (1536, "bfloat16"), (1536, "uint8")])
 def test_rows_kernel_store_forms(cuda, n, dtype):
-    """Frames larger than the last-level cache leave by streaming stores: the
-    same pixels as the scenes give in smaller batches, alone and with depth and
-    ids (by ordinary stores)."""
+    """Which stores are streaming depends on the output's bytes: the same
+    pixels, alone and with depth and ids, as the scenes give in smaller batches."""
     st = ground_states(n, 3).cuda()
     vp = None  # the whole batch's: a view's aspect follows the batch's tile grid
 
@@ -51,9 +51,9 @@ def test_rows_kernel_store_forms(cuda, n, dtype):
         return r.render()["pixels"], full["pixels"], full["depth"], full["vis"]
 
     whole = frames(0, n)
-    for a in range(0, n, 1024):
-        for x, y in zip(whole, frames(a, a + 1024)):
-            assert _bits(x[a:a + 1024]).equal(_bits(y)), (a, x.dtype)
+    for a in range(0, n, 512):
+        for x, y in zip(whole, frames(a, a + 512)):
+            assert _bits(x[a:a + 512]).equal(_bits(y)), (a, x.dtype)
 
 
 @pytest.mark.parametrize("cap", [0, 8])
