@@ -453,7 +453,7 @@ def tile_workloads_leg(launches: int = 30) -> dict:
         torch.cuda.empty_cache()
     out["uneven_persistent"] = {
         "workload": "8192 scenes 84x84 uint8, log-uniform 1-256 instances of box / UV sphere / "
-                    "cylinder, one persistent (scene, tile) work-queue launch; uniform: same "
+                    "cylinder, one band workgroup per scene; uniform: same "
                     "draws with every scene at the mean instance count",
         **res,
         "uneven_over_uniform_per_triangle": round(res["uneven"]["ns_per_triangle"] /

@@ -131,9 +131,13 @@ typedef struct pbr_render_opts {
   int32_t lane_pixels;        /* scene: 4 or 8 pixels per lane, 0 = auto    */
   int32_t tile_size;          /* tiles: 8, 16, 32 or 64 pixel square tiles,
                                  0 = full-width bands; with bin_capacity 0
-                                 too and meshes of at most 136 vertices and
-                                 256 triangles these are drawn straight from
-                                 the instances, without records             */
+                                 too these are drawn straight from the
+                                 instances, without records, where every mesh
+                                 has at most 136 vertices and 256 triangles,
+                                 the meshes together at most 512 triangles, a
+                                 node at most 2^22 instances, a frame at most
+                                 four bands (of about 7900 pixels), and a
+                                 batch of few scenes few enough vertices    */
   int64_t slot_budget;        /* tiles: upper bound of the batch's triangle
                                  slots (sum over scenes of active instances
                                  x triangles); 0 = num_scenes x the largest

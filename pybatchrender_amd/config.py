@@ -19,9 +19,12 @@ New fields (defaults keep the reference's behaviour):
                    one setup pass, then one workgroup per scene tile) or
                    'chunked' (any triangle count, setup repeated per row strip)
     tile_size      tile kernels: 8, 16, 32 or 64 pixel square tiles (0 =
-                   full-width bands; with bin_capacity 0 and meshes of at most
-                   136 vertices and 256 triangles each band is drawn straight
-                   from the scene's instances)
+                   full-width bands; with bin_capacity 0 each band is drawn
+                   straight from the scene's instances where every mesh has at
+                   most 136 vertices and 256 triangles, the meshes together at
+                   most 512 triangles, a frame at most four bands of about 7900
+                   pixels, and a batch of up to 16 scenes at most 24576 + 6144
+                   per scene vertices a scene)
     bin_capacity   tile kernels: entries of each LDS bin of a tile before it
                    is rasterised and emptied, 1024..16384 (0 = 1904)
     row_list_cap   rows kernel: row-list entries per band, 8..256 (0 = 256)

@@ -1,9 +1,9 @@
 // pbr_bands.hip - the band path: one workgroup draws one band of full rows of
 // one scene from the scene's instances, with no records in device memory.
 //
-//   setup + raster  the scene's instances are dealt to the eight waves in
-//                   chunks (as many instances of one node as the wave's vertex
-//                   table holds).  A wave transforms and snaps the chunk's
+//   setup + raster  the scene's instances are dealt to the workgroup's eight or
+//                   sixteen waves in chunks (as many instances of one node as
+//                   the wave's vertex table holds).  A wave transforms and snaps the chunk's
 //                   vertices once into its LDS table, drops the chunk if all
 //                   of them lie outside one plane, off the band or between two
 //                   pixel centres, tests each triangle on three table entries,

@@ -58,8 +58,10 @@ _CAM_METHODS = frozenset(("set_positions", "set_eye", "_update_view", "_compose_
 
 
 class SteeringRenderer(PBRRenderer):
-    # _step reads no posed node's buffers after posing (it sets colours and
-    # the camera): step() poses and renders in one launch
+    # On the GPU a step's poses, colours and view are one launch of their own
+    # (_step_device).  Where that does not take the step, the tensor operations
+    # of _step read no posed node's buffers after posing, so that the render
+    # launch may apply the poses.
     fuse_poses = True
 
     def __init__(self, cfg: PBRConfig | dict | None = None) -> None:
