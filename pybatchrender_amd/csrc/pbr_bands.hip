@@ -1176,9 +1176,9 @@ struct BandPlan {
 //   400 to 2000          1.07 / 0.10  1.23 / 0.18  1.47 / 0.29  1.92 / 0.49  2.57 / 0.82
 // The line is where the mean over both is about one.  From 128 scenes on it is 1.8
 // to 2.3, the lowest 0.74 (1024 scenes of 160 x 160 with 500 boxes below a pixel).
-bool few_large_scenes(const pbr_scene_desc* D, const pbr_render_opts* opts) {
+bool few_large_scenes(const pbr_scene_desc* D, const pbr_render_opts* opts, int64_t cus) {
   const int64_t n = D->num_scenes;
-  if (n < 1 || 16 * n > device_cus()) return false;
+  if (n < 1 || 16 * n > cus) return false;
   double verts = 0.0;
   bool counts = false;
   for (int j = 0; j < D->num_nodes; ++j) {
@@ -1205,7 +1205,8 @@ bool few_large_scenes(const pbr_scene_desc* D, const pbr_render_opts* opts) {
 // and three to eight nodes with a sphere of 224 triangles each 1.3 to 4.5.
 bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& P) {
   if (opts && (opts->tile_size > 0 || opts->bin_capacity > 0)) return false;
-  if (few_large_scenes(D, opts)) return false;
+  const int64_t cus = device_cus();
+  if (few_large_scenes(D, opts, cus)) return false;
   memset(&P, 0, sizeof(P));
   BandFrame& F = P.F;
   F.W = D->width;
@@ -1255,7 +1256,7 @@ bool bands_plan(const pbr_scene_desc* D, const pbr_render_opts* opts, BandPlan& 
   // 16 / 16 and bands): 64 scenes of 84 x 84 with up to 256 instances 99 / 68 /
   // 50, of 128 x 128 with 64 boxes 26 / 26 / 18, of 64 x 64 steering 50 / 47 /
   // 45; 512 steering scenes in one workgroup per CU at a time 96, not 73.
-  const int64_t n = D->num_scenes, cus = device_cus();
+  const int64_t n = D->num_scenes;
   if (n * F.bands <= cus) {
     const int wide = (int)((2 * kBandLds - stat - rest(kWideWaves)) / 8);
     int bands = 1;

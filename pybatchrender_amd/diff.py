@@ -105,22 +105,19 @@ def _live_descriptor(renderer, vertices, light, colors):
     # transforms and a view-projection that a kernel cannot read in place: the
     # renderer's descriptor may hold a copy made before their last change
     for j, node in enumerate(g["nodes"]):
-        t = _readable(node.transforms_b44)
-        if t is not node.transforms_b44:
-            desc.nodes[j].transforms = t.data_ptr()
-            keep.append(t)
-    vp = renderer._pbr_cam.VP_k44
-    t = _readable(vp)
-    if t is not vp:
-        desc.view_proj = t.data_ptr()
-        keep.append(t)
+        t = node.transforms_b44
+        if t.dtype is not torch.float32 or not t.is_contiguous() or t.is_neg():
+            keep.append(_readable(t))
+            desc.nodes[j].transforms = keep[-1].data_ptr()
+    t = renderer._pbr_cam.VP_k44
+    if t.dtype is not torch.float32 or not t.is_contiguous() or t.is_neg():
+        keep.append(_readable(t))
+        desc.view_proj = keep[-1].data_ptr()
     return desc, keep
 
 
 def _readable(t: torch.Tensor) -> torch.Tensor:
-    """t if its memory holds its values as contiguous float32, else a copy."""
-    if t.dtype is torch.float32 and t.is_contiguous() and not t.is_neg():
-        return t
+    """t's values as contiguous float32 in memory."""
     return t.detach().to(torch.float32).contiguous().resolve_neg()
 
 

@@ -48,13 +48,16 @@ def _plain(t, shape: tuple, device: torch.device) -> bool:
     this shape on this device that autograd does not follow and whose memory
     holds its values (not their negatives, see torch's negative bit)."""
     return (type(t) is torch.Tensor and t.dtype is torch.float32 and t.device == device
-            and tuple(t.shape) == shape and t.is_contiguous() and not t.requires_grad
+            and t.shape == shape and t.is_contiguous() and not t.requires_grad
             and not t.is_neg())
 
 
-# what the tensor operations of a step call (PBRCam.set_positions)
-_CAM_METHODS = frozenset(("set_positions", "set_eye", "_update_view", "_compose_view", "_refresh",
-                          "_update_vp"))
+def _own_methods(cam: PBRCam) -> bool:
+    """Whether the camera object itself has its own version of a method that
+    the tensor operations of a step call (set_positions)."""
+    own = cam.__dict__
+    return ("set_positions" in own or "set_eye" in own or "_update_view" in own
+            or "_compose_view" in own or "_refresh" in own or "_update_vp" in own)
 
 
 class SteeringRenderer(PBRRenderer):
@@ -163,16 +166,18 @@ class SteeringRenderer(PBRRenderer):
         player = self.player_node
         if (type(self).set_poses is not PBRRenderer.set_poses or "set_poses" in self.__dict__
                 or type(player).set_colors is not PBRNode.set_colors
-                or "set_colors" in player.__dict__ or not _CAM_METHODS.isdisjoint(cam.__dict__)):
+                or "set_colors" in player.__dict__ or _own_methods(cam)):
             return False
         col = player.colors_b4 if player.has_geometry else None
         P = cam._get_projection()
         reads = (cam._right, cam._up, cam._fwd, P, self._camera_eye_offset, self._color_player,
                  self._color_crash)
         shapes = ((n, 3), (n, 3), (n, 3), (4, 4), (1, 3), (4,), (4,))
-        if not all(_plain(t, s, self.device) for t, s in zip(reads, shapes)):
-            return False
-        if col is not None and not _plain(col, (n, 4), self.device):
+        dev = self.device
+        for t, s in zip(reads, shapes):
+            if not _plain(t, s, dev):
+                return False
+        if col is not None and not _plain(col, (n, 4), dev):
             return False
         # the memory of a state with the negative bit holds other signs
         if (type(st) is not torch.Tensor or st.is_neg()
@@ -187,13 +192,14 @@ class SteeringRenderer(PBRRenderer):
                                   (self.right_border, dict(x=half, y=py, z=z)))]
         poses = [p for p in poses if p is not None]
         # nothing that the launch writes may be what another thread reads
-        written = [t for node in (player, self.left_border, self.right_border) if node.has_geometry
-                   for t in (node.transforms_b44, node.rot3_b33, node.scale_b11, node.colors_b4)]
         src = st.untyped_storage().data_ptr()
-        if any(t.untyped_storage().data_ptr() == src for t in written):
-            return False
-        eye = torch.empty((n, 3), dtype=torch.float32, device=self.device)
-        view = torch.empty((2, n, 4, 4), dtype=torch.float32, device=self.device)
+        for node in (player, self.left_border, self.right_border):
+            if node.has_geometry:
+                for t in (node.transforms_b44, node.rot3_b33, node.scale_b11, node.colors_b4):
+                    if t.untyped_storage().data_ptr() == src:
+                        return False
+        eye = torch.empty((n, 3), dtype=torch.float32, device=dev)
+        view = torch.empty((2, n, 4, 4), dtype=torch.float32, device=dev)
         b = _abi.pbr_steering_batch()
         b.state, b.row_stride, b.col_stride = st.data_ptr(), st.stride(0), st.stride(1)
         b.num_scenes, b.columns = n, st.shape[1]
