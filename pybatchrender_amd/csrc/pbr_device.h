@@ -496,9 +496,10 @@ __device__ __forceinline__ void load_mat4(const float* src, float M[16]) {
 // make later kernels wait.  Ordinary / streaming, us per call with two frames
 // in turn: 1024 scenes of 128 x 128 float32 + depth (band path) 134 / 109,
 // 8192 of 84 x 84 uint8 560 / 533 (the row-span kernel streams by the rule of
-// frame_stores in pbr_rows.hip).  Only for stores in which a wave writes one contiguous piece:
-// lines that several stores fill, each at its own time, are better put
-// together in the cache (single pixels that lanes scatter: 1024 scenes 212).
+// frame_stores in pbr_rows.hip).  Only for stores in which a wave writes one
+// contiguous piece: lines that several stores fill, each at its own time, are
+// better put together in the cache (single pixels that lanes scatter: 1024
+// scenes 212).
 template <int N> struct StreamWord;
 template <> struct StreamWord<4> {
   typedef uint32_t T __attribute__((aligned(1)));
